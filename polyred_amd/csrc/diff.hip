@@ -372,11 +372,13 @@ __global__ __launch_bounds__(256) void k_diff(DevScene s, ViewConsts v, DiffBuff
 // [block0, block0 + nblocks) of a virtual grid, block0 ascending and a
 // multiple of 8 (so a view's tiles keep the XCD spread of its own launch);
 // the workgroups stride over that grid, accumulating in LDS, and flush once.
-// The views' gradient and loss buffers are the same.
+// The views' gradient and loss buffers are the same.  `step` (may be null):
+// a fit's step counter, advanced by one.
 template <bool BACKWARD>
 __global__ __launch_bounds__(256) void k_diff_views(DevScene s, const DiffView* __restrict__ views, int32_t n_views,
-                                                    int32_t total_blocks) {
+                                                    int32_t total_blocks, int32_t* step) {
     __shared__ DiffAcc acc;
+    if (BACKWARD && step && blockIdx.x == 0 && threadIdx.x == 0) *step += 1;  // (k_adam reads it)
     if (BACKWARD) acc_clear(acc);
     for (int bid = blockIdx.x; bid < total_blocks; bid += gridDim.x) {
         int lo = 0, hi = n_views - 1;
@@ -407,20 +409,28 @@ __global__ __launch_bounds__(256) void k_diff_gbuffer(DevScene s, ViewConsts v, 
     g[3 * P + o] = make_float4(p.a.x, p.a.y, p.a.z, 0.0f);
 }
 
-// One workgroup: every listed parameter, then the step counter and the loss
-// history (the loss is that of the parameters before this step).
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ par, const float* __restrict__ grad,
+// Adam on the listed parameters, one a thread.  The step counter was advanced
+// by this step's adjoint (k_diff_views); each listed gradient is zeroed here
+// once read, and the loss by workgroup 0 once kept (the loss is that of the
+// parameters before this step), so a step is these two launches with no
+// clearing pass.  Memory: 40 bytes a parameter.  One workgroup for every
+// parameter took 238 us with 87 k of them (the vertex colours of 60 spheres);
+// a grid of them 5 us.
+__global__ __launch_bounds__(256) void k_adam(float* __restrict__ par, float* __restrict__ grad,
                                               const float* __restrict__ base, float* __restrict__ theta,
                                               float* __restrict__ m, float* __restrict__ v,
                                               const int32_t* __restrict__ idx, const float* __restrict__ lower,
-                                              AdamConsts a, int32_t* step, const double* loss, double* hist) {
-    const int t = *step + 1;
+                                              AdamConsts a, const int32_t* __restrict__ step, double* loss,
+                                              double* hist) {
+    const int t = *step;
     const float c1 = (float)(1.0 - pow64((double)a.beta1, (double)t));
     const float c2 = (float)(1.0 - pow64((double)a.beta2, (double)t));
-    for (int k = threadIdx.x; k < a.n; k += blockDim.x) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < a.n) {
         const int i = idx[k];
         const float b0 = base[i];
         const float g = grad[i] * b0;  // d loss / d theta for p = base * (1 + theta)
+        grad[i] = 0.0f;
         const float mk = a.beta1 * m[k] + (1.0f - a.beta1) * g;
         const float vk = a.beta2 * v[k] + (1.0f - a.beta2) * (g * g);
         m[k] = mk, v[k] = vk;
@@ -432,10 +442,9 @@ __global__ __launch_bounds__(256) void k_adam(float* __restrict__ par, const flo
         }
         theta[k] = th, par[i] = pv;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        *step = t;
+    if (k == 0) {
         if (t <= a.hist_cap) hist[t - 1] = *loss;
+        *loss = 0.0;
     }
 }
 
@@ -451,13 +460,13 @@ int32_t diff_blocks(const ViewConsts& v) {
 }
 
 void launch_diff_views(hipStream_t st, bool backward, const DevScene& s, const DiffView* views, int32_t n_views,
-                       int32_t total_blocks) {
+                       int32_t total_blocks, int32_t* step) {
     if (n_views <= 0 || total_blocks <= 0) return;
     // (a fixed grid of 2048 workgroups, 8 per CU, strides over the views' tiles)
     const int grid = total_blocks < 2048 ? total_blocks : 2048;
     if (backward)
-        hipLaunchKernelGGL(k_diff_views<true>, dim3(grid), dim3(256), 0, st, s, views, n_views, total_blocks);
-    else hipLaunchKernelGGL(k_diff_views<false>, dim3(grid), dim3(256), 0, st, s, views, n_views, total_blocks);
+        hipLaunchKernelGGL(k_diff_views<true>, dim3(grid), dim3(256), 0, st, s, views, n_views, total_blocks, step);
+    else hipLaunchKernelGGL(k_diff_views<false>, dim3(grid), dim3(256), 0, st, s, views, n_views, total_blocks, step);
 }
 
 void launch_diff_store_gbuffer(hipStream_t st, const DevScene& s, const ViewConsts& v, const DiffBuffers& b,
@@ -466,10 +475,11 @@ void launch_diff_store_gbuffer(hipStream_t st, const DevScene& s, const ViewCons
     if (P) hipLaunchKernelGGL(k_diff_gbuffer, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, st, s, v, b, gbuf);
 }
 
-void launch_adam(hipStream_t st, float* par, const float* grad, const float* base, float* theta, float* m, float* v,
-                 const int32_t* idx, const float* lower, AdamConsts a, int32_t* step, const double* loss,
+void launch_adam(hipStream_t st, float* par, float* grad, const float* base, float* theta, float* m, float* v,
+                 const int32_t* idx, const float* lower, AdamConsts a, const int32_t* step, double* loss,
                  double* hist) {
-    hipLaunchKernelGGL(k_adam, dim3(1), dim3(256), 0, st, par, grad, base, theta, m, v, idx, lower, a, step, loss,
+    const unsigned grid = a.n > 256 ? (unsigned)((a.n + 255) / 256) : 1u;
+    hipLaunchKernelGGL(k_adam, dim3(grid), dim3(256), 0, st, par, grad, base, theta, m, v, idx, lower, a, step, loss,
                        hist);
 }
 

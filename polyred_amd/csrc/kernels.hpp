@@ -101,21 +101,23 @@ struct DiffView {
     int32_t block0, nblocks;
 };
 int32_t diff_blocks(const ViewConsts& v);
+// step (may be null): a fit's step counter, advanced by the adjoint
 void launch_diff_views(hipStream_t st, bool backward, const DevScene& s, const DiffView* views, int32_t n_views,
-                       int32_t total_blocks);
+                       int32_t total_blocks, int32_t* step);
 // The stored G-buffer of one view (world position + material, normal +
 // shadow scale, view vector, albedo: 4 float4 planes of H*W).
 void launch_diff_store_gbuffer(hipStream_t st, const DevScene& s, const ViewConsts& v, const DiffBuffers& b,
                                float4* gbuf);
 // Adam (Kingma & Ba 2015, Algorithm 1) on the parameters p = base * (1 + theta)
 // listed in idx; t is the device step counter, loss the step's loss, kept
-// in hist[t - 1].
+// in hist[t - 1].  Leaves the listed gradients and the loss at zero for the
+// next step's adjoint.
 struct AdamConsts {
     float lr, beta1, beta2, eps;
     int32_t n, hist_cap;
 };
-void launch_adam(hipStream_t st, float* par, const float* grad, const float* base, float* theta, float* m, float* v,
-                 const int32_t* idx, const float* lower, AdamConsts a, int32_t* step, const double* loss,
+void launch_adam(hipStream_t st, float* par, float* grad, const float* base, float* theta, float* m, float* v,
+                 const int32_t* idx, const float* lower, AdamConsts a, const int32_t* step, double* loss,
                  double* hist);
 
 // Layout of the AO march tables, in float (4-byte) units.  Binade buckets are

@@ -2089,7 +2089,7 @@ int prh_fit_targets(prh_fit* f, const prh_diff_params* truth) {
     hipStream_t st = f->ctx->stream;
     if ((rc = upload_params(f->views[0], f->l, truth, f->par, st))) return rc;
     if ((rc = fit_views(f, false, DIFF_ALL, st))) return rc;
-    launch_diff_views(st, false, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks);
+    launch_diff_views(st, false, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks, nullptr);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     return PRH_OK;
@@ -2140,6 +2140,9 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->m), l.total, 0u);
     launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->v), l.total, 0u);
     launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->step), 1, 0u);
+    // (each step's Adam pass leaves the gradients it read, and the loss, at zero)
+    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->grad), l.total, 0u);
+    launch_fill_u64(st, reinterpret_cast<uint64_t*>(f->loss), 1, 0ull);
     HIP_TRY(hipStreamSynchronize(st));  // idx and lower are locals
     if (o->steps > f->hist_cap) {
         if (f->hist) {
@@ -2164,14 +2167,12 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     if ((rc = fit_views(f, true, (uint32_t)o->groups, st))) return rc;
     HIP_TRY(hipGetLastError());
     const AdamConsts a{o->lr, o->beta1, o->beta2, o->eps, n_idx, f->hist_cap};
-    // one step: clear, adjoint over every view, Adam; captured once, replayed
+    // one step: the adjoint over every view, Adam; captured once, replayed
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
     if (o->steps > 0) {
         HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-        launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->grad), l.total, 0u);
-        launch_fill_u64(st, reinterpret_cast<uint64_t*>(f->loss), 1, 0ull);
-        launch_diff_views(st, true, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks);
+        launch_diff_views(st, true, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks, f->step);
         launch_adam(st, f->par, f->grad, f->base, f->theta, f->m, f->v, f->idx, f->lower, a, f->step, f->loss,
                     f->hist);
         const hipError_t e = hipStreamEndCapture(st, &g);
