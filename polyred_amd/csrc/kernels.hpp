@@ -69,8 +69,10 @@ struct ShadeBuffers {
 // The differentiable shading pass (diff.hip): parameters, fixed inputs and
 // gradient outputs, all in HBM.
 constexpr int DIFF_MAX_LIGHTS = 8;
+constexpr int DIFF_REPS = 8;
 struct DiffBuffers {
     const uint64_t* vis;       // fixed visibility (the last frame)
+    const int4* tri_rec;       // per triangle: transformed vertices and flat material (k_tri_rec)
     const float4* tv_scr;      // screen xy + recipw per transformed vertex
     const float4* tv_nor;      // n.Apply(Normal) per transformed vertex (the default normals)
     const float4* tv_wp;       // back-transformed position per transformed vertex
@@ -85,25 +87,41 @@ struct DiffBuffers {
     const uint8_t* shadow_count;  // [H][W] fixed shadow visibility: the shading is scaled by 2^-count; or null
     const float4* gbuf;        // [4][H][W] stored G-buffer (diff_store_gbuffer), or null: rebuilt from vis
     const float* target;       // [H][W][3] raster rows (adjoint)
+    uint32_t* list;            // [H*W] the shaded pixels, x | y << 16, by strips (adjoint; launch_diff_list)
     float* linear;             // [H][W][3] raster rows (forward), NaN where not shaded
     float *g_albedo, *g_normal, *g_kd, *g_ks, *g_shin, *g_lpos, *g_lint;  // zeroed before the adjoint
-    double* loss;
+    double* loss;              // [DIFF_REPS] summed by the reader
     uint32_t want;             // DIFF_* gradient groups to accumulate
+    // replicas of g_kd .. g_lint, rep_stride floats apart, summed by the
+    // reader: DIFF_REPS or 1
+    int32_t reps, rep_stride;
 };
 // Gradient groups (the bits of prh.h's PRH_FIT_* flags).
 constexpr uint32_t DIFF_ALBEDO = 1, DIFF_NORMAL = 2, DIFF_KD = 4, DIFF_KS = 8, DIFF_SHININESS = 16,
                    DIFF_LIGHT_POS = 32, DIFF_LIGHT_INT = 64, DIFF_ALL = 127;
-void launch_diff(hipStream_t st, bool backward, const DevScene& s, const ViewConsts& v, const DiffBuffers& b);
-// One view of a multi-view launch: its blocks are [block0, block0 + nblocks).
+// One view of a multi-view launch: its forward's workgroups are [block0,
+// block0 + nblocks), its list's [strip0, ...).
 struct DiffView {
     ViewConsts v;
     DiffBuffers b;
-    int32_t block0, nblocks;
+    int32_t block0, nblocks, strip0;
 };
 int32_t diff_blocks(const ViewConsts& v);
-// step (may be null): a fit's step counter, advanced by the adjoint
-void launch_diff_views(hipStream_t st, bool backward, const DevScene& s, const DiffView* views, int32_t n_views,
-                       int32_t total_blocks, int32_t* step);
+int32_t diff_strips(const ViewConsts& v);
+size_t diff_chunks(const ViewConsts& v);  // entries of the chunk table a view may fill
+void launch_diff_forward(hipStream_t st, const DevScene& s, const ViewConsts& v, const DiffBuffers& b);
+void launch_diff_forward_views(hipStream_t st, const DevScene& s, const DiffView* views, int32_t n, int32_t blocks);
+// The adjoint: the gradients (n floats), the loss and the count of chunks
+// zeroed, the views' shaded pixels listed, then the adjoint over the list.
+void launch_diff_clear(hipStream_t st, float* grad, size_t n, double* loss, int32_t* count);
+void launch_diff_list(hipStream_t st, const DiffView& w, uint2* chunks, int32_t* count);
+void launch_diff_list_views(hipStream_t st, const DiffView* views, int32_t n, int32_t strips, uint2* chunks,
+                            int32_t* count);
+void launch_adjoint(hipStream_t st, const DevScene& s, const DiffView& w, const uint2* chunks, const int32_t* count);
+// vertices: the views want albedo or normal gradients (and store no
+// G-buffer); step (may be null): a fit's step counter, advanced by the adjoint
+void launch_adjoint_views(hipStream_t st, const DevScene& s, const DiffView* views, size_t max_chunks,
+                          const uint2* chunks, const int32_t* count, bool vertices, int32_t* step);
 // The stored G-buffer of one view (world position + material, normal +
 // shadow scale, view vector, albedo: 4 float4 planes of H*W).
 void launch_diff_store_gbuffer(hipStream_t st, const DevScene& s, const ViewConsts& v, const DiffBuffers& b,
@@ -111,10 +129,12 @@ void launch_diff_store_gbuffer(hipStream_t st, const DevScene& s, const ViewCons
 // Adam (Kingma & Ba 2015, Algorithm 1) on the parameters p = base * (1 + theta)
 // listed in idx; t is the device step counter, loss the step's loss, kept
 // in hist[t - 1].  Leaves the listed gradients and the loss at zero for the
-// next step's adjoint.
+// next step's adjoint.  Gradients from rep_from on have `reps` replicas,
+// rep_stride apart.
 struct AdamConsts {
     float lr, beta1, beta2, eps;
     int32_t n, hist_cap;
+    int32_t reps, rep_from, rep_stride;
 };
 void launch_adam(hipStream_t st, float* par, float* grad, const float* base, float* theta, float* m, float* v,
                  const int32_t* idx, const float* lower, AdamConsts a, const int32_t* step, double* loss,

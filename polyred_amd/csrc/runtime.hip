@@ -1043,8 +1043,10 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     if (!rc) chk(ralloc(r, &r->tile_off, r->tile_slots + 1));
     if (!rc) chk(ralloc(r, &r->chunk_off, r->tile_slots + 1));
 
+    // (outside the exact-order pass these two are the adjoint's pixel list and
+    // its chunk table, with its count of chunks)
     if (!rc) chk(ralloc(r, &r->first_all, P));
-    if (!rc) chk(ralloc(r, &r->first_nan, P));
+    if (!rc) chk(ralloc(r, &r->first_nan, std::max(P, 2 * diff_chunks(vc) + 2)));
     if (!rc) chk(ralloc(r, &r->tile_cursor, r->tile_slots));
     if (!rc && r->n_slots > 0) {
         chk(ralloc(r, &r->s_scan_sums, 2 * (size_t)scan_blocks(r->s_tile_slots)));
@@ -1502,14 +1504,20 @@ int batch_graph(prh_ctx* ctx, prh_renderer* const* rs, int n, bool wide) {
 }
 
 // Offsets (in floats) of the differentiable parameters / gradients block.
+// A gradient block holds `reps` replicas of its part from kd on, total - kd
+// apart (the adjoint's workgroups spread over them; the reader sums them).
 struct DiffLayout {
     size_t albedo, normal, kd, ks, shin, lpos, lint, total;
+    int reps;
+    size_t tail() const { return total - kd; }
+    size_t grad_total() const { return kd + reps * tail(); }
 };
 DiffLayout diff_layout(const prh_renderer* r) {
     const size_t V = r->sc->d.n_tverts, M = r->sc->d.n_materials, L = r->sc->d.n_lights;
     DiffLayout l;
     l.albedo = 0, l.normal = 3 * V, l.kd = 6 * V, l.ks = l.kd + 3 * M, l.shin = l.ks + 3 * M;
     l.lpos = l.shin + M, l.lint = l.lpos + 3 * L, l.total = l.lint + L + 1;
+    l.reps = M <= 512 ? DIFF_REPS : 1;  // (many materials: their own gradients spread the atomics)
     return l;
 }
 
@@ -1537,17 +1545,18 @@ int shadow_counts(prh_renderer* r, hipStream_t st, const uint8_t** out) {
 DiffBuffers diff_buffers(const prh_renderer* r, const DiffLayout& l, const float* par, float* grad, double* loss,
                          bool normal, const uint8_t* count) {
     DiffBuffers b;
-    b.vis = r->vis, b.tv_scr = r->tv_scr, b.tv_nor = r->tv_nor, b.tv_wp = r->tv_wp;
+    b.vis = r->vis, b.tri_rec = r->tri_rec, b.tv_scr = r->tv_scr, b.tv_nor = r->tv_nor, b.tv_wp = r->tv_wp;
     b.albedo = par + l.albedo, b.normal = normal ? par + l.normal : nullptr;
     b.kd = par + l.kd, b.ks = par + l.ks, b.shininess = par + l.shin;
     b.light_pos = par + l.lpos, b.light_int = par + l.lint;
     b.ambient = r->sc->ambient_sum;
     b.shadow_count = count, b.gbuf = nullptr;
-    b.target = nullptr, b.linear = nullptr;
+    b.target = nullptr, b.linear = nullptr, b.list = r->first_all;
     b.g_albedo = grad + l.albedo, b.g_normal = grad + l.normal, b.g_kd = grad + l.kd;
     b.g_ks = grad + l.ks, b.g_shin = grad + l.shin, b.g_lpos = grad + l.lpos, b.g_lint = grad + l.lint;
     b.loss = loss;
     b.want = DIFF_ALL;
+    b.reps = l.reps, b.rep_stride = (int32_t)l.tail();
     return b;
 }
 
@@ -1577,6 +1586,43 @@ int check_params(const prh_renderer* r, const prh_diff_params* p) {
     return PRH_OK;
 }
 
+// Enqueues the adjoint of one view: clears, lists the shaded pixels, runs.
+// The list and the chunk table are the renderer's exact-order buffers.
+void enqueue_adjoint(prh_renderer* r, const DiffBuffers& b, float* grad, size_t n, hipStream_t st) {
+    DiffView w{};
+    w.v = r->vc, w.b = b;
+    int32_t* count = reinterpret_cast<int32_t*>(r->first_nan);
+    uint2* chunks = reinterpret_cast<uint2*>(r->first_nan) + 1;
+    launch_diff_clear(st, grad, n, b.loss, count);
+    launch_diff_list(st, w, chunks, count);
+    launch_adjoint(st, r->sc->d, w, chunks, count);
+}
+
+// The gradients of an adjoint and its loss, from the gradient block to the
+// host, the replicas summed (synchronises).
+int download_grads(const prh_renderer* r, const DiffLayout& l, const float* grad, const double* loss_dev,
+                   const prh_diff_grads* grads, double* loss, hipStream_t st) {
+    const DevScene& d = r->sc->d;
+    const size_t V = d.n_tverts, M = d.n_materials, L = d.n_lights, tail = l.tail();
+    std::vector<float> t(l.reps * tail);
+    double part[DIFF_REPS];
+    if (grads->albedo && V) HIP_TRY(hipMemcpyAsync(grads->albedo, grad + l.albedo, 12 * V, hipMemcpyDeviceToHost, st));
+    if (grads->normal && V) HIP_TRY(hipMemcpyAsync(grads->normal, grad + l.normal, 12 * V, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(t.data(), grad + l.kd, 4 * t.size(), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(part, loss_dev, sizeof part, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    for (int k = 1; k < l.reps; k++)
+        for (size_t i = 0; i < tail; i++) t[i] += t[k * tail + i];
+    auto put = [&](float* dst, size_t off, size_t n) {
+        if (dst && n) memcpy(dst, t.data() + (off - l.kd), 4 * n);
+    };
+    put(grads->kd, l.kd, 3 * M), put(grads->ks, l.ks, 3 * M), put(grads->shininess, l.shin, M);
+    put(grads->light_pos, l.lpos, 3 * L), put(grads->light_int, l.lint, L);
+    *loss = 0.0;
+    for (double v : part) *loss += v;
+    return PRH_OK;
+}
+
 // One launch of the differentiable shading: forward (target == nullptr,
 // result in diff_lin) or adjoint (loss and gradients copied to the host).
 int diff_run(prh_renderer* r, const prh_diff_params* p, const float* target, double* loss,
@@ -1594,10 +1640,10 @@ int diff_run(prh_renderer* r, const prh_diff_params* p, const float* target, dou
             if (!rc) rc = v;
         };
         chk(ralloc(r, &r->diff_par, l.total));
-        if (!rc) chk(ralloc(r, &r->diff_grad, l.total));
+        if (!rc) chk(ralloc(r, &r->diff_grad, l.grad_total()));
         if (!rc) chk(ralloc(r, &r->diff_target, 3 * P));
         if (!rc) chk(ralloc(r, &r->diff_lin, 3 * P));
-        if (!rc) chk(ralloc(r, &r->diff_loss, 1));
+        if (!rc) chk(ralloc(r, &r->diff_loss, DIFF_REPS));
         for (int i = 0; i < 2 && !rc; i++)
             if (hipEventCreate(&r->dev[i]) != hipSuccess) rc = fail(PRH_E_HIP, "hipEventCreate failed");
         if (rc) {
@@ -1605,7 +1651,6 @@ int diff_run(prh_renderer* r, const prh_diff_params* p, const float* target, dou
             return rc;
         }
     }
-    const size_t V = d.n_tverts, M = d.n_materials, L = d.n_lights;
     int rc1 = upload_params(r, l, p, r->diff_par, st);
     const uint8_t* count = nullptr;
     if (!rc1) rc1 = shadow_counts(r, st, &count);
@@ -1615,25 +1660,13 @@ int diff_run(prh_renderer* r, const prh_diff_params* p, const float* target, dou
     const bool backward = target != nullptr;
     if (backward) {
         HIP_TRY(hipMemcpyAsync(r->diff_target, target, 12 * P, hipMemcpyHostToDevice, st));
-        launch_fill_u32(st, reinterpret_cast<uint32_t*>(r->diff_grad), l.total, 0u);
-        launch_fill_u64(st, reinterpret_cast<uint64_t*>(r->diff_loss), 1, 0ull);
     }
     (void)hipEventRecord(r->dev[0], st);
-    launch_diff(st, backward, d, r->vc, b);
+    if (backward) enqueue_adjoint(r, b, r->diff_grad, l.grad_total(), st);
+    else launch_diff_forward(st, d, r->vc, b);
     (void)hipEventRecord(r->dev[1], st);
-    if (backward) {
-        auto down = [&](float* dst, size_t off, size_t n) -> hipError_t {
-            return dst && n ? hipMemcpyAsync(dst, r->diff_grad + off, n * 4, hipMemcpyDeviceToHost, st) : hipSuccess;
-        };
-        HIP_TRY(down(grads->albedo, l.albedo, 3 * V));
-        HIP_TRY(down(grads->normal, l.normal, 3 * V));
-        HIP_TRY(down(grads->kd, l.kd, 3 * M));
-        HIP_TRY(down(grads->ks, l.ks, 3 * M));
-        HIP_TRY(down(grads->shininess, l.shin, M));
-        HIP_TRY(down(grads->light_pos, l.lpos, 3 * L));
-        HIP_TRY(down(grads->light_int, l.lint, L));
-        HIP_TRY(hipMemcpyAsync(loss, r->diff_loss, 8, hipMemcpyDeviceToHost, st));
-    }
+    if (backward) rc1 = download_grads(r, l, r->diff_grad, r->diff_loss, grads, loss, st);
+    if (rc1) return rc1;
     HIP_TRY(hipStreamSynchronize(st));
     (void)hipEventElapsedTime(&r->stats.ms_diff, r->dev[0], r->dev[1]);
     return PRH_OK;
@@ -1689,7 +1722,10 @@ struct prh_fit {
     std::vector<const uint8_t*> count;
     std::vector<float4*> gbuf;
     DiffView* d_views;
-    int32_t total_blocks;
+    int32_t total_blocks, total_strips;  // of the forward and of the list
+    uint2* chunks;      // the adjoint's chunk table over all views
+    int32_t* n_chunks;  // and its count
+    size_t max_chunks;
     hipEvent_t ev[4];
     prh_fit_stats stats;
 };
@@ -1713,7 +1749,7 @@ int fit_check(prh_fit* f) {
 // Every view's buffers, launch blocks in view order, uploaded to d_views.
 int fit_views(prh_fit* f, bool backward, uint32_t want, hipStream_t st) {
     std::vector<DiffView> h(f->views.size());
-    int32_t blk = 0;
+    int32_t blk = 0, strip = 0;
     for (size_t i = 0; i < f->views.size(); i++) {
         prh_renderer* r = f->views[i];
         DiffBuffers b = diff_buffers(r, f->l, f->par, f->grad, f->loss, false, f->count[i]);
@@ -1727,8 +1763,10 @@ int fit_views(prh_fit* f, bool backward, uint32_t want, hipStream_t st) {
         h[i].v = r->vc, h[i].b = b;
         h[i].block0 = blk, h[i].nblocks = diff_blocks(r->vc);
         blk += h[i].nblocks;
+        h[i].strip0 = strip;
+        strip += diff_strips(r->vc);
     }
-    f->total_blocks = blk;
+    f->total_blocks = blk, f->total_strips = strip;
     HIP_TRY(hipMemcpyAsync(f->d_views, h.data(), h.size() * sizeof(DiffView), hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));  // h is a local
     return PRH_OK;
@@ -1948,16 +1986,20 @@ int prh_diff_backward_noalloc(prh_renderer* r, const prh_diff_params* p, const f
     uint8_t* base = r->ctx->scratch;
     if (!base) return fail(PRH_E_HIP, "prh_diff_backward_noalloc: no scratch array on this device: " + r->ctx->scratch_err);
     // the scratch array's layout for this frame, each part 256-byte aligned
-    const DiffLayout l = diff_layout(r);
+    DiffLayout l = diff_layout(r);
     const bool counts = r->sh.shadow_map;
-    size_t need = 0;
-    auto take = [&](size_t n) {
-        const size_t o = need;
-        need += (n + 255) & ~(size_t)255;
-        return o;
-    };
-    const size_t o_par = take(4 * l.total), o_grad = take(4 * l.total), o_tgt = take(12 * P), o_loss = take(8);
-    const size_t o_cnt = counts ? take(P) : 0;
+    size_t need, o_par, o_grad, o_tgt, o_loss, o_cnt;
+    for (;; l.reps = 1) {
+        need = 0;
+        auto take = [&](size_t n) {
+            const size_t o = need;
+            need += (n + 255) & ~(size_t)255;
+            return o;
+        };
+        o_par = take(4 * l.total), o_grad = take(4 * l.grad_total()), o_tgt = take(12 * P), o_loss = take(8 * DIFF_REPS);
+        o_cnt = counts ? take(P) : 0;
+        if (need <= PRH_NOALLOC_SCRATCH_BYTES || l.reps == 1) break;  // (without the replicas where they do not fit)
+    }
     if (need > PRH_NOALLOC_SCRATCH_BYTES)
         return fail(PRH_E_INVALID, "prh_diff_backward_noalloc: the frame needs " + std::to_string(need) +
                                        " bytes of scratch, more than the " +
@@ -1968,33 +2010,18 @@ int prh_diff_backward_noalloc(prh_renderer* r, const prh_diff_params* p, const f
     double* lossd = reinterpret_cast<double*>(base + o_loss);
     uint8_t* cnt = counts ? base + o_cnt : nullptr;
     const DevScene& d = r->sc->d;
-    const size_t V = d.n_tverts, M = d.n_materials, L = d.n_lights;
     hipStream_t st = r->ctx->stream;
     if ((rc = upload_params(r, l, p, par, st))) return rc;
     HIP_TRY(hipMemcpyAsync(tgt, target, 12 * P, hipMemcpyHostToDevice, st));
-    // the array keeps the previous call's contents: clear what accumulates,
-    // with fill kernels (no memset nodes if a caller captures this)
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(grad), l.total, 0u);
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(lossd), 1, 0ull);
     if (counts) launch_shadow_count(st, d, r->sh, shade_buffers(r), cnt);  // every pixel written
     HIP_TRY(hipGetLastError());
     DiffBuffers b = diff_buffers(r, l, par, grad, lossd, p->normal != nullptr, cnt);
     b.target = tgt, b.linear = nullptr;
-    launch_diff(st, true, d, r->vc, b);
+    // (the array keeps the previous call's contents: this clears what
+    // accumulates, with a kernel: no memset nodes if a caller captures it)
+    enqueue_adjoint(r, b, grad, l.grad_total(), st);
     HIP_TRY(hipGetLastError());
-    auto down = [&](float* dst, size_t off, size_t n) -> hipError_t {
-        return dst && n ? hipMemcpyAsync(dst, grad + off, n * 4, hipMemcpyDeviceToHost, st) : hipSuccess;
-    };
-    HIP_TRY(down(grads->albedo, l.albedo, 3 * V));
-    HIP_TRY(down(grads->normal, l.normal, 3 * V));
-    HIP_TRY(down(grads->kd, l.kd, 3 * M));
-    HIP_TRY(down(grads->ks, l.ks, 3 * M));
-    HIP_TRY(down(grads->shininess, l.shin, M));
-    HIP_TRY(down(grads->light_pos, l.lpos, 3 * L));
-    HIP_TRY(down(grads->light_int, l.lint, L));
-    HIP_TRY(hipMemcpyAsync(loss, lossd, 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    return PRH_OK;
+    return download_grads(r, l, grad, lossd, grads, loss, st);
 }
 
 int prh_fit_new(prh_renderer* const* views, int32_t n, int32_t flags, prh_fit** out) {
@@ -2027,16 +2054,20 @@ int prh_fit_new(prh_renderer* const* views, int32_t n, int32_t flags, prh_fit** 
         if (!rc) rc = v;
     };
     chk(falloc(f, &f->par, T));
-    chk(falloc(f, &f->grad, T));
+    chk(falloc(f, &f->grad, f->l.grad_total()));
     chk(falloc(f, &f->base, T));
     chk(falloc(f, &f->theta, T));
     chk(falloc(f, &f->m, T));
     chk(falloc(f, &f->v, T));
     chk(falloc(f, &f->lower, T));
     chk(falloc(f, &f->idx, T));
-    chk(falloc(f, &f->loss, 1));
+    chk(falloc(f, &f->loss, DIFF_REPS));
     chk(falloc(f, &f->step, 1));
     chk(falloc(f, &f->d_views, (size_t)n));
+    f->max_chunks = 0;
+    for (prh_renderer* r : f->views) f->max_chunks += diff_chunks(r->vc);
+    chk(falloc(f, &f->chunks, f->max_chunks));
+    chk(falloc(f, &f->n_chunks, 1));
     for (int k = 0; k < 4 && !rc; k++)
         if (hipEventCreate(&f->ev[k]) != hipSuccess) rc = fail(PRH_E_HIP, "hipEventCreate failed");
     double vis_bytes = 0;
@@ -2089,7 +2120,7 @@ int prh_fit_targets(prh_fit* f, const prh_diff_params* truth) {
     hipStream_t st = f->ctx->stream;
     if ((rc = upload_params(f->views[0], f->l, truth, f->par, st))) return rc;
     if ((rc = fit_views(f, false, DIFF_ALL, st))) return rc;
-    launch_diff_views(st, false, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks, nullptr);
+    launch_diff_forward_views(st, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     return PRH_OK;
@@ -2141,8 +2172,7 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->v), l.total, 0u);
     launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->step), 1, 0u);
     // (each step's Adam pass leaves the gradients it read, and the loss, at zero)
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->grad), l.total, 0u);
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(f->loss), 1, 0ull);
+    launch_diff_clear(st, f->grad, l.grad_total(), f->loss, f->n_chunks);
     HIP_TRY(hipStreamSynchronize(st));  // idx and lower are locals
     if (o->steps > f->hist_cap) {
         if (f->hist) {
@@ -2165,14 +2195,17 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     }
     HIP_TRY(hipEventRecord(f->ev[3], st));
     if ((rc = fit_views(f, true, (uint32_t)o->groups, st))) return rc;
+    // the shaded pixels, which the steps share
+    launch_diff_list_views(st, f->d_views, (int32_t)f->views.size(), f->total_strips, f->chunks, f->n_chunks);
     HIP_TRY(hipGetLastError());
-    const AdamConsts a{o->lr, o->beta1, o->beta2, o->eps, n_idx, f->hist_cap};
+    const AdamConsts a{o->lr, o->beta1, o->beta2, o->eps, n_idx, f->hist_cap, l.reps, (int32_t)l.kd, (int32_t)l.tail()};
     // one step: the adjoint over every view, Adam; captured once, replayed
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
     if (o->steps > 0) {
         HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-        launch_diff_views(st, true, f->sc->d, f->d_views, (int32_t)f->views.size(), f->total_blocks, f->step);
+        launch_adjoint_views(st, f->sc->d, f->d_views, f->max_chunks, f->chunks, f->n_chunks,
+                             (o->groups & PRH_FIT_ALBEDO) != 0, f->step);
         launch_adam(st, f->par, f->grad, f->base, f->theta, f->m, f->v, f->idx, f->lower, a, f->step, f->loss,
                     f->hist);
         const hipError_t e = hipStreamEndCapture(st, &g);
