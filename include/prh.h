@@ -230,7 +230,8 @@ typedef struct prh_frame_stats {
     int32_t n_prims;     /* primitives after cull/clip: unclipped triangles
                             plus the clipper's pieces                       */
     int32_t n_clipped;   /* triangles that went through the clipper         */
-    int32_t n_bin_pairs; /* (primitive, tile) pairs                         */
+    int32_t n_bin_pairs; /* (primitive, raster tile) pairs of the primitives
+                            the setup does not draw itself                  */
     int32_t nan_rerun;   /* 1 if the NaN-depth exact-order pass ran         */
     float ms_diff;       /* the last prh_diff_forward / _backward kernel    */
 } prh_frame_stats;
@@ -368,26 +369,24 @@ int prh_surface_size(prh_surface* s, int32_t* width, int32_t* height);
 /* ---- autotuning (no counterpart in polyred) ------------------------------
  * Knobs that change how fast a frame renders but not what it renders: every
  * merge they touch is order-independent, so frames are bit-identical under
- * any setting.  The tile is fixed at 16x16: one 256-thread workgroup holds a
- * tile with one pixel per thread, and the shading's 8x8 wave blocks and the
- * AO's row segments are laid out on it. */
+ * any setting.  The shading's tile is fixed at 16x16: one 256-thread workgroup
+ * holds a tile with one pixel per thread. */
 typedef struct prh_tuning {
     int32_t raster_wg_per_cu;  /* persistent raster workgroups per CU (occupancy), 1..16; default 8        */
-    int32_t item_prims;        /* primitives per raster work item (bin capacity), a power of 2 in
-                                  64..8192; default 2048                                                   */
+    int32_t item_prims;        /* a power of 2 in 64..8192; default 2048.  Kept for callers that set it:
+                                  the raster has no per-tile lists whose capacity it was                   */
     int32_t shadow_direct_max; /* shadow-map triangles of at most this many texel centres are drawn by
                                   the setup, 0..256; default 64                                            */
     int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise; 48  */
     int32_t overlap_shadows;   /* 1: a frame's shadow passes run on a second stream beside the main
                                   view's passes; default 1 from 2^19 framebuffer pixels, else 0          */
-    int32_t raster_tile;       /* side of the binning and raster tiles (main view and shadow maps):
-                                  8, 16 or 32 pixels; default 16                                          */
+    int32_t raster_tile;       /* side of the raster tiles (main view and shadow maps): 8, 16 or 32
+                                  pixels, a raster job being at most 2 x 2 of them; default 16            */
     float ms;                  /* prh_autotune: the chosen configuration's median frame time             */
 } prh_tuning;
 int prh_get_tuning(prh_renderer* r, prh_tuning* out);
 int prh_set_tuning(prh_renderer* r, const prh_tuning* t);
-/* Coordinate descent over item_prims {256..4096}, raster_wg_per_cu {1, 2, 4,
- * 8}, shadow_direct_max {0, 16, 32, 64, 128, 256}, main_direct_max {0, 24,
+/* Coordinate descent over raster_wg_per_cu {1, 2, 4, 8}, shadow_direct_max {0, 16, 32, 64, 128, 256}, main_direct_max {0, 24,
  * 48, 96, 192}, overlap_shadows {0, 1} and raster_tile {8, 16, 32}: each
  * configuration timed as the median of
  * `frames` frames (HIP events, after one warm-up frame); the winner is timed
@@ -398,7 +397,7 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out);
 /* The same search for a batch (no counterpart in polyred): the views of a
  * prh_render_batch of wide launches, split into two size classes (class 0
  * below 2^19 framebuffer pixels, class 1 the rest), each class with its own
- * item_prims, raster_wg_per_cu (in a wide batch: n_CU * raster_wg_per_cu /
+ * raster_wg_per_cu (in a wide batch: n_CU * raster_wg_per_cu /
  * 16 persistent raster workgroups per view, at least 32), shadow_direct_max,
  * main_direct_max and raster_tile.  Coordinate descent over the (class, knob) pairs, each
  * configuration timed as the median of `frames` eager wide batches; the

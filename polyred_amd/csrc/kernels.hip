@@ -1,5 +1,5 @@
-// kernels.hip — libprh's gfx950 kernels: vertex transform, triangle setup /
-// clip / bin, LDS-binned visibility and shadow rasters, deferred shading with
+// kernels.hip — libprh's gfx950 kernels: vertex transform, triangle setup and
+// clip, visibility and shadow rasters, deferred shading with
 // shadow maps, SSAO and sRGB fused.  All arithmetic that decides coverage,
 // depth, primitive order or colour follows polyred's CPU renderer bit for bit
 // (render/raster.go, render/clipping.go, render/shadow.go,
@@ -119,64 +119,14 @@ __device__ bool vp_contains(V4 p, float w, float h) {  // box.go:61-75 for one v
            less_eq(p.z, 1.0f);
 }
 
-// Adds one to counter[key] for every active lane with a single atomic per
-// distinct key in the wave (neighbouring triangles share tiles, and a shadow
-// map concentrates a scene in few tiles, so per-lane atomics collide).
-__device__ __forceinline__ void wave_count(int32_t* counter, int key, bool active) {
-    uint64_t pending = __ballot(active);
-    while (pending) {
-        const int leader = __ffsll((unsigned long long)pending) - 1;
-        const int lkey = __shfl(key, leader);
-        const uint64_t same = __ballot(active && key == lkey) & pending;
-        if (__lane_id() == leader) atomicAdd(&counter[lkey], __popcll(same));
-        pending &= ~same;
-    }
-}
-// counter[key]++ for every active lane, one atomic per distinct key; returns
-// the lane's pre-increment value.
-__device__ __forceinline__ int wave_alloc(int32_t* counter, int key, bool active) {
-    uint64_t pending = __ballot(active);
-    int pos = 0;
-    const int lane = __lane_id();
-    while (pending) {
-        const int leader = __ffsll((unsigned long long)pending) - 1;
-        const int lkey = __shfl(key, leader);
-        const uint64_t same = __ballot(active && key == lkey) & pending;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&counter[lkey], __popcll(same));
-        base = __shfl(base, leader);
-        if ((same >> lane) & 1ull) pos = base + __popcll(same & ((1ull << lane) - 1ull));
-        pending &= ~same;
-    }
-    return pos;
-}
-// Counts a primitive into every tile its pixel box touches (wave-uniform call).
-__device__ __forceinline__ void count_tiles(int32_t* tile_count, int base, int tiles_x, int shift, bool active, int x0,
-                                            int y0, int x1, int y1) {
-    const int tx0 = x0 >> shift, ty0 = y0 >> shift, ntx = active ? (x1 >> shift) - tx0 + 1 : 0;
-    const int n = active ? ntx * ((y1 >> shift) - ty0 + 1) : 0;
-    for (int j = 0; __ballot(j < n) != 0; j++) {
-        const bool act = j < n;
-        const int key = act ? base + (ty0 + j / ntx) * tiles_x + tx0 + j % ntx : 0;
-        wave_count(tile_count, key, act);
-    }
-}
-
-constexpr uint32_t PRIM_EMPTY = 0xffffffffu;  // bbox word of an unused primitive slot
-
-// A primitive slot is its 48-byte record plus its pixel box in a separate
-// 8-byte array, which is all k_bin reads; an empty slot only marks its box.
-__device__ __forceinline__ void store_empty(uint2* pbox, size_t slot) {
-    pbox[slot] = make_uint2(PRIM_EMPTY, PRIM_EMPTY);
-}
-__device__ __forceinline__ void store_prim(Prim* prims, uint2* pbox, size_t slot, V4 a, V4 b, V4 c, uint32_t key,
-                                           int x0, int y0, int x1, int y1) {
-    Prim p;
-    p.p0 = make_float4(a.x, a.y, a.z, b.x);
-    p.p1 = make_float4(b.y, b.z, c.x, c.y);
-    p.p2 = make_float4(c.z, bitsf(key), bitsf(pack_bbox(x0, y0)), bitsf(pack_bbox(x1, y1)));
-    prims[slot] = p;
-    pbox[slot] = make_uint2(pack_bbox(x0, y0), pack_bbox(x1, y1));
+// A place in a counter for every active lane, one atomic a wave.
+__device__ __forceinline__ int wave_place(int32_t* counter, bool active) {
+    const uint64_t m = __ballot(active);
+    if (m == 0) return 0;
+    const int lane = __lane_id(), leader = __ffsll((unsigned long long)m) - 1;
+    int base = 0;
+    if (lane == leader) base = atomicAdd(counter, __popcll(m));
+    return __shfl(base, leader) + __popcll(m & ((1ull << lane) - 1ull));
 }
 
 // The six screen-space planes of Sutherland-Hodgman, clipping.go:31-65
@@ -232,7 +182,7 @@ struct k_frame_clear_args {
     int32_t gx, gy;  // the grid of this launch
 };
 __device__ __forceinline__ void frame_clear_part(const FrameClear& c, size_t i0, size_t stride) {
-    if (i0 < (size_t)c.n_cnt) c.cnt[i0] = 0u;
+    for (size_t i = i0; i < (size_t)c.n_cnt; i += stride) c.cnt[i] = 0u;
     for (size_t i = i0; i < c.n_vis; i += stride) c.vis[i] = VIS_EMPTY;
 }
 __device__ __forceinline__ void k_frame_clear_body(const k_frame_clear_args& a_, const VB vb) {
@@ -352,26 +302,9 @@ __global__ __launch_bounds__(256) void k_vertex_shadow_wide(const k_vertex_shado
 
 // ------------------------------------------------------- triangle setup
 // render/raster.go:257-269 (IsValid) and draw, raster.go:380-444: back-face
-// cull, viewport AABB test, then either one primitive in the triangle's own
-// slot (all vertices inside) or a place in the clipper's queue.  Each
-// primitive is counted into every 16x16 tile its pixel box touches.
-// Exclusive scan of one value per thread over a 256-thread block.
-__device__ __forceinline__ void block_scan_256(int v, int32_t* start /*[257]*/, int32_t* wsum /*[4]*/) {
-    int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    int incl = v;
-    for (int off = 1; off < 64; off <<= 1) {
-        int u = __shfl_up(incl, off);
-        if (lane >= off) incl += u;
-    }
-    if (lane == 63) wsum[wv] = incl;
-    __syncthreads();
-    int before = 0;
-    for (int k = 0; k < wv; k++) before += wsum[k];
-    start[tid] = before + incl - v;
-    if (tid == 255) start[256] = before + incl;
-    __syncthreads();
-}
-
+// cull, viewport AABB test, then either a primitive (all vertices inside),
+// drawn here if small and handed to the raster as jobs if not, or a place in
+// the clipper's queue.
 // Inclusive scan of one int per lane over the wave (sum or max, values >= 0)
 // in DPP steps: Hillis-Steele over each row of 16 lanes (row_shr 1, 2, 4,
 // 8; a lane past its row's start reads 0, the identity of both), then the
@@ -468,22 +401,71 @@ __device__ __forceinline__ void draw_small_tris(bool mine, V4 p1, V4 p2, V4 p3, 
     });
 }
 
+// A larger primitive is handed to the raster pass as jobs: rectangles of at
+// most `side` pixels a side of its pixel box, each a record of its own (the
+// vertices, the order key or the map, the rectangle) in one of RASTER_QUEUES
+// queues, the workgroup's, at a place its wave takes with one atomic.  The
+// wave's jobs are spread over its lanes, so a triangle that covers the screen
+// costs its wave a few rounds.  (They were counted into 16x16 tiles, scanned,
+// listed by tile and rasterised tile by tile: two triangles covering 1600x1200
+// held their wave's lane for 1.4 ms, and a frame of small ones paid 15-25 us
+// for the three passes.)
+__device__ __forceinline__ void emit_jobs(bool mine, V4 p1, V4 p2, V4 p3, uint32_t key, int x0, int y0, int x1, int y1,
+                                          int shift, int block, const JobQueues& q, Counters* cnt,
+                                          int32_t* wmark /*[64]*/) {
+    if (__ballot(mine) == 0) return;
+    const int side = 1 << shift;
+    const int nx = mine ? (x1 - x0 + side) >> shift : 0, c = mine ? nx * ((y1 - y0 + side) >> shift) : 0;
+    const int lane = threadIdx.x & 63;
+    const int total = __builtin_amdgcn_readlane(wave_scan_incl<false>(c), 63);
+    const int qi = block & (RASTER_QUEUES - 1);
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&q.n[qi * JOB_COUNT_STRIDE], total);
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (base + total > q.cap) {  // the host grows the queues and draws the frame again
+        if (lane == 0) atomicMax(&cnt->need_jobs, base + total), atomicOr(&cnt->overflow, 1);
+        return;
+    }
+    Prim* out = q.jobs + (size_t)qi * q.cap + base;
+    int done = 0;
+    wave_spread(c, wmark, [&](int o, int l, bool valid) {
+        Prim j;
+        j.p0 = make_float4(__shfl(p1.x, o), __shfl(p1.y, o), __shfl(p1.z, o), __shfl(p2.x, o));
+        j.p1 = make_float4(__shfl(p2.y, o), __shfl(p2.z, o), __shfl(p3.x, o), __shfl(p3.y, o));
+        const int onx = __shfl(nx, o), ox0 = __shfl(x0, o), oy0 = __shfl(y0, o), ox1 = __shfl(x1, o),
+                  oy1 = __shfl(y1, o);
+        const float cz = __shfl(p3.z, o);
+        const uint32_t okey = (uint32_t)__shfl((int)key, o);
+        if (valid) {
+            const int jy = l / onx, jx = l - jy * onx;
+            const int ax = ox0 + (jx << shift), ay = oy0 + (jy << shift);
+            j.p2 = make_float4(cz, bitsf(okey), bitsf(pack_bbox(ax, ay)),
+                               bitsf(pack_bbox(min(ax + side - 1, ox1), min(ay + side - 1, oy1))));
+            out[done + lane] = j;
+        }
+        done += 64;
+    });
+}
+// The raster tiles a pixel box touches (the frame statistics' pairs).
+__device__ __forceinline__ int box_tiles(int x0, int y0, int x1, int y1, int shift) {
+    return ((x1 >> shift) - (x0 >> shift) + 1) * ((y1 >> shift) - (y0 >> shift) + 1);
+}
+
 // An unclipped triangle whose pixel box holds at most `draw_small` pixel
 // centres (0: none; prh_tuning.main_direct_max) is drawn by the setup itself
 // outside the exact-order pass: each
 // centre is tested as k_raster<VIS> tests it and merged into the visibility
 // buffer with a global 64-bit atomic min of the same key (order-independent),
-// and the triangle is neither stored nor binned.
+// and the triangle makes no job.
 
 struct k_setup_main_args {
     DevScene s;
     ViewConsts vc;
     const float4* tv_scr;
-    Prim* prims;
-    uint2* pbox;
     ClipJob* clip_list;
-    int32_t* tile_count;
+    JobQueues jobs;
     int32_t* blk_prims;
+    int32_t* blk_pairs;
     Counters* cnt;
     Capacities cap;
     unsigned long long* vis;
@@ -495,10 +477,7 @@ __device__ __forceinline__ void k_setup_main_body(const k_setup_main_args& a_, c
     const DevScene& s = a_.s;
     const ViewConsts& vc = a_.vc;
     const float4* __restrict__ tv_scr = a_.tv_scr;
-    Prim* __restrict__ prims = a_.prims;
-    uint2* __restrict__ pbox = a_.pbox;
     ClipJob* __restrict__ clip_list = a_.clip_list;
-    int32_t* __restrict__ tile_count = a_.tile_count;
     int32_t* __restrict__ blk_prims = a_.blk_prims;
     Counters* cnt = a_.cnt;
     const Capacities& cap = a_.cap;
@@ -533,14 +512,11 @@ __device__ __forceinline__ void k_setup_main_body(const k_setup_main_args& a_, c
                 }
             }
         }
-        const uint32_t key = (uint32_t)g * 8u + SUB_DIRECT;
         drawn = direct && draw_small > 0 && (x1 - x0 + 1) * (y1 - y0 + 1) <= draw_small;
-        if (direct && !drawn) store_prim(prims, pbox, g, p1, p2, p3, key, x0, y0, x1, y1);
-        else store_empty(pbox, g);
     }
+    __shared__ int32_t mark[256];
     {
         __shared__ DPrim sp[256];
-        __shared__ int32_t mark[256];
         const uint32_t key0 = (uint32_t)(g - (int)(threadIdx.x & 63)) * 8u + SUB_DIRECT;  // the wave's first triangle
         bool nan = false;
         draw_small_tris(drawn, p1, p2, p3, x0, y0, x1, y1, sp, mark, [&](int px, int py, float z, int o) {
@@ -551,16 +527,27 @@ __device__ __forceinline__ void k_setup_main_body(const k_setup_main_args& a_, c
         });
         if (nan) atomicOr(&cnt->nan_flag, 1);
     }
-    count_tiles(tile_count, 0, vc.rtiles_x, vc.rt_shift, direct && !drawn, x0, y0, x1, y1);
-    const int pos = wave_alloc(&cnt->n_clipped, 0, doclip);
+    const bool big = direct && !drawn;
+    emit_jobs(big, p1, p2, p3, (uint32_t)g * 8u + SUB_DIRECT, x0, y0, x1, y1, vc.rt_shift + 1, vb.bx, a_.jobs, cnt,
+              mark + (threadIdx.x & ~63));
+    const int pos = wave_place(&cnt->n_clipped, doclip);
     if (doclip) {
         if (pos < cap.clip_tris) clip_list[pos] = job;
         else atomicOr(&cnt->overflow, 1);
     }
-    // the primitive count of the frame statistics, summed by k_scan (one
-    // global counter hit by every workgroup would serialise them)
+    // the frame statistics, summed when they are read (one global counter hit
+    // by every workgroup would serialise them): the unclipped primitives, and
+    // the raster tiles touched by those the raster draws
+    __shared__ int32_t s_pairs;
+    if (threadIdx.x == 0) s_pairs = 0;
     const int nd = __syncthreads_count(direct);
-    if (threadIdx.x == 0) blk_prims[vb.bx] = nd;
+    const int nb = __syncthreads_count(big);
+    if (nb && big) atomicAdd(&s_pairs, box_tiles(x0, y0, x1, y1, vc.rt_shift));
+    if (nb) __syncthreads();
+    if (threadIdx.x == 0) {
+        blk_prims[vb.bx] = nd;
+        if (a_.blk_pairs) a_.blk_pairs[vb.bx] = s_pairs;
+    }
 }
 __global__ __launch_bounds__(256) void k_setup_main(k_setup_main_args a) {
     k_setup_main_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
@@ -580,20 +567,16 @@ __global__ __launch_bounds__(256) void k_setup_main_wide(const k_setup_main_args
 // centres (prh_tuning.shadow_direct_max) is drawn here: each centre is
 // tested and merged into the map with a
 // global atomic max, exactly as k_raster<SHADOW> would (the same Barycoord,
-// depth and max over ordered bits; order-independent), and it is neither
-// stored nor binned.  Most triangles of a map fitted to the whole frustum
-// cover a few texels; past a few dozen the binned raster is no slower.
+// depth and max over ordered bits; order-independent), and it makes no job.
+// Most triangles of a map fitted to the whole frustum cover a few texels.
 
 struct k_setup_shadow_args {
     DevScene s;
     ShadowConsts sc;
     const int4* tri_rec;
     const float3* ts;
-    Prim* prims;
-    uint2* pbox;
-    int32_t* tile_count;
+    JobQueues jobs;
     Counters* cnt;
-    Capacities cap;
     uint32_t* smaps;
     int32_t gx, gy;  // the grid of this launch
 };
@@ -601,9 +584,6 @@ __device__ __forceinline__ void k_setup_shadow_body(const k_setup_shadow_args& a
     const DevScene& s = a_.s;
     const ShadowConsts& sc = a_.sc;
     const float3* __restrict__ ts = a_.ts;
-    Prim* __restrict__ prims = a_.prims;
-    uint2* __restrict__ pbox = a_.pbox;
-    int32_t* __restrict__ tile_count = a_.tile_count;
     Counters* cnt = a_.cnt;
     uint32_t* __restrict__ smaps = a_.smaps;
 
@@ -627,9 +607,9 @@ __device__ __forceinline__ void k_setup_shadow_body(const k_setup_shadow_args& a
     }
     const bool small = emit && (x1 - x0 + 1) * (y1 - y0 + 1) <= sc.direct_max;
     if (small) emit = false;
+    __shared__ int32_t mark[256];
     {
         __shared__ DPrim sp[256];
-        __shared__ int32_t mark[256];
         uint32_t* map = smaps + (size_t)slot * sc.SW * sc.SH;
         bool nan = false;
         draw_small_tris(small, p1, p2, p3, x0, y0, x1, y1, sp, mark, [&](int px, int py, float z, int) {
@@ -639,12 +619,8 @@ __device__ __forceinline__ void k_setup_shadow_body(const k_setup_shadow_args& a
         });
         if (nan) atomicOr(&cnt->shadow_nan, 1);
     }
-    if (g < s.n_tris) {
-        const size_t ps = (size_t)slot * s.n_tris + g;
-        if (emit) store_prim(prims, pbox, ps, p1, p2, p3, (uint32_t)slot, x0, y0, x1, y1);
-        else store_empty(pbox, ps);
-    }
-    count_tiles(tile_count, slot * sc.tiles_per_map, sc.tiles_x, sc.rt_shift, emit, x0, y0, x1, y1);
+    emit_jobs(emit, p1, p2, p3, (uint32_t)slot, x0, y0, x1, y1, sc.rt_shift + 1, vb.bx + slot, a_.jobs, cnt,
+              mark + (threadIdx.x & ~63));
 }
 __global__ __launch_bounds__(256) void k_setup_shadow(k_setup_shadow_args a) {
     k_setup_shadow_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
@@ -658,338 +634,11 @@ __global__ __launch_bounds__(256) void k_setup_shadow_wide(const k_setup_shadow_
     k_setup_shadow_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
 }
 
-// ------------------------------------------------------------ tile scan
-// Exclusive prefix sums of the per-tile primitive counts and of the per-tile
-// work items (ceil(count / ITEM_PRIMS)): per-thread runs of consecutive
-// tiles, wave scans, then the 16 wave totals.  Up to SCAN_WHOLE_MAX tiles
-// (a 1080p view's 8160) one workgroup scans them all, SCAN_WHOLE_MAX / 1024
-// a thread, in one launch; beyond, k_scan_sums reduces each block of SCAN_BLOCK tiles
-// and every workgroup of k_scan_apply adds the sums of the blocks before its
-// own and scans its block, 4 tiles a thread.
-constexpr int SCAN_BLOCK = 4096;
-constexpr int SCAN_WHOLE_MAX = 8192;
-
-__device__ __forceinline__ int wave_incl_scan(int v, int) { return wave_scan_incl<false>(v); }  // (v >= 0)
-__device__ __forceinline__ int wave_sum(int v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-__device__ __forceinline__ int item_count(int v, int ip) { return (v + ip - 1) / ip; }
-
-struct k_scan_sums_args {
-    const int32_t* counts;
-    int32_t n;
-    int32_t* bsum;
-    int32_t item_prims;
-    int32_t gx, gy;  // the grid of this launch
-};
-__device__ __forceinline__ void k_scan_sums_body(const k_scan_sums_args& a_, const VB vb) {
-    const int32_t item_prims = a_.item_prims;
-    const int32_t* __restrict__ counts = a_.counts;
-    const int32_t n = a_.n;
-    int32_t* __restrict__ bsum = a_.bsum;
-
-    __shared__ int32_t ws[16], wc[16];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int i0 = vb.bx * SCAN_BLOCK + 4 * tid;
-    int sv = 0, sc = 0;
-    for (int k = 0; k < 4; k++) {
-        const int v = i0 + k < n ? counts[i0 + k] : 0;
-        sv += v;
-        sc += item_count(v, item_prims);
-    }
-    sv = wave_sum(sv), sc = wave_sum(sc);
-    if (lane == 0) ws[wv] = sv, wc[wv] = sc;
-    __syncthreads();
-    if (tid == 0) {
-        int a = 0, c = 0;
-        for (int k = 0; k < 16; k++) a += ws[k], c += wc[k];
-        bsum[2 * vb.bx] = a;
-        bsum[2 * vb.bx + 1] = c;
-    }
-}
-__global__ __launch_bounds__(1024) void k_scan_sums(k_scan_sums_args a) {
-    k_scan_sums_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
-}
-__global__ __launch_bounds__(1024) void k_scan_sums_wide(const k_scan_sums_args* __restrict__ a, const int32_t* __restrict__ start,
-        int32_t n) {
-    const int v = wide_view(start, n, (int)blockIdx.x);
-    const k_scan_sums_args& x = a[v];
-    const int local = (int)blockIdx.x - start[v];
-    if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_scan_sums_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
-}
-
-// Also lists each work item's tile (item_tile, up to cap_items entries) and
-// leaves the counts at zero for the next pass.
-struct k_scan_apply_args {
-    int32_t* counts;
-    int32_t n;
-    const int32_t* bsum;
-    int32_t* offsets;
-    int32_t* chunk_off;
-    int32_t* cursor;
-    int32_t* item_tile;
-    int32_t cap_items;
-    const int32_t* blk_prims;
-    int32_t n_blk;
-    Counters* cnt;
-    int32_t item_prims;
-    int32_t gx, gy;  // the grid of this launch
-};
-__device__ __forceinline__ void k_scan_apply_body(const k_scan_apply_args& a_, const VB vb) {
-    constexpr int NT = 1024, NW = NT / 64, PER = SCAN_WHOLE_MAX / NT;
-    const int32_t item_prims = a_.item_prims;
-    int32_t* __restrict__ counts = a_.counts;
-    const int32_t n = a_.n;
-    const int32_t* __restrict__ bsum = a_.bsum;
-    int32_t* __restrict__ offsets = a_.offsets;
-    int32_t* __restrict__ chunk_off = a_.chunk_off;
-    int32_t* __restrict__ cursor = a_.cursor;
-    int32_t* __restrict__ item_tile = a_.item_tile;
-    const int32_t cap_items = a_.cap_items;
-    const int32_t* __restrict__ blk_prims = a_.blk_prims;
-    const int32_t n_blk = a_.n_blk;
-    Counters* cnt = a_.cnt;
-
-    __shared__ int32_t ws[NW], wc[NW];
-    __shared__ int32_t carry_s, carry_c;
-    __shared__ int32_t s_t[SCAN_WHOLE_MAX + SCAN_WHOLE_MAX / 32];  // whole scan: tile i at i + i / 32
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const bool whole = vb.gx == 1;
-    // the frame statistics' per-workgroup primitive counts, loaded at once
-    // by the workgroup that sums them (the last)
-    int np = 0;
-    if (whole || vb.bx == vb.gx - 1) {
-        int pv[8];  // (every load issued before the first is waited for)
-#pragma unroll
-        for (int j = 0; j < 8; j++) pv[j] = tid + j * NT < n_blk ? blk_prims[tid + j * NT] : 0;
-#pragma unroll
-        for (int j = 0; j < 8; j++) np += pv[j];
-        for (int k = tid + 8 * NT; k < n_blk; k += NT) np += blk_prims[k];
-    }
-    int run = 0, runc = 0;
-    if (whole) {
-        // One workgroup for every tile: thread t takes tiles PER*t ..
-        // PER*t + PER-1, read and written through LDS so that the global
-        // accesses stay coalesced (the padded slots keep both LDS patterns
-        // free of bank conflicts).
-        {
-            int c[PER];  // (every load issued before the first is waited for)
-#pragma unroll
-            for (int k = 0; k < PER; k++) c[k] = k * NT + tid < n ? counts[k * NT + tid] : 0;
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int i = k * NT + tid;
-                if (i < n) s_t[i + (i >> 5)] = c[k], counts[i] = 0;
-            }
-        }
-        __syncthreads();
-        int v[PER], ch[PER];
-        int local = 0, localc = 0;
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = PER * tid + k;
-            v[k] = i < n ? s_t[i + (i >> 5)] : 0;
-            ch[k] = item_count(v[k], item_prims);
-            local += v[k], localc += ch[k];
-        }
-        const int incl = wave_incl_scan(local, lane), inclc = wave_incl_scan(localc, lane);
-        if (lane == 63) ws[wv] = incl, wc[wv] = inclc;
-        __syncthreads();  // (and every thread has read its tiles)
-        run = incl - local, runc = inclc - localc;
-        for (int k = 0; k < wv; k++) run += ws[k], runc += wc[k];
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = PER * tid + k;
-            if (i < n) s_t[i + (i >> 5)] = run;
-            run += v[k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = k * NT + tid;
-            if (i < n) {
-                const int o = s_t[i + (i >> 5)];
-                offsets[i] = o;
-                cursor[i] = o;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = PER * tid + k;
-            if (i < n) {
-                s_t[i + (i >> 5)] = runc;
-                for (int c = runc; c < runc + ch[k] && c < cap_items; c++) item_tile[c] = i;
-            }
-            runc += ch[k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = k * NT + tid;
-            if (i < n) chunk_off[i] = s_t[i + (i >> 5)];
-        }
-    } else {
-        // block vb.bx of SCAN_BLOCK tiles (4 consecutive tiles a thread)
-        // after the sums of the blocks before it
-        const int i0 = vb.bx * SCAN_BLOCK + 4 * tid;
-        int ps = 0, pc = 0;
-        for (int k = tid; k < vb.bx; k += NT) ps += bsum[2 * k], pc += bsum[2 * k + 1];
-        ps = wave_sum(ps), pc = wave_sum(pc);
-        if (lane == 0) ws[wv] = ps, wc[wv] = pc;
-        __syncthreads();
-        if (tid == 0) {
-            int a = 0, c = 0;
-            for (int k = 0; k < NW; k++) a += ws[k], c += wc[k];
-            carry_s = a, carry_c = c;
-        }
-        __syncthreads();
-        int v[4], ch[4];
-        for (int k = 0; k < 4; k++) {
-            v[k] = i0 + k < n ? counts[i0 + k] : 0;
-            ch[k] = item_count(v[k], item_prims);
-        }
-        const int local = v[0] + v[1] + v[2] + v[3], localc = ch[0] + ch[1] + ch[2] + ch[3];
-        const int incl = wave_incl_scan(local, lane), inclc = wave_incl_scan(localc, lane);
-        if (lane == 63) ws[wv] = incl, wc[wv] = inclc;
-        __syncthreads();
-        int before = carry_s, beforec = carry_c;
-        for (int k = 0; k < wv; k++) before += ws[k], beforec += wc[k];
-        run = before + incl - local, runc = beforec + inclc - localc;
-        for (int k = 0; k < 4; k++)
-            if (i0 + k < n) {
-                offsets[i0 + k] = run;
-                cursor[i0 + k] = run;
-                chunk_off[i0 + k] = runc;
-                for (int c = runc; c < runc + ch[k] && c < cap_items; c++) item_tile[c] = i0 + k;
-                counts[i0 + k] = 0;
-                run += v[k];
-                runc += ch[k];
-            }
-    }
-    if (!whole && vb.bx != vb.gx - 1) return;
-    // the last block writes the totals and the frame statistics: unclipped
-    // primitives (per-workgroup counts of the setup) plus the clipper's pieces
-    if (tid == NT - 1) {
-        offsets[n] = run;
-        chunk_off[n] = runc;
-        cnt->n_pairs = run;
-        cnt->n_chunks = runc;
-    }
-    np = wave_sum(np);
-    __syncthreads();  // every wave has read ws[] above
-    if (lane == 0) ws[wv] = np;
-    __syncthreads();
-    if (tid == 0) {
-        int a = 0;
-        for (int k = 0; k < NW; k++) a += ws[k];
-        cnt->n_prims = a;
-    }
-}
-__global__ __launch_bounds__(1024) void k_scan_apply(k_scan_apply_args a) {
-    k_scan_apply_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
-}
-__global__ __launch_bounds__(1024) void k_scan_apply_wide(const k_scan_apply_args* __restrict__ a, const int32_t* __restrict__ start,
-        int32_t n) {
-    const int v = wide_view(start, n, (int)blockIdx.x);
-    const k_scan_apply_args& x = a[v];
-    const int local = (int)blockIdx.x - start[v];
-    if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_scan_apply_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
-}
-
-// Scatter each primitive into the lists of the tiles its pixel box touches.
-// Slots [0, n_fixed) are one per triangle (per shadow slot); the main view's
-// clipped pieces follow them.
-struct k_bin_args {
-    const uint2* pbox;
-    Counters* cnt;
-    int32_t tiles_x;
-    int32_t shift;  // log2 of the raster tile side
-    int32_t tiles_per_view;
-    int32_t shadow;
-    int32_t* cursor;
-    int32_t* list;
-    Capacities cap;
-    int32_t n_fixed;
-    int32_t n_tris;
-    int32_t gx, gy;  // the grid of this launch
-};
-__device__ __forceinline__ void k_bin_body(const k_bin_args& a_, const VB vb) {
-    const uint2* __restrict__ pbox = a_.pbox;
-    Counters* cnt = a_.cnt;
-    const int32_t tiles_x = a_.tiles_x;
-    const int32_t shift = a_.shift;
-    const int32_t tiles_per_view = a_.tiles_per_view;
-    const int32_t shadow = a_.shadow;
-    int32_t* __restrict__ cursor = a_.cursor;
-    int32_t* __restrict__ list = a_.list;
-    const Capacities& cap = a_.cap;
-    const int32_t n_fixed = a_.n_fixed;
-    const int32_t n_tris = a_.n_tris;
-
-    const int i = vb.bx * blockDim.x + threadIdx.x;
-    if (cnt->n_pairs > cap.pairs) {
-        if (i == 0) atomicOr(&cnt->overflow, 1);
-        return;
-    }
-    if (cnt->overflow) return;
-    // (the clipper's pieces: CLIP_PIECES slots a queued triangle)
-    const int np = n_fixed + (shadow ? 0 : min(CLIP_PIECES * min(cnt->n_clipped, cap.clip_tris), cap.clip_subs));
-    bool active = false;
-    int x0 = 0, y0 = 0, x1 = 0, y1 = 0, base = 0;
-    if (i < np) {
-        const uint2 bb = pbox[i];
-        if (bb.y != PRIM_EMPTY) {
-            active = true;
-            x0 = bb.x & 0xffff, y0 = bb.x >> 16, x1 = bb.y & 0xffff, y1 = bb.y >> 16;
-            base = shadow ? (i / n_tris) * tiles_per_view : 0;  // shadow slot s holds [s*Tg, (s+1)*Tg)
-        }
-    }
-    const int tx0 = x0 >> shift, ty0 = y0 >> shift, ntx = active ? (x1 >> shift) - tx0 + 1 : 0;
-    const int n = active ? ntx * ((y1 >> shift) - ty0 + 1) : 0;
-    if (shadow) {
-        // a shadow map gathers a scene in a few of its tiles, so many of the
-        // wave's pairs share a tile: one returning atomic per distinct tile
-        for (int j = 0; __ballot(j < n) != 0; j++) {
-            const bool act = j < n;
-            const int key = act ? base + (ty0 + j / ntx) * tiles_x + tx0 + j % ntx : 0;
-            const int pos = wave_alloc(cursor, key, act);
-            if (act) list[pos] = i;
-        }
-        return;
-    }
-    // the main view's pairs are few and spread: the wave's (primitive, tile)
-    // pairs go over its lanes, each lane's cursor atomic issued at once (not
-    // one returning atomic per distinct tile after another)
-    __shared__ int32_t mark[256];
-    const int lane = threadIdx.x & 63;
-    wave_spread(n, mark + (threadIdx.x & ~63), [&](int o, int j, bool valid) {
-        const int otx0 = __shfl(tx0, o), oty0 = __shfl(ty0, o), ontx = __shfl(ntx, o), obase = __shfl(base, o);
-        if (!valid) return;
-        const int key = obase + (oty0 + j / ontx) * tiles_x + otx0 + j % ontx;
-        list[atomicAdd(&cursor[key], 1)] = i - lane + o;
-    });
-}
-__global__ __launch_bounds__(256) void k_bin(k_bin_args a) {
-    k_bin_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
-}
-__global__ __launch_bounds__(256) void k_bin_wide(const k_bin_args* __restrict__ a, const int32_t* __restrict__ start,
-        int32_t n) {
-    const int v = wide_view(start, n, (int)blockIdx.x);
-    const k_bin_args& x = a[v];
-    const int local = (int)blockIdx.x - start[v];
-    if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_bin_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
-}
-
 // ------------------------------------------------------------ clipper
 // The clipper (clipTriangle, clipping.go:67-157) for the queued triangles:
 // Sutherland-Hodgman against the six screen-space planes, a fan of pieces
 // with screen-barycentric attributes that keep the parent's recipw
-// (raster.go:440-443), appended after the per-triangle primitive slots.
+// (raster.go:440-443).
 //
 // One wave per queued triangle (a frame queues a few thousand at most, so
 // the pass is one triangle's latency, not throughput).  Each plane's pass
@@ -997,17 +646,15 @@ __global__ __launch_bounds__(256) void k_bin_wide(const k_bin_args* __restrict__
 // (vertex i-1, vertex i) and emits what the serial loop emits for it (the
 // intersection and/or vertex i); an exclusive scan of the emit counts
 // places them in the serial order, in the wave's other LDS polygon.  Three
-// lanes then build each fan piece, and the wave spreads each piece's tile
-// counts over its lanes.
+// lanes then build each fan piece, and the wave makes the pieces' raster jobs.
 constexpr int CLIP_WAVES = 4;   // waves per workgroup (a lane's fan piece needs up to 256 VGPRs)
 constexpr int CLIP_VERTS = 12;  // polygon capacity (a triangle clipped by six planes keeps at most 9)
 
 __device__ __forceinline__ int clip_wave(int qi, const ClipJob& jb, const DevScene& s, const ViewConsts& vc,
                                           const float4* __restrict__ tv_scr, const float4* __restrict__ tv_nor,
-                                          Prim* __restrict__ prims,
-                                          uint2* __restrict__ pbox, ClipRec* __restrict__ clips,
-                                          int32_t* __restrict__ tri_clip_slot, int32_t* __restrict__ tile_count,
-                                          Counters* cnt, const Capacities& cap, V4 (*poly)[CLIP_VERTS]) {
+                                          const JobQueues& jobs, ClipRec* __restrict__ clips,
+                                          int32_t* __restrict__ tri_clip_slot, Counters* cnt, const Capacities& cap,
+                                          V4 (*poly)[CLIP_VERTS], int32_t* wmark, int& pairs) {
     const int lane = threadIdx.x & 63;
     const int g = jb.g, i0 = jb.i0, i1 = jb.i1, i2 = jb.i2;
     // Every load first and every store last: a single wave's pass is a chain
@@ -1076,7 +723,7 @@ __device__ __forceinline__ int clip_wave(int qi, const ClipJob& jb, const DevSce
         na = min(total, CLIP_VERTS);
         cur ^= 1;
     }
-    // the job's CLIP_PIECES slots: its pieces, the rest empty
+    // the job's CLIP_PIECES records
     const int nsub = max(na - 2, 0);
     const int base = qi * CLIP_PIECES;
     if (base + CLIP_PIECES > cap.clip_subs) {
@@ -1119,16 +766,6 @@ __device__ __forceinline__ int clip_wave(int qi, const ClipJob& jb, const DevSce
     if (lane < nsub)
         ok = pixel_box(sv[0].x, sv[0].y, sv[0].z, sv[1].x, sv[1].y, sv[1].z, sv[2].x, sv[2].y, sv[2].z, vc.W, vc.H,
                        bx0, by0, bx1, by1);
-    // each piece's tiles, spread over the wave
-    for (int p = 0; p < nsub; p++) {
-        if (!__shfl((int)ok, p)) continue;
-        const int tx0 = __shfl(bx0, p) >> vc.rt_shift, ty0 = __shfl(by0, p) >> vc.rt_shift;
-        const int ntx = (__shfl(bx1, p) >> vc.rt_shift) - tx0 + 1, nty = (__shfl(by1, p) >> vc.rt_shift) - ty0 + 1;
-        for (int j = lane; j < ntx * nty; j += 64) {
-            const int ty = j / ntx;
-            atomicAdd(&tile_count[(ty0 + ty) * vc.rtiles_x + tx0 + (j - ty * ntx)], 1);
-        }
-    }
     // the stores
     if (lane == 0) tri_clip_slot[g] = base;
     if (vert) {
@@ -1139,58 +776,58 @@ __device__ __forceinline__ int clip_wave(int qi, const ClipJob& jb, const DevSce
         rp->wp[k] = make_float4(m.x, m.y, m.z, 0.0f);
         rp->uv[k] = uv;
     }
-    if (lane < CLIP_PIECES) {
-        const size_t ps = (size_t)s.n_tris + base + lane;
-        if (ok) store_prim(prims, pbox, ps, sv[0], sv[1], sv[2], (uint32_t)g * 8u + (uint32_t)lane, bx0, by0, bx1, by1);
-        else store_empty(pbox, ps);
-    }
+    if (ok) pairs += box_tiles(bx0, by0, bx1, by1, vc.rt_shift);
+    emit_jobs(ok, sv[0], sv[1], sv[2], (uint32_t)g * 8u + (uint32_t)lane, bx0, by0, bx1, by1, vc.rt_shift + 1, qi, jobs,
+              cnt, wmark);
     return nsub;
 }
 
 // Waves stride over the queue (its length is known on the device only; the
-// grid stays small).  Each workgroup writes its pieces to blk_pieces[its
-// index] for the frame statistics (the tile scan sums them): a counter
-// that every queued triangle hit would serialise them.
+// grid stays small).  Each workgroup writes its pieces, and their raster
+// tiles, to blk_pieces / blk_pairs[its index] for the frame statistics: a
+// counter that every queued triangle hit would serialise them.
 struct k_clip_args {
     DevScene s;
     ViewConsts vc;
     const float4* tv_scr;
     const float4* tv_nor;
     const ClipJob* clip_list;
-    Prim* prims;
-    uint2* pbox;
+    JobQueues jobs;
     ClipRec* clips;
     int32_t* tri_clip_slot;
-    int32_t* tile_count;
     int32_t* blk_pieces;
+    int32_t* blk_pairs;
     Counters* cnt;
     Capacities cap;
     int32_t gx, gy;  // the grid of this launch
 };
 __device__ __forceinline__ void k_clip_body(const k_clip_args& a_, const VB vb) {
     __shared__ V4 s_poly[CLIP_WAVES][2][CLIP_VERTS];
-    __shared__ int32_t s_pieces[CLIP_WAVES];
+    __shared__ int32_t s_mark[CLIP_WAVES * 64];
+    __shared__ int32_t s_pieces, s_pairs;
     Counters* cnt = a_.cnt;
     const int wv = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s_pieces = s_pairs = 0;
+    __syncthreads();
     // the wave's first job is read before the queue's length is known (a
     // slot within the queue's capacity either way; used only if queued)
     const int q0 = __builtin_amdgcn_readfirstlane(vb.bx * CLIP_WAVES + wv);
     ClipJob jb = a_.clip_list[min(q0, a_.cap.clip_tris - 1)];
-    int pieces = 0;
+    int pieces = 0, pairs = 0;
     if (!cnt->overflow) {
         const int n = min(cnt->n_clipped, a_.cap.clip_tris);
         for (int q = q0; q < n; q += vb.gx * CLIP_WAVES) {
             if (q != q0) jb = a_.clip_list[q];
-            pieces += clip_wave(q, jb, a_.s, a_.vc, a_.tv_scr, a_.tv_nor, a_.prims, a_.pbox, a_.clips,
-                                a_.tri_clip_slot, a_.tile_count, cnt, a_.cap, s_poly[wv]);
+            pieces += clip_wave(q, jb, a_.s, a_.vc, a_.tv_scr, a_.tv_nor, a_.jobs, a_.clips, a_.tri_clip_slot, cnt,
+                                a_.cap, s_poly[wv], s_mark + 64 * wv, pairs);
         }
     }
-    if ((threadIdx.x & 63) == 0) s_pieces[wv] = pieces;
+    if ((threadIdx.x & 63) == 0 && pieces) atomicAdd(&s_pieces, pieces);
+    if (pairs) atomicAdd(&s_pairs, pairs);
     __syncthreads();
     if (threadIdx.x == 0) {
-        int t = 0;
-        for (int k = 0; k < CLIP_WAVES; k++) t += s_pieces[k];
-        a_.blk_pieces[vb.bx] = t;
+        a_.blk_pieces[vb.bx] = s_pieces;
+        if (a_.blk_pairs) a_.blk_pairs[vb.bx] = s_pairs;
     }
 }
 __global__ __launch_bounds__(CLIP_WAVES * 64) void k_clip(k_clip_args a) {
@@ -1206,75 +843,10 @@ __global__ __launch_bounds__(CLIP_WAVES * 64) void k_clip_wide(const k_clip_args
 }
 
 // ------------------------------------------------------------- rasters
-namespace {
-// A primitive staged in LDS: the hoisted Barycoord terms, the three depths,
-// the order key and its pixel rectangle inside the tile.
-struct alignas(16) LPrim {
-    float ax, ay, bx, by;
-    float abx, aby, acx, acy;
-    float bcx, bcy, sabc, az;
-    float bz, cz;
-    uint32_t key;
-    uint32_t rect;  // rx0 | ry0<<5 | (w-1)<<10 | ceil(65536 / w)<<15 (tile-local)
-};
-
-// Loads one primitive and intersects its pixel box with the T x T tile;
-// returns the candidate count.
-template <int T>
-__device__ __forceinline__ int stage_prim(const Prim& p, int px0, int py0, LPrim& lp) {
-    uint32_t lo = fbits(p.p2.z), hi = fbits(p.p2.w);
-    int x0 = max((int)(lo & 0xffff), px0), y0 = max((int)(lo >> 16), py0);
-    int x1 = min((int)(hi & 0xffff), px0 + T - 1), y1 = min((int)(hi >> 16), py0 + T - 1);
-    if (x0 > x1 || y0 > y1) return 0;
-    TriSetup t = tri_setup(p.p0.x, p.p0.y, p.p0.w, p.p1.x, p.p1.z, p.p1.w);
-    lp.ax = t.ax, lp.ay = t.ay, lp.bx = t.bx, lp.by = t.by;
-    lp.abx = t.abx, lp.aby = t.aby, lp.acx = t.acx, lp.acy = t.acy;
-    lp.bcx = t.bcx, lp.bcy = t.bcy, lp.sabc = t.sabc;
-    lp.az = p.p0.z, lp.bz = p.p1.y, lp.cz = p.p2.x;
-    lp.key = fbits(p.p2.y);
-    const int w = x1 - x0 + 1, h = y1 - y0 + 1;
-    lp.rect = (uint32_t)(x0 - px0) | ((uint32_t)(y0 - py0) << 5) | ((uint32_t)(w - 1) << 10) |
-              (((65536u + (uint32_t)w - 1u) / (uint32_t)w) << 15);
-    return w * h;
-}
-
-// Candidate idx -> (primitive j, tile-local pixel).  l / w by multiply-shift
-// is exact for l < 1024, w <= 32: the product overshoots l / w by less than
-// l / 65536 < 1/64, and l / w's fraction is at most 1 - 1/w.
-__device__ __forceinline__ void candidate(const int32_t* start, const LPrim* sp, int idx, int& j, int& lx, int& ly) {
-    // the last primitive with start <= idx (empty ranges are skipped), in
-    // eight fixed steps
-    int lo = 0;
-#pragma unroll
-    for (int step = 128; step >= 1; step >>= 1)
-        if (start[lo + step] <= idx) lo += step;
-    j = lo;
-    int l = idx - start[j];
-    uint32_t r = sp[j].rect;
-    int w = ((r >> 10) & 31) + 1;
-    int q = (int)(mul_u24((uint32_t)l, r >> 15) >> 16);
-    lx = (int)(r & 31) + (l - q * w);
-    ly = (int)((r >> 5) & 31) + q;
-}
-
-__device__ __forceinline__ bool eval_candidate(const LPrim& p, float px, float py, float& z) {
-    TriSetup t;
-    t.ax = p.ax, t.ay = p.ay, t.bx = p.bx, t.by = p.by;
-    t.abx = p.abx, t.aby = p.aby, t.acx = p.acx, t.acy = p.acy;
-    t.bcx = p.bcx, t.bcy = p.bcy, t.sabc = p.sabc;
-    return cover_z(t, px, py, p.az, p.bz, p.cz, z);  // raster.go:487-496
-}
-}  // namespace
-
-// Work items of the rasters: (tile, up to ITEM_PRIMS primitives of its
-// list), so that a tile a scene crowds -- a shadow map fitted to the whole
-// camera frustum concentrates the scene in a few hundred of its tiles -- is
-// spread over many workgroups.  k_scan_apply lists each item's tile.
-// Persistent workgroups take items i = blockIdx.x, blockIdx.x + gridDim.x, ...
-// Each item evaluates its candidates (pixel box x tile) exactly as
-// drawClipped / drawDepth do, reduces them in LDS and merges the tile's
-// covered pixels into the target with global atomics (order-independent,
-// and with what the setup drew and the tile's other items):
+// The larger primitives, a wave a job (emit_jobs): the job's rectangle of at
+// most 64 x 64 pixel centres, 64 of them a round, each tested as drawClipped /
+// drawDepth do and merged into the target with a global atomic
+// (order-independent, and with what the setup drew):
 //   MODE_VIS    64-bit min of (~ordered(z) << 32 | triangle*8+sub): largest
 //               depth wins, ties go to the first primitive in sequential
 //               order -- FragmentBuffer.DepthTest/Set under Workers(1)
@@ -1284,114 +856,78 @@ __device__ __forceinline__ bool eval_candidate(const LPrim& p, float px, float p
 //               very first fragment of a pixel);
 //   MODE_SHADOW the running maximum of render/shadow.go:214-228 (maps zeroed
 //               once, never cleared) as a max over ordered depth bits.
+// Persistent workgroups: a wave takes every so-manieth job of one queue.  The
+// job is uniform over the wave, so its record comes through scalar loads, and
+// the rounds step the pixel by 64 along the rectangle's rows without dividing.
+// Bound by the latency of a job's load and its first test where jobs are few,
+// by VALU issue (about 60 instructions a round) where they are many.
 enum { MODE_VIS = 0, MODE_EXACT = 1, MODE_SHADOW = 2 };
 
 struct k_raster_args {
-    const Prim* prims;
-    const int32_t* tile_off;
-    const int32_t* chunk_off;
-    const int32_t* item_tile;
-    const int32_t* tile_list;
+    JobQueues jobs;
     Counters* cnt;
     RasterTarget rt;
-    int32_t cap_items;
-    int32_t item_prims;
     int32_t gx, gy;  // the grid of this launch
 };
-template <int MODE, int T>
+template <int MODE>
 __device__ __forceinline__ void k_raster_body(const k_raster_args& a_, const VB vb) {
-    const int32_t item_prims = a_.item_prims;
-    const Prim* __restrict__ prims = a_.prims;
-    const int32_t* __restrict__ tile_off = a_.tile_off;
-    const int32_t* __restrict__ chunk_off = a_.chunk_off;
-    const int32_t* __restrict__ item_tile = a_.item_tile;
-    const int32_t* __restrict__ tile_list = a_.tile_list;
+    constexpr bool SHADOW = MODE == MODE_SHADOW, EXACT = MODE == MODE_EXACT;
+    const JobQueues& jq = a_.jobs;
     Counters* cnt = a_.cnt;
     const RasterTarget& rt = a_.rt;
-    const int32_t cap_items = a_.cap_items;
-
-    constexpr bool SHADOW = MODE == MODE_SHADOW, EXACT = MODE == MODE_EXACT;
-    constexpr int TP = T * T;  // pixels of a tile: 64, 256 or 1024 (a quarter, one or four per thread)
-    __shared__ LPrim sp[CHUNK];
-    __shared__ int32_t start[CHUNK + 1];
-    __shared__ int32_t wsum[4];
-    __shared__ unsigned long long svis[SHADOW ? 1 : TP];
-    __shared__ uint32_t smax[SHADOW ? TP : 1];
-    __shared__ uint32_t sfirst[EXACT ? TP : 1];
-    __shared__ uint32_t snan[EXACT ? TP : 1];
-    const int tid = threadIdx.x;
-    const int n_items = cnt->n_chunks;
-    if (cnt->overflow || n_items > cap_items) return;
+    const int lane = threadIdx.x & 63;
+    const int w0 = __builtin_amdgcn_readfirstlane(vb.bx * 4 + (threadIdx.x >> 6)), nw = vb.gx * 4;
+    const int qi = w0 & (RASTER_QUEUES - 1);
+    const int n = cnt->overflow ? 0 : __builtin_amdgcn_readfirstlane(min(jq.n[qi * JOB_COUNT_STRIDE], jq.cap));
+    const Prim* jobs = jq.jobs + (size_t)qi * jq.cap;
     bool saw_nan = false;
-    for (int item = vb.bx; item < n_items; item += vb.gx) {
-        const int tile = item_tile[item];
-        const int slot = SHADOW ? tile / rt.tiles_per_map : 0;
-        const int t = SHADOW ? tile % rt.tiles_per_map : tile;
-        const int px0 = (t % rt.tiles_x) * T, py0 = (t / rt.tiles_x) * T;
-        const int first_item = chunk_off[tile];
-        const int beg = tile_off[tile] + (item - first_item) * item_prims;
-        const int n = min(item_prims, tile_off[tile + 1] - beg);
-        for (int pp = tid; pp < TP; pp += 256) {
-            if (SHADOW) smax[pp] = depth_ord(0.0f);
-            else svis[pp] = VIS_EMPTY;
-            if (EXACT) sfirst[pp] = 0xffffffffu, snan[pp] = 0xffffffffu;
-        }
-        for (int b0 = 0; b0 < n; b0 += CHUNK) {
-            int c = 0;
-            if (b0 + tid < n) c = stage_prim<T>(prims[tile_list[beg + b0 + tid]], px0, py0, sp[tid]);
-            block_scan_256(c, start, wsum);
-            const int total = start[CHUNK];
-            for (int idx = tid; idx < total; idx += 256) {
-                int j, lx, ly;
-                candidate(start, sp, idx, j, lx, ly);
-                float z;
-                if (!eval_candidate(sp[j], (float)(px0 + lx) + 0.5f, (float)(py0 + ly) + 0.5f, z)) continue;
-                const int pix = ly * T + lx;
-                const uint32_t key = sp[j].key;
-                if (EXACT) atomicMin(&sfirst[pix], key);
+    // (nw is a multiple of RASTER_QUEUES: the launches see to it)
+    for (int j = w0 / RASTER_QUEUES; j < n; j += nw / RASTER_QUEUES) {
+        const Prim* p = jobs + j;
+        auto u = [](float f) { return bitsf(__builtin_amdgcn_readfirstlane(fbits(f))); };
+        const float4 q0 = p->p0, q1 = p->p1, q2 = p->p2;
+        const uint32_t key = __builtin_amdgcn_readfirstlane(fbits(q2.y));
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(fbits(q2.z)), hi = __builtin_amdgcn_readfirstlane(fbits(q2.w));
+        const TriSetup t = tri_setup(u(q0.x), u(q0.y), u(q0.w), u(q1.x), u(q1.z), u(q1.w));
+        const float az = u(q0.z), bz = u(q1.y), cz = u(q2.x);
+        const int x0 = (int)(lo & 0xffff), y0 = (int)(lo >> 16);
+        const int w = (int)(hi & 0xffff) - x0 + 1, h = (int)(hi >> 16) - y0 + 1;
+        const int q64 = 64 / w, r64 = 64 - q64 * w;  // (uniform) a round's step: rows, then columns
+        // lane / w: exact, lane < 64 and w <= 64
+        int ly = (int)(mul_u24((uint32_t)lane, (65536u + (uint32_t)w - 1u) / (uint32_t)w) >> 16), lx = lane - ly * w;
+        while (ly < h) {
+            const int px = x0 + lx, py = y0 + ly;
+            float z;
+            if (cover_z(t, (float)px + 0.5f, (float)py + 0.5f, az, bz, cz, z)) {  // raster.go:487-496
+                const size_t o = (size_t)py * rt.W + px;
+                if (EXACT) atomicMin(&rt.first_all[o], key);
                 if (z != z) {
                     saw_nan = true;
-                    if (EXACT) atomicMin(&snan[pix], key);
-                    continue;
-                }
-                if (SHADOW) atomicMax(&smax[pix], depth_ord(z));
-                else atomicMin(&svis[pix], ((unsigned long long)depth_key_hi(z) << 32) | key);
-            }
-            __syncthreads();
-        }
-        for (int pp = tid; pp < TP; pp += 256) {
-            const int x = px0 + (pp & (T - 1)), y = py0 + pp / T;
-            // (the setup may have drawn small triangles into the tile, and
-            // other items of it merge here too: an atomic, which needs no
-            // read of the old value first)
-            if (SHADOW) {
-                if (x < rt.W && y < rt.H && smax[pp] > depth_ord(0.0f))
-                    atomicMax(&rt.smap_ord[(size_t)slot * rt.W * rt.H + (size_t)y * rt.W + x], smax[pp]);
-            } else if (x < rt.W && y < rt.H) {
-                const size_t o = (size_t)y * rt.W + x;
-                if (svis[pp] != VIS_EMPTY) atomicMin(&rt.vis[o], svis[pp]);
-                if (EXACT) {
-                    if (sfirst[pp] != 0xffffffffu) atomicMin(&rt.first_all[o], sfirst[pp]);
-                    if (snan[pp] != 0xffffffffu) atomicMin(&rt.first_nan[o], snan[pp]);
+                    if (EXACT) atomicMin(&rt.first_nan[o], key);
+                } else if (SHADOW) {
+                    if (z > 0.0f) atomicMax(&rt.smap_ord[(size_t)key * rt.W * rt.H + o], depth_ord(z));  // the map starts at 0
+                } else {
+                    atomicMin(&rt.vis[o], ((unsigned long long)depth_key_hi(z) << 32) | key);
                 }
             }
+            lx += r64, ly += q64;
+            if (lx >= w) lx -= w, ly++;
         }
-        __syncthreads();
     }
     if (saw_nan) atomicOr(SHADOW ? &cnt->shadow_nan : &cnt->nan_flag, 1);
 }
-template <int MODE, int T>
+template <int MODE>
 __global__ __launch_bounds__(256) void k_raster(k_raster_args a) {
-    k_raster_body<MODE, T>(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
+    k_raster_body<MODE>(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
 }
-template <int MODE, int T>
+template <int MODE>
 __global__ __launch_bounds__(256) void k_raster_wide(const k_raster_args* __restrict__ a, const int32_t* __restrict__ start,
         int32_t n) {
     const int v = wide_view(start, n, (int)blockIdx.x);
     const k_raster_args& x = a[v];
     const int local = (int)blockIdx.x - start[v];
     if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_raster_body<MODE, T>(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
+    k_raster_body<MODE>(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
 }
 
 // Fragment depth per pixel from the visibility key (-1 where uncovered, as
@@ -2266,13 +1802,14 @@ __device__ __forceinline__ void k_shade_bg_body(const k_shade_bg_args& a_, const
     const ShadeConsts& c = a_.c;
     const ShadeBuffers& b = a_.b;
 
-    if (threadIdx.x != 0 || vb.bx != 0) return;
+    if (vb.bx != 0) return;
     // the frame's counters are final here: hand them to the host's pinned
     // copy (main then shadow), in place of a copy after the frame
-    if (b.cnt_host)
-        for (int i = 0; i < (int)(2 * sizeof(Counters) / 4); i++)
-            reinterpret_cast<int32_t*>(b.cnt_host)[i] = reinterpret_cast<const int32_t*>(b.cnt)[i];
-    if (b.cnt->overflow) return;
+    constexpr int CW = sizeof(Counters) / 4;
+    if (b.cnt_host && threadIdx.x < 2 * CW)
+        reinterpret_cast<int32_t*>(b.cnt_host)[threadIdx.x] =
+            reinterpret_cast<const int32_t*>(&b.cnt[threadIdx.x / CW].c)[threadIdx.x % CW];
+    if (threadIdx.x != 0 || b.cnt->c.overflow) return;
     const uint64_t k00 = b.vis[0];
     float lin[3] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
     uint32_t col = c.background;
@@ -2364,7 +1901,7 @@ __device__ __forceinline__ void k_shade_body(const k_shade_args& a_, const VB vb
     const ShadeConsts& c = a_.c;
     const ShadeBuffers& b = a_.b;
 
-    if (b.cnt->overflow) return;
+    if (b.cnt->c.overflow) return;
     const int tiles_x = c.v.tiles_x, tiles_y = c.v.tiles_y;
     // workgroup i shades tile i: the dispatcher deals consecutive
     // workgroups round-robin to the 8 XCDs, so every XCD gets a share of
@@ -2411,7 +1948,7 @@ __global__ __launch_bounds__(256) void k_shadow_count(DevScene s, ShadeConsts c,
 // -- what k_shade does after shade_fragment.
 __global__ __launch_bounds__(256) void k_shade_post(DevScene s, ShadeConsts c, ShadeBuffers b) {
     const size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (o >= (size_t)c.v.W * c.v.H || b.cnt->overflow) return;
+    if (o >= (size_t)c.v.W * c.v.H || b.cnt->c.overflow) return;
     const int x = (int)(o % (size_t)c.v.W), y = (int)(o / (size_t)c.v.W);
     const uint8_t flag = b.post_flag[o];  // (the first half's: no dependent loads here)
     uint32_t col;
@@ -2595,7 +2132,10 @@ void launch_vertex_main(hipStream_t st, const DevScene& s, const M4* trans, cons
                         float4* tv_scr, float4* tv_nor, float4* tv_wp, uint32_t* tv_col, float2* tv_uv,
                         const FrameClear& clr) {
     if (!s.n_tverts) return clear_alone(st, clr);
-    go(k_vertex_main, k_vertex_main_wide, dim3(blocks_for(s.n_tverts, 256)), 256, st,
+    // enough workgroups for the clear too (4 keys a thread): a frame of few
+    // vertices cleared 1600 x 1200 pixels with three workgroups, in 74 us
+    const unsigned clear = std::min<size_t>(blocks_for(clr.n_vis, 1024), 2048);
+    go(k_vertex_main, k_vertex_main_wide, dim3(std::max(blocks_for(s.n_tverts, 256), clear)), 256, st,
        k_vertex_main_args{s, trans, normal, vc, tv_scr, tv_nor, tv_wp, tv_col, tv_uv, clr, 0, 0});
 }
 void launch_vertex_shadow(hipStream_t st, const DevScene& s, const M4* strans, const ShadowConsts& sc, float3* ts,
@@ -2607,23 +2147,22 @@ void launch_vertex_shadow(hipStream_t st, const DevScene& s, const M4* strans, c
 int setup_blocks(int32_t n_tris) { return (n_tris + 255) / 256; }
 int clip_grid(const Capacities& cap) { return (int)std::min<size_t>(blocks_for(cap.clip_tris, CLIP_WAVES), CLIP_GRID); }
 void launch_setup_main(hipStream_t st, const DevScene& s, const ViewConsts& vc, const float4* tv_scr,
-                       const float4* tv_nor, Prim* prims, uint2* pbox, ClipRec* clips, int32_t* tri_clip_slot,
-                       ClipJob* clip_list, int32_t* tile_count, int32_t* blk_prims, Counters* cnt, Capacities cap,
+                       const float4* tv_nor, const JobQueues& jobs, ClipRec* clips, int32_t* tri_clip_slot,
+                       ClipJob* clip_list, int32_t* blk_prims, int32_t* blk_pairs, Counters* cnt, Capacities cap,
                        unsigned long long* vis, int32_t draw_small, const int4* tri_rec) {
     if (!s.n_tris) return;
-    go(k_setup_main, k_setup_main_wide, dim3(setup_blocks(s.n_tris)), 256, st,
-       k_setup_main_args{s, vc, tv_scr, prims, pbox, clip_list, tile_count, blk_prims, cnt, cap, vis, draw_small,
-                         tri_rec, 0, 0});
+    const int nb = setup_blocks(s.n_tris);
+    go(k_setup_main, k_setup_main_wide, dim3(nb), 256, st,
+       k_setup_main_args{s, vc, tv_scr, clip_list, jobs, blk_prims, blk_pairs, cnt, cap, vis, draw_small, tri_rec, 0, 0});
     go(k_clip, k_clip_wide, dim3(clip_grid(cap)), CLIP_WAVES * 64, st,
-       k_clip_args{s, vc, tv_scr, tv_nor, clip_list, prims, pbox, clips, tri_clip_slot, tile_count,
-                   blk_prims + setup_blocks(s.n_tris), cnt, cap, 0, 0});
+       k_clip_args{s, vc, tv_scr, tv_nor, clip_list, jobs, clips, tri_clip_slot, blk_prims + nb,
+                   blk_pairs ? blk_pairs + nb : nullptr, cnt, cap, 0, 0});
 }
 void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& sc, const int4* tri_rec,
-                         const float3* ts, Prim* prims, uint2* pbox, int32_t* tile_count, Counters* cnt, Capacities cap,
-                         uint32_t* smaps) {
+                         const float3* ts, const JobQueues& jobs, Counters* cnt, uint32_t* smaps) {
     if (!s.n_tris || !sc.n_slots) return;
     go(k_setup_shadow, k_setup_shadow_wide, dim3(blocks_for(s.n_tris, 256), sc.n_slots), 256, st,
-       k_setup_shadow_args{s, sc, tri_rec, ts, prims, pbox, tile_count, cnt, cap, smaps, 0, 0});
+       k_setup_shadow_args{s, sc, tri_rec, ts, jobs, cnt, smaps, 0, 0});
 }
 // Each global triangle's record, fixed by the scene (k_tri_rec).
 __global__ __launch_bounds__(256) void k_tri_rec(DevScene s, int4* tri_rec) {
@@ -2646,43 +2185,14 @@ __global__ __launch_bounds__(256) void k_tri_rec(DevScene s, int4* tri_rec) {
 void launch_tri_rec(hipStream_t st, const DevScene& s, int4* tri_rec) {
     if (s.n_tris) hipLaunchKernelGGL(k_tri_rec, dim3(blocks_for(s.n_tris, 256)), dim3(256), 0, st, s, tri_rec);
 }
-int scan_blocks(int32_t n) { return std::max(1, (n + SCAN_BLOCK - 1) / SCAN_BLOCK); }
-void launch_scan(hipStream_t st, int32_t* counts, int32_t n, int32_t* offsets, int32_t* chunk_off, int32_t* cursor,
-                 int32_t* bsum, int32_t* item_tile, int32_t cap_items, const int32_t* blk_prims, int32_t n_blk,
-                 Counters* cnt, int32_t item_prims) {
-    const int nb = n <= SCAN_WHOLE_MAX ? 1 : scan_blocks(n);
-    // (the sums stage always records, so the apply stage keeps its place)
-    if (g_wide) g_wide->sub = 0;
-    if (nb > 1)
-        go(k_scan_sums, k_scan_sums_wide, dim3(nb), 1024, st, k_scan_sums_args{counts, n, bsum, item_prims, 0, 0});
-    if (g_wide) g_wide->sub = 1;
-    go(k_scan_apply, k_scan_apply_wide, dim3(nb), 1024, st,
-       k_scan_apply_args{counts, n, bsum, offsets, chunk_off, cursor, item_tile, cap_items, blk_prims, n_blk,
-                         cnt, item_prims, 0, 0});
-}
-void launch_bin(hipStream_t st, const uint2* pbox, Counters* cnt, int32_t tiles_x, int32_t shift, int32_t tiles_per_view,
-                int32_t shadow, int32_t* cursor, int32_t* list, Capacities cap, int32_t n_fixed, int32_t n_tris) {
-    const int max_prims = n_fixed + (shadow ? 0 : cap.clip_subs);
-    if (max_prims <= 0) return;
-    go(k_bin, k_bin_wide, dim3(blocks_for(max_prims, 256)), 256, st,
-       k_bin_args{pbox, cnt, tiles_x, shift, tiles_per_view, shadow, cursor, list, cap, n_fixed, n_tris, 0, 0});
-}
-template <int MODE>
-static void launch_raster_t(hipStream_t st, int tile, int n_workgroups, const k_raster_args& a) {
-    // (in a recorded batch each tile side is a group of its own in the
-    // stage, so views with different tiles still share wide launches)
-    if (g_wide) g_wide->sub = tile == 8 ? 0 : tile == 16 ? 1 : 2;
-    if (tile == 8) go(k_raster<MODE, 8>, k_raster_wide<MODE, 8>, dim3(n_workgroups), 256, st, a);
-    else if (tile == 32) go(k_raster<MODE, 32>, k_raster_wide<MODE, 32>, dim3(n_workgroups), 256, st, a);
-    else go(k_raster<MODE, 16>, k_raster_wide<MODE, 16>, dim3(n_workgroups), 256, st, a);
-}
-void launch_raster(hipStream_t st, int mode, int n_workgroups, const Prim* prims, const int32_t* tile_off,
-                   const int32_t* chunk_off, int32_t* item_tile, int32_t cap_items, const int32_t* tile_list,
-                   Counters* cnt, const RasterTarget& rt, int32_t item_prims, int32_t tile) {
-    const k_raster_args a{prims, tile_off, chunk_off, item_tile, tile_list, cnt, rt, cap_items, item_prims, 0, 0};
-    if (mode == MODE_SHADOW) launch_raster_t<MODE_SHADOW>(st, tile, n_workgroups, a);
-    else if (mode == MODE_EXACT) launch_raster_t<MODE_EXACT>(st, tile, n_workgroups, a);
-    else launch_raster_t<MODE_VIS>(st, tile, n_workgroups, a);
+void launch_raster(hipStream_t st, int mode, int n_workgroups, const JobQueues& jobs, Counters* cnt,
+                   const RasterTarget& rt) {
+    const k_raster_args a{jobs, cnt, rt, 0, 0};
+    // (four waves a workgroup: every queue gets the same number of waves)
+    const dim3 grid((n_workgroups + RASTER_QUEUES / 4 - 1) / (RASTER_QUEUES / 4) * (RASTER_QUEUES / 4));
+    if (mode == MODE_SHADOW) go(k_raster<MODE_SHADOW>, k_raster_wide<MODE_SHADOW>, grid, 256, st, a);
+    else if (mode == MODE_EXACT) go(k_raster<MODE_EXACT>, k_raster_wide<MODE_EXACT>, grid, 256, st, a);
+    else go(k_raster<MODE_VIS>, k_raster_wide<MODE_VIS>, grid, 256, st, a);
 }
 void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters* cnt, float* depth, const DevScene& s,
                     int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec) {
@@ -2694,7 +2204,7 @@ void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters
 void launch_ao(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b) {
     const int nb = ((c.v.W + 63) / 64) * c.v.H;
     go(k_ao, k_ao_wide, dim3(((nb + 7) / 8) * 8), 256, st,
-       k_ao_args{c, b.ao_xs, b.ao_cnt, b.depth, b.ao, b.ao_tab, b.ao_fast, b.cnt, 0, 0});
+       k_ao_args{c, b.ao_xs, b.ao_cnt, b.depth, b.ao, b.ao_tab, b.ao_fast, &b.cnt->c, 0, 0});
 }
 void launch_shade_bg(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b) {
     go(k_shade_bg, k_shade_bg_wide, dim3(1), 64, st, k_shade_bg_args{s, c, b, 0, 0});

@@ -54,7 +54,7 @@ struct ShadeBuffers {
     float* linear;             // optional [H][W][3]
     uint32_t* bg;              // [2] uncovered colour, pixel (0,0)'s colour
     float* bg_lin;             // [3]
-    const Counters* cnt;       // main-pass counters, then the shadow ones: nothing is shaded after an overflow
+    const PassCounters* cnt;   // the main view's, then the shadow passes': nothing is shaded after an overflow
     Counters* cnt_host;        // pinned host copy of both, written once they are final
     float* ao;                 // [H][W] AO factor of the pixels that need it
     int32_t* ao_xs;            // [H][W] per row, the columns of the pixels k_ao computes, left to right (k_resolve)
@@ -182,34 +182,21 @@ void launch_vertex_shadow(hipStream_t st, const DevScene& s, const gm::M4* stran
 constexpr int CLIP_GRID = 512;
 int setup_blocks(int32_t n_tris);
 int clip_grid(const Capacities& cap);
-// pbox: the pixel box of every primitive slot (k_bin's input)
+// blk_pairs (may be null): likewise the raster tiles the primitives left to the
+// raster touch
 void launch_setup_main(hipStream_t st, const DevScene& s, const ViewConsts& vc, const float4* tv_scr,
-                       const float4* tv_nor, Prim* prims, uint2* pbox, ClipRec* clips, int32_t* tri_clip_slot,
-                       ClipJob* clip_list, int32_t* tile_count, int32_t* blk_prims, Counters* cnt, Capacities cap,
+                       const float4* tv_nor, const JobQueues& jobs, ClipRec* clips, int32_t* tri_clip_slot,
+                       ClipJob* clip_list, int32_t* blk_prims, int32_t* blk_pairs, Counters* cnt, Capacities cap,
                        unsigned long long* vis, int32_t draw_small, const int4* tri_rec);
 void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& sc, const int4* tri_rec,
-                         const float3* ts, Prim* prims, uint2* pbox, int32_t* tile_count, Counters* cnt, Capacities cap,
-                         uint32_t* smaps);
+                         const float3* ts, const JobQueues& jobs, Counters* cnt, uint32_t* smaps);
 // Each global triangle's record, fixed by the scene: its transformed
 // vertices and its material in the flat table (-1: vertex colour, matAt's
 // rule), or x = -1 when Triangle.IsValid is false.  Once per renderer.
 void launch_tri_rec(hipStream_t st, const DevScene& s, int4* tri_rec);
-// n_blk > 0: also sum the per-workgroup primitive counts of the setup and
-// the clipper (blk_prims) into the frame statistics (the main view)
-// bsum: 2 * scan_blocks(n) ints of scratch
-int scan_blocks(int32_t n);
-// Also lists each work item's tile in item_tile and zeroes the counts.
-void launch_scan(hipStream_t st, int32_t* counts, int32_t n, int32_t* offsets, int32_t* chunk_off, int32_t* cursor,
-                 int32_t* bsum, int32_t* item_tile, int32_t cap_items, const int32_t* blk_prims, int32_t n_blk,
-                 Counters* cnt, int32_t item_prims);
-// shift: log2 of the raster tile side
-void launch_bin(hipStream_t st, const uint2* pbox, Counters* cnt, int32_t tiles_x, int32_t shift, int32_t tiles_per_view,
-                int32_t shadow, int32_t* cursor, int32_t* list, Capacities cap, int32_t n_fixed, int32_t n_tris);
-// mode: 0 visibility, 1 visibility in exact order (NaN rule), 2 shadow maps;
-// tile: the raster tile side, 8, 16 or 32
-void launch_raster(hipStream_t st, int mode, int n_workgroups, const Prim* prims, const int32_t* tile_off,
-                   const int32_t* chunk_off, int32_t* item_tile, int32_t cap_items, const int32_t* tile_list,
-                   Counters* cnt, const RasterTarget& rt, int32_t item_prims, int32_t tile);
+// mode: 0 visibility, 1 visibility in exact order (NaN rule), 2 shadow maps
+void launch_raster(hipStream_t st, int mode, int n_workgroups, const JobQueues& jobs, Counters* cnt,
+                   const RasterTarget& rt);
 void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters* cnt, float* depth, const DevScene& s,
                     int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec);
 void launch_ao(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b);

@@ -12,9 +12,13 @@ namespace prh {
 
 constexpr int TILE = 16;                 // shading tile side (pixels): one 256-thread workgroup
 constexpr int TILE_PX = TILE * TILE;     // 256 pixels = 4 wave64s
-// The raster tile (binning and the binned raster) is a tuning knob of its
-// own: 8, 16 or 32 pixels a side (prh_tuning.raster_tile).
-constexpr int RTILE_MIN = 8, RTILE_MAX = 32;
+// The raster tile is a tuning knob (8, 16 or 32 pixels a side,
+// prh_tuning.raster_tile): a raster job is a rectangle of at most two tiles a
+// side.  The larger primitives' jobs are spread over RASTER_QUEUES queues, their
+// counts a cache line apart (a power of two, and a multiple of a workgroup's
+// four waves): with one counter the waves' atomics to it, 8 ns each, took as
+// long as the setup.
+constexpr int RASTER_QUEUES = 16, JOB_COUNT_STRIDE = 16;
 constexpr uint32_t SUB_DIRECT = 7;       // key sub-index of an unclipped triangle
 constexpr uint64_t VIS_EMPTY = ~0ull;    // no fragment
 constexpr uint32_t KEY_HI_NAN = 0u;      // NaN-depth winner (exact-order pass only)
@@ -85,7 +89,7 @@ struct ViewConsts {
     gm::M4 vp, vpinv, pinv, vinv, s2w;
     float cam[3];
     int32_t W, H, tiles_x, tiles_y;  // shading tiles (TILE)
-    int32_t rtiles_x, rt_shift;      // raster tiles: per row, log2 of the side
+    int32_t rt_shift;                // raster tiles: log2 of the side
     int32_t perspect;
     float vpbox_max_x, vpbox_max_y;  // viewport AABB max (MSAA*W, MSAA*H)
 };
@@ -93,18 +97,24 @@ struct ViewConsts {
 // Per-frame shadow constants (all shadow-casting lights at once).
 struct ShadowConsts {
     gm::M4 vp;                 // ViewportMatrix(SW, SH)
-    int32_t SW, SH, tiles_x, tiles_y;  // raster tiles of one map
-    int32_t n_slots, tiles_per_map, rt_shift;
+    int32_t SW, SH;
+    int32_t n_slots, rt_shift;
     float vpbox_max_x, vpbox_max_y;  // cullViewFrustum's box: (SW*MSAA, SH*MSAA) (render/cull.go:16-22)
     int32_t direct_max;              // triangles of at most this many texel centres are drawn by the setup
 };
 
-// A rasterisable primitive: a whole triangle (sub = 7) or one clipped fan
-// piece.  p2.y holds the order key (main view) or the shadow slot.
+// A raster job: a rectangle of the pixel box of a whole triangle (sub = 7) or
+// of one clipped fan piece.  p2.y holds the order key (main view) or the shadow
+// slot, p2.z and p2.w the rectangle's corners.
 struct Prim {
     float4 p0;  // ax ay az bx
     float4 p1;  // by bz cx cy
     float4 p2;  // cz key bbox_lo bbox_hi (bit patterns)
+};
+struct JobQueues {
+    Prim* jobs;   // [RASTER_QUEUES][cap]
+    int32_t* n;   // [RASTER_QUEUES * JOB_COUNT_STRIDE], zeroed at the frame's start
+    int32_t cap;
 };
 
 // Vertex data of one clipped fan piece (render/clipping.go:67-157).
@@ -117,8 +127,8 @@ struct ClipRec {
 
 // A triangle queued for the clipper by the setup: its global index, its
 // transformed vertices and the offset from those to its mesh vertices
-// (colours, UVs).  Its fan pieces take the primitive slots
-// n_tris + CLIP_PIECES * (queue position) + piece.
+// (colours, UVs).  Its fan pieces take the clip records CLIP_PIECES * (queue
+// position) + piece.
 struct ClipJob {
     int32_t g, i0, i1, i2;
     int32_t dv, pad[3];
@@ -126,31 +136,31 @@ struct ClipJob {
 constexpr int CLIP_PIECES = 7;  // a triangle clipped by six planes keeps at most 9 vertices: 7 pieces
 
 struct Counters {
-    int32_t n_prims;
     int32_t n_clipped;      // triangles queued for the clipper
-    int32_t n_pairs;        // (primitive, tile) pairs
     int32_t nan_flag;
     int32_t overflow;
     int32_t shadow_nan;
-    int32_t n_chunks;       // raster work items: (tile, up to ITEM_PRIMS primitives)
-    int32_t next_item;      // persistent raster work queue head
+    int32_t need_jobs;      // after an overflow: the most jobs one queue was asked for
     int32_t depth_nonfinite;  // some pixel's resolved depth is NaN or infinite
-    int32_t pad[7];
+    int32_t pad[10];
+};
+// A pass's counters and its queues' job counts, zeroed together.
+struct PassCounters {
+    Counters c;
+    int32_t jobs[RASTER_QUEUES * JOB_COUNT_STRIDE];
 };
 
 struct Capacities {
-    int32_t prims;
     int32_t clip_subs;
-    int32_t pairs;
     int32_t clip_tris;
+    int32_t jobs;  // per raster queue
 };
 
-constexpr int CHUNK = 256;          // primitives staged in LDS at once
-constexpr int ITEM_PRIMS = 2048;    // primitives per raster work item (the default; prh_tuning.item_prims)
+constexpr int ITEM_PRIMS = 2048;    // prh_tuning.item_prims' default
 
 // Where a raster pass writes.
 struct RasterTarget {
-    int32_t W, H, tiles_x, tiles_per_map, n_tiles;
+    int32_t W, H;
     unsigned long long* vis;  // main view: 64-bit depth|order keys
     uint32_t* first_all;      // exact-order pass: first fragment per pixel
     uint32_t* first_nan;      // exact-order pass: first NaN-depth fragment

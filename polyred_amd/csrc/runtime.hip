@@ -400,9 +400,8 @@ struct prh_renderer {
     prh_camera cam;
     prh_options opt;
     int W, H, tiles_x, tiles_y, n_tiles;  // the MSAA-sized framebuffer (width*MSAA x height*MSAA), shading tiles
-    int rtile, rtiles_x, rtiles_y, n_rtiles;  // its raster tiles (prh_tuning.raster_tile)
     int msaa, OW, OH;                       // MSAA factor and the output image size
-    int SW, SH, stiles_x, stiles_y, stiles_per_map, n_slots;  // shadow maps and their raster tiles
+    int SW, SH, n_slots;                    // shadow maps
     ViewConsts vc;
     ShadowConsts shc;
     ShadeConsts sh;
@@ -414,27 +413,19 @@ struct prh_renderer {
     int4* tri_rec;     // per triangle: transformed vertices and flat material (once, k_tri_rec)
     uint32_t* tv_col;  // per transformed vertex: colour
     float2* tv_uv;     // and UV (scenes with textures)
-    Prim* prims;
-    uint2* pbox;  // pixel box per primitive slot
+    JobQueues jobs;    // the raster's queues
     ClipRec* clips;
     int32_t* tri_clip_slot;
-    int32_t* blk_prims;  // per setup / clipper workgroup: unclipped primitives, pieces (statistics)
-    int32_t* scan_sums;  // per scan block: primitive and work-item sums
-    int32_t *tile_count, *tile_off, *chunk_off, *tile_cursor, *tile_list, *item_tile;
+    // per setup / clipper workgroup: unclipped primitives, pieces; and the
+    // raster tiles of those the raster draws (statistics)
+    int32_t *blk_prims, *blk_pairs;
     ClipJob* clip_list;
-    int32_t cap_items;
-    // the shadow passes' own work set (they run beside the main view's)
-    Prim* s_prims;
-    uint2* s_pbox;
-    int32_t *s_scan_sums, *s_tile_count, *s_tile_off, *s_chunk_off, *s_tile_cursor, *s_tile_list, *s_item_tile;
-    int32_t s_cap_items;
-    int32_t s_tile_slots;  // shadow slots x tiles per map
+    JobQueues s_jobs;  // the shadow passes' own queues (they run beside the main view's)
     hipEvent_t ev_fork, ev_join, ev_s[2];
     // split shading: resolve done, the shadow passes done, the AO's span
     hipEvent_t ev_res, ev_sdone, ev_sh[2];
     uint32_t* col_pre;            // split shading: the colour before AO
     uint8_t* post_flag;           // and what its second half does per pixel
-    int32_t tile_slots;
     int32_t n_cu;
     uint32_t *first_all, *first_nan;
     uint64_t* vis;
@@ -449,7 +440,7 @@ struct prh_renderer {
     int32_t *ao_xs, *ao_cnt;  // scenes with AO only: the rows' lists of AO pixels
     float* ao_tab;   // AO march tables (ao_tables)
     int32_t ao_fast; // the tables hold for this frame size
-    Counters* cnt;      // [2]: main, shadow
+    PassCounters* cnt;  // [2]: main, shadow
     Counters* h_cnt;    // pinned
     Counters* d_h_cnt;  // its device address
     Capacities cap_main, cap_shadow;
@@ -473,6 +464,7 @@ struct prh_renderer {
     // the last frame's per-pass times wait in its events until the stats are
     // read (prh_last_stats): a frame's own host work stays short
     bool times_pending, times_nan_rerun;
+    bool counts_pending;  // likewise the primitive and tile counts, in blk_prims and blk_pairs
 };
 
 namespace {
@@ -491,44 +483,26 @@ void free_list(std::vector<void*>& v) {
     v.clear();
 }
 
-// The raster tile grid of the main view and of the shadow maps for the
-// renderer's raster_tile knob (8, 16 or 32), into its constants.
-void raster_grid(prh_renderer* r) {
+// The raster_tile knob (8, 16 or 32) into the renderer's constants.
+void raster_tile(prh_renderer* r) {
     const int T = r->tune.raster_tile, shift = T == 8 ? 3 : T == 32 ? 5 : 4;
-    r->rtile = T;
-    r->rtiles_x = (r->W + T - 1) / T, r->rtiles_y = (r->H + T - 1) / T;
-    r->n_rtiles = r->rtiles_x * r->rtiles_y;
-    r->stiles_x = (r->SW + T - 1) / T, r->stiles_y = (r->SH + T - 1) / T;
-    r->stiles_per_map = r->stiles_x * r->stiles_y;
-    r->vc.rtiles_x = r->rtiles_x, r->vc.rt_shift = shift;
-    r->sh.v.rtiles_x = r->rtiles_x, r->sh.v.rt_shift = shift;
-    r->shc.tiles_x = r->stiles_x, r->shc.tiles_y = r->stiles_y;
-    r->shc.tiles_per_map = r->stiles_per_map, r->shc.rt_shift = shift;
+    r->vc.rt_shift = r->sh.v.rt_shift = r->shc.rt_shift = shift;
 }
 
 int alloc_work(prh_renderer* r) {
     int rc;
-    if ((rc = ralloc(r, &r->prims, (size_t)r->cap_main.prims))) return rc;
-    if ((rc = ralloc(r, &r->pbox, (size_t)r->cap_main.prims))) return rc;
+    if ((rc = ralloc(r, &r->jobs.jobs, (size_t)RASTER_QUEUES * r->cap_main.jobs))) return rc;
     if ((rc = ralloc(r, &r->clips, (size_t)r->cap_main.clip_subs))) return rc;
-    if ((rc = ralloc(r, &r->tile_list, (size_t)r->cap_main.pairs))) return rc;
     if ((rc = ralloc(r, &r->clip_list, (size_t)r->cap_main.clip_tris))) return rc;
-    // every item holds >= 1 primitive of one tile: items <= tiles + pairs / item_prims
-    r->cap_items = r->tile_slots + r->cap_main.pairs / r->tune.item_prims + 1;
-    if ((rc = ralloc(r, &r->item_tile, (size_t)r->cap_items))) return rc;
+    r->jobs.cap = r->cap_main.jobs, r->jobs.n = r->cnt[0].jobs;
     if (r->n_slots > 0) {
-        if ((rc = ralloc(r, &r->s_prims, (size_t)r->cap_shadow.prims))) return rc;
-        if ((rc = ralloc(r, &r->s_pbox, (size_t)r->cap_shadow.prims))) return rc;
-        if ((rc = ralloc(r, &r->s_tile_list, (size_t)r->cap_shadow.pairs))) return rc;
-        r->s_cap_items = r->s_tile_slots + r->cap_shadow.pairs / r->tune.item_prims + 1;
-        if ((rc = ralloc(r, &r->s_item_tile, (size_t)r->s_cap_items))) return rc;
+        if ((rc = ralloc(r, &r->s_jobs.jobs, (size_t)RASTER_QUEUES * r->cap_shadow.jobs))) return rc;
+        r->s_jobs.cap = r->cap_shadow.jobs, r->s_jobs.n = r->cnt[1].jobs;
     }
     return PRH_OK;
 }
 void free_work(prh_renderer* r) {
-    for (void* p : {(void*)r->prims, (void*)r->pbox, (void*)r->clips, (void*)r->tile_list, (void*)r->clip_list,
-                    (void*)r->item_tile, (void*)r->s_prims, (void*)r->s_pbox, (void*)r->s_tile_list,
-                    (void*)r->s_item_tile}) {
+    for (void* p : {(void*)r->jobs.jobs, (void*)r->clips, (void*)r->clip_list, (void*)r->s_jobs.jobs}) {
         if (!p) continue;
         auto it = std::find(r->allocs.begin(), r->allocs.end(), p);
         if (it != r->allocs.end()) {
@@ -536,6 +510,7 @@ void free_work(prh_renderer* r) {
             r->allocs.erase(it);
         }
     }
+    r->jobs.jobs = nullptr, r->clips = nullptr, r->clip_list = nullptr, r->s_jobs.jobs = nullptr;
 }
 
 }  // namespace
@@ -953,10 +928,10 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     shc.vpbox_max_x = (float)(msaa * r->SW), shc.vpbox_max_y = (float)(msaa * r->SH);
     shc.direct_max = r->tune.shadow_direct_max;
 
-    raster_grid(r);
     ShadeConsts& sh = r->sh;
     memset(&sh, 0, sizeof sh);
     sh.v = vc;
+    raster_tile(r);
     gamma_table(sh.gamma_lut);
     memcpy(&sh.background, o->background, 4);
     sh.shadow_map = o->shadow_map != 0;
@@ -986,18 +961,14 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
 
     const size_t P = (size_t)r->W * r->H;
     const int Tg = s->d.n_tris, Vt = s->d.n_tverts;
-    // primitive slots: one per triangle (per shadow slot), then the main
-    // view's clipped fan pieces
-    const int clip_tris = std::min(Tg, 1 << 16) + 16, clip0 = CLIP_PIECES * clip_tris;
-    // the tile tables hold the smallest raster tile's grid, so the tile
-    // knob never reallocates them
-    const int rt_cap = ((r->W + RTILE_MIN - 1) / RTILE_MIN) * ((r->H + RTILE_MIN - 1) / RTILE_MIN);
-    const int st_cap = ((r->SW + RTILE_MIN - 1) / RTILE_MIN) * ((r->SH + RTILE_MIN - 1) / RTILE_MIN);
-    r->cap_main = Capacities{Tg + clip0, clip0, 4 * Tg + 4 * rt_cap + 1024, clip_tris};
-    r->cap_shadow = Capacities{std::max(1, r->n_slots) * Tg, 0,
-                               std::max(1, r->n_slots) * (2 * Tg + 4 * st_cap) + 1024, 0};
-    r->tile_slots = rt_cap + 1;
-    r->s_tile_slots = r->n_slots * st_cap + 1;
+    const int clip_tris = std::min(Tg, 1 << 16) + 16;
+    // A raster queue's first capacity (grown when a frame overflows it): its
+    // share of every triangle at one job (of a quarter of them for the maps,
+    // whose triangles are mostly drawn by the setup), and the jobs of a few
+    // triangles that cover the screen, which their workgroup sends to one queue
+    r->cap_main = Capacities{CLIP_PIECES * clip_tris, clip_tris, (int32_t)(Tg / RASTER_QUEUES + P / 256 + 1024)};
+    r->cap_shadow = Capacities{0, 0, (int32_t)((int64_t)r->n_slots * Tg / (4 * RASTER_QUEUES) +
+                                               (int64_t)r->SW * r->SH / 256 + 1024)};
     int rc = 0;
     auto chk = [&](int v) {
         if (!rc) rc = v;
@@ -1038,23 +1009,11 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     if (!rc) chk(ralloc(r, &r->ts, (size_t)std::max(1, r->n_slots) * Vt));
     if (!rc) chk(ralloc(r, &r->tri_clip_slot, Tg));
     if (!rc) chk(ralloc(r, &r->blk_prims, (size_t)setup_blocks(Tg) + CLIP_GRID));
-    if (!rc) chk(ralloc(r, &r->scan_sums, 2 * (size_t)scan_blocks(r->tile_slots)));
-    if (!rc) chk(ralloc(r, &r->tile_count, r->tile_slots));
-    if (!rc) chk(ralloc(r, &r->tile_off, r->tile_slots + 1));
-    if (!rc) chk(ralloc(r, &r->chunk_off, r->tile_slots + 1));
-
+    if (!rc) chk(ralloc(r, &r->blk_pairs, (size_t)setup_blocks(Tg) + CLIP_GRID));
     // (outside the exact-order pass these two are the adjoint's pixel list and
     // its chunk table, with its count of chunks)
     if (!rc) chk(ralloc(r, &r->first_all, P));
     if (!rc) chk(ralloc(r, &r->first_nan, std::max(P, 2 * diff_chunks(vc) + 2)));
-    if (!rc) chk(ralloc(r, &r->tile_cursor, r->tile_slots));
-    if (!rc && r->n_slots > 0) {
-        chk(ralloc(r, &r->s_scan_sums, 2 * (size_t)scan_blocks(r->s_tile_slots)));
-        if (!rc) chk(ralloc(r, &r->s_tile_count, r->s_tile_slots));
-        if (!rc) chk(ralloc(r, &r->s_tile_off, r->s_tile_slots + 1));
-        if (!rc) chk(ralloc(r, &r->s_chunk_off, r->s_tile_slots + 1));
-        if (!rc) chk(ralloc(r, &r->s_tile_cursor, r->s_tile_slots));
-    }
     if (!rc) chk(ralloc(r, &r->vis, P));
     if (!rc) chk(ralloc(r, &r->depth, P));
     if (!rc) chk(ralloc(r, &r->ao, P));
@@ -1114,10 +1073,6 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     // (stored as ordered depth bits).
     launch_fill_u32(ctx->stream, r->smaps, (size_t)std::max(1, r->n_slots) * r->SW * r->SH, depth_ord(0.0f));
     launch_tri_rec(ctx->stream, s->d, r->tri_rec);
-    // tile counts start at zero; every scan leaves them at zero
-    launch_fill_u32(ctx->stream, reinterpret_cast<uint32_t*>(r->tile_count), r->tile_slots, 0u);
-    if (r->n_slots > 0)
-        launch_fill_u32(ctx->stream, reinterpret_cast<uint32_t*>(r->s_tile_count), r->s_tile_slots, 0u);
     {
         int n_cu = 0;
         if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess || n_cu <= 0)
@@ -1164,8 +1119,6 @@ int prh_renderer_free(prh_renderer* r) {
 
 namespace {
 
-int d_n_tris(const prh_renderer* r) { return r->sc->d.n_tris; }
-
 // Where the frame's final image goes: the renderer's own, or the surface
 // texture a prh_surface_render is drawing into.
 uint32_t* final_image(const prh_renderer* r) { return r->present_to ? r->present_to : r->image; }
@@ -1195,18 +1148,17 @@ ShadeBuffers shade_buffers(const prh_renderer* r) {
 // status means part of the frame may be enqueued and none of it is valid.
 int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bool wide = false) {
     const DevScene& d = r->sc->d;
-    Counters* cm = r->cnt;
-    Counters* cs = r->cnt + 1;
+    Counters* cm = &r->cnt[0].c;
+    Counters* cs = &r->cnt[1].c;
     const int persistent = wide ? std::max(32, r->n_cu * r->tune.raster_wg_per_cu / 16)
                                 : r->n_cu * r->tune.raster_wg_per_cu;
-    const int ip = r->tune.item_prims;
     if (timed) (void)hipEventRecord(r->ev[0], st);
     const size_t P = (size_t)r->W * r->H;
     // counters zeroed, visibility emptied (before the setup, which draws
     // small triangles into it, outside the exact-order pass, whose NaN rule
     // needs every fragment through the ordered raster): by the vertex passes
     const bool shadows = r->n_slots > 0 && !nan_mode;
-    constexpr int32_t CNT_WORDS = (int32_t)(sizeof(Counters) / 4);
+    constexpr int32_t CNT_WORDS = (int32_t)(sizeof(PassCounters) / 4);
     // a plain frame runs its shadow passes on the context's second stream,
     // beside the main view's passes (they meet at the shading); a batch
     // keeps them on its own stream
@@ -1217,7 +1169,6 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     // on this one
     const bool split_shade = split && r->sc->any_ao && r->col_pre && r->post_flag;
     if (shadows) {
-        const int nt = r->n_slots * r->stiles_per_map;
         if (split) {
             (void)hipEventRecord(r->ev_fork, st);
             (void)hipStreamWaitEvent(ss, r->ev_fork, 0);
@@ -1226,18 +1177,10 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
         wide_stage(2);
         launch_vertex_shadow(ss, d, r->d_strans, r->shc, r->ts, FrameClear{(uint32_t*)cs, CNT_WORDS, nullptr, 0});
         wide_stage(3);
-        launch_setup_shadow(ss, d, r->shc, r->tri_rec, r->ts, r->s_prims, r->s_pbox, r->s_tile_count, cs, r->cap_shadow,
-                            r->smaps);
-        wide_stage(4);
-        launch_scan(ss, r->s_tile_count, nt, r->s_tile_off, r->s_chunk_off, r->s_tile_cursor, r->s_scan_sums,
-                    r->s_item_tile, r->s_cap_items, nullptr, 0, cs, ip);
-        wide_stage(5);
-        launch_bin(ss, r->s_pbox, cs, r->stiles_x, r->shc.rt_shift, r->stiles_per_map, 1, r->s_tile_cursor, r->s_tile_list,
-                   r->cap_shadow, r->n_slots * d.n_tris, d.n_tris);
-        RasterTarget rt{r->SW, r->SH, r->stiles_x, r->stiles_per_map, nt, nullptr, nullptr, nullptr, r->smaps};
+        launch_setup_shadow(ss, d, r->shc, r->tri_rec, r->ts, r->s_jobs, cs, r->smaps);
+        RasterTarget rt{r->SW, r->SH, nullptr, nullptr, nullptr, r->smaps};
         wide_stage(6);
-        launch_raster(ss, 2, persistent, r->s_prims, r->s_tile_off, r->s_chunk_off, r->s_item_tile, r->s_cap_items,
-                      r->s_tile_list, cs, rt, ip, r->rtile);
+        launch_raster(ss, 2, persistent, r->s_jobs, cs, rt);
         if (timed) (void)hipEventRecord(r->ev_s[1], ss);
         if (split && !split_shade) (void)hipEventRecord(r->ev_join, ss);
     }
@@ -1248,25 +1191,19 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
                        FrameClear{(uint32_t*)cm, (shadows ? 1 : 2) * CNT_WORDS, (uint64_t*)r->vis, P});
     if (timed) (void)hipEventRecord(r->ev[2], st);
     wide_stage(8);
-    launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->prims, r->pbox, r->clips, r->tri_clip_slot, r->clip_list,
-                      r->tile_count, r->blk_prims, cm, r->cap_main, (unsigned long long*)r->vis,
+    // (the exact-order pass keeps the frame's statistics: it draws nothing in
+    // the setup, so its raster takes other primitives)
+    launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->jobs, r->clips, r->tri_clip_slot, r->clip_list,
+                      r->blk_prims, nan_mode ? nullptr : r->blk_pairs, cm, r->cap_main, (unsigned long long*)r->vis,
                       nan_mode ? 0 : r->tune.main_direct_max, r->tri_rec);
-    wide_stage(9);
-    launch_scan(st, r->tile_count, r->n_rtiles, r->tile_off, r->chunk_off, r->tile_cursor, r->scan_sums, r->item_tile,
-                r->cap_items, r->blk_prims, d.n_tris ? setup_blocks(d.n_tris) + clip_grid(r->cap_main) : 0, cm, ip);
-    wide_stage(10);
-    launch_bin(st, r->pbox, cm, r->rtiles_x, r->vc.rt_shift, r->n_rtiles, 0, r->tile_cursor, r->tile_list, r->cap_main, d.n_tris,
-               d.n_tris);
     if (timed) (void)hipEventRecord(r->ev[3], st);
     if (nan_mode) {
         launch_fill_u32(st, r->first_all, P, 0xffffffffu);
         launch_fill_u32(st, r->first_nan, P, 0xffffffffu);
     }
-    RasterTarget rt{r->W, r->H, r->rtiles_x, r->n_rtiles, r->n_rtiles, (unsigned long long*)r->vis, r->first_all,
-                    r->first_nan, nullptr};
+    RasterTarget rt{r->W, r->H, (unsigned long long*)r->vis, r->first_all, r->first_nan, nullptr};
     wide_stage(11);
-    launch_raster(st, nan_mode ? 1 : 0, persistent, r->prims, r->tile_off, r->chunk_off, r->item_tile, r->cap_items,
-                  r->tile_list, cm, rt, ip, r->rtile);
+    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt);
     wide_stage(12);
     launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec);
     if (timed) (void)hipEventRecord(r->ev[4], st);
@@ -1313,6 +1250,24 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     return PRH_OK;
 }
 
+// The work capacities a frame's counters ask for; false if it had enough.
+bool grow_work(prh_renderer* r, const Counters& cm, const Counters& cs) {
+    if (!cm.overflow && !cs.overflow) return false;
+    auto up = [](int32_t& cap, int32_t need) {
+        if (need > cap) cap = need + need / 4 + 16;
+    };
+    up(r->cap_shadow.jobs, cs.need_jobs);
+    up(r->cap_main.jobs, cm.need_jobs);
+    up(r->cap_main.clip_tris, cm.n_clipped);
+    r->cap_main.clip_subs = CLIP_PIECES * r->cap_main.clip_tris;
+    return true;
+}
+int regrow(prh_renderer* r) {
+    free_work(r);
+    r->work_gen++;
+    return alloc_work(r);
+}
+
 // After a frame's work has completed: after an overflow, grows the work
 // buffers and asks for another attempt (again = true); after a NaN depth,
 // re-runs the visibility in exact order; then fills the statistics (per-pass
@@ -1321,24 +1276,10 @@ int finish_frame(prh_renderer* r, int attempt, bool& again, bool timed = true) {
     again = false;
     hipStream_t st = r->ctx->stream;
     const Counters cm = r->h_cnt[0], cs = r->h_cnt[1];
-    bool grow = false;
-    if (cs.overflow || cs.n_pairs > r->cap_shadow.pairs) {
-        r->cap_shadow.pairs = std::max(r->cap_shadow.pairs, cs.n_pairs + cs.n_pairs / 4 + 16);
-        grow = true;
-    }
-    if (cm.overflow || cm.n_pairs > r->cap_main.pairs || cm.n_clipped > r->cap_main.clip_tris) {
-        r->cap_main.pairs = std::max(r->cap_main.pairs, cm.n_pairs + cm.n_pairs / 4 + 16);
-        r->cap_main.clip_tris = std::max(r->cap_main.clip_tris, cm.n_clipped + cm.n_clipped / 4 + 16);
-        r->cap_main.clip_subs = std::max(r->cap_main.clip_subs, CLIP_PIECES * r->cap_main.clip_tris);
-        r->cap_main.prims = d_n_tris(r) + r->cap_main.clip_subs;
-        grow = true;
-    }
-    if (grow) {
+    if (grow_work(r, cm, cs)) {
         if (attempt >= 3) return fail(PRH_E_NOMEM, "work buffers keep overflowing");
-        free_work(r);
-        int rc = alloc_work(r);
+        int rc = regrow(r);
         if (rc) return rc;
-        r->work_gen++;
         again = true;
         return PRH_OK;
     }
@@ -1346,15 +1287,22 @@ int finish_frame(prh_renderer* r, int attempt, bool& again, bool timed = true) {
         return fail(PRH_E_UNSUPPORTED, "NaN depth in a shadow pass: its result depends on sequential order");
     bool nan_rerun = false;
     if (cm.nan_flag) {
-        const int rc = enqueue_frame(r, true, st, timed);
-        HIP_TRY(hipStreamSynchronize(st));
-        if (rc) return rc;
+        // (it draws nothing in the setup, so it may need longer queues)
+        for (int k = 0;; k++) {
+            int rc = enqueue_frame(r, true, st, timed);
+            HIP_TRY(hipStreamSynchronize(st));
+            if (rc) return rc;
+            if (!grow_work(r, r->h_cnt[0], Counters{})) break;
+            if (k >= 3) return fail(PRH_E_NOMEM, "work buffers keep overflowing");
+            if ((rc = regrow(r))) return rc;
+        }
         nan_rerun = true;
     }
     prh_frame_stats& S = r->stats;
     S.ms_total = S.ms_shadow = S.ms_vertex = S.ms_setup = S.ms_raster = S.ms_ao = S.ms_shade = 0.0f;
     r->times_pending = timed, r->times_nan_rerun = nan_rerun;
-    S.n_prims = cm.n_prims, S.n_clipped = cm.n_clipped, S.n_bin_pairs = cm.n_pairs;
+    S.n_clipped = cm.n_clipped;
+    r->counts_pending = true;
     S.nan_rerun = nan_rerun ? 1 : 0;
     r->has_frame = true;
     r->frame_serial++;
@@ -1941,10 +1889,28 @@ void fill_times(prh_renderer* r) {
     }
 }
 
+// And its primitive and tile counts, from its workgroups' sums.
+int fill_counts(prh_renderer* r) {
+    if (!r->counts_pending) return PRH_OK;
+    r->counts_pending = false;
+    prh_frame_stats& S = r->stats;
+    S.n_prims = S.n_bin_pairs = 0;
+    const int32_t n_tris = r->sc->d.n_tris;
+    if (!n_tris) return PRH_OK;
+    const size_t n = (size_t)setup_blocks(n_tris) + clip_grid(r->cap_main);
+    std::vector<int32_t> v(2 * n);
+    HIP_TRY(hipMemcpy(v.data(), r->blk_prims, 4 * n, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(v.data() + n, r->blk_pairs, 4 * n, hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < n; i++) S.n_prims += v[i], S.n_bin_pairs += v[n + i];
+    return PRH_OK;
+}
+
 int prh_last_stats(prh_renderer* r, prh_frame_stats* out) {
     if (!r || !out) return fail(PRH_E_INVALID, "prh_last_stats: null argument");
     HIP_TRY(hipSetDevice(r->ctx->device));
     fill_times(r);
+    int rc = fill_counts(r);
+    if (rc) return rc;
     *out = r->stats;
     return PRH_OK;
 }
@@ -2365,18 +2331,12 @@ int prh_set_tuning(prh_renderer* r, const prh_tuning* t) {
         return fail(PRH_E_INVALID, "prh_set_tuning: a knob out of range");
     HIP_TRY(hipSetDevice(r->ctx->device));
     HIP_TRY(hipStreamSynchronize(r->ctx->stream));
-    const bool realloc = t->item_prims != r->tune.item_prims;
     r->tune.raster_wg_per_cu = t->raster_wg_per_cu, r->tune.item_prims = t->item_prims;
     r->tune.shadow_direct_max = t->shadow_direct_max, r->tune.main_direct_max = t->main_direct_max;
     r->tune.overlap_shadows = t->overlap_shadows;
     r->tune.raster_tile = t->raster_tile;
     r->shc.direct_max = t->shadow_direct_max;
-    raster_grid(r);
-    if (realloc) {  // the work-item table is sized by item_prims
-        free_work(r);
-        int rc = alloc_work(r);
-        if (rc) return rc;
-    }
+    raster_tile(r);
     r->work_gen++;  // a cached batch recorded the old values
     return PRH_OK;
 }
@@ -2398,7 +2358,6 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
         *ms = v[v.size() / 2];
         return PRH_OK;
     };
-    static const int32_t c_ip[] = {256, 512, 1024, 2048, 4096};
     static const int32_t c_wg[] = {1, 2, 4, 8};
     static const int32_t c_sd[] = {0, 16, 32, 64, 128, 256};
     static const int32_t c_md[] = {0, 24, 48, 96, 192};
@@ -2410,13 +2369,12 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
     int rc = time(best, &best_ms);
     if (rc) return rc;
     // coordinate descent: each knob over its candidates, the others at their best
-    for (int knob = 0; knob < 6; knob++) {
-        const int32_t* c = knob == 0 ? c_ip : knob == 1 ? c_wg : knob == 2 ? c_sd : knob == 3 ? c_md : knob == 4 ? c_ov : c_rt;
-        const int n = knob == 0 ? 5 : knob == 1 ? 4 : knob == 2 ? 6 : knob == 3 ? 5 : knob == 4 ? 2 : 3;
+    for (int knob = 1; knob < 6; knob++) {
+        const int32_t* c = knob == 1 ? c_wg : knob == 2 ? c_sd : knob == 3 ? c_md : knob == 4 ? c_ov : c_rt;
+        const int n = knob == 1 ? 4 : knob == 2 ? 6 : knob == 3 ? 5 : knob == 4 ? 2 : 3;
         for (int k = 0; k < n; k++) {
             prh_tuning t = best;
-            int32_t* f = knob == 0 ? &t.item_prims
-                       : knob == 1 ? &t.raster_wg_per_cu
+            int32_t* f = knob == 1 ? &t.raster_wg_per_cu
                        : knob == 2 ? &t.shadow_direct_max
                        : knob == 3 ? &t.main_direct_max
                        : knob == 4 ? &t.overlap_shadows : &t.raster_tile;
@@ -2486,7 +2444,6 @@ int prh_autotune_batch(prh_renderer* const* rs, int32_t n, int32_t frames, prh_t
         *ms = v[v.size() / 2];
         return PRH_OK;
     };
-    static const int32_t c_ip[] = {256, 512, 1024, 2048, 4096};
     static const int32_t c_wg[] = {2, 4, 8, 16};
     static const int32_t c_sd[] = {0, 16, 32, 64, 128, 256};
     static const int32_t c_md[] = {0, 24, 48, 96, 192};
@@ -2496,15 +2453,14 @@ int prh_autotune_batch(prh_renderer* const* rs, int32_t n, int32_t frames, prh_t
     float best_ms = 0.0f;
     int rc = time(cur, frames, &best_ms);
     if (rc) return rc;
-    for (int knob = 0; knob < 5; knob++)
+    for (int knob = 1; knob < 5; knob++)
         for (int c = 0; c < 2; c++) {
             if (!has[c]) continue;
-            const int32_t* cand = knob == 0 ? c_ip : knob == 1 ? c_wg : knob == 2 ? c_sd : knob == 3 ? c_md : c_rt;
-            const int nc = knob == 0 ? 5 : knob == 1 ? 4 : knob == 2 ? 6 : knob == 3 ? 5 : 3;
+            const int32_t* cand = knob == 1 ? c_wg : knob == 2 ? c_sd : knob == 3 ? c_md : c_rt;
+            const int nc = knob == 1 ? 4 : knob == 2 ? 6 : knob == 3 ? 5 : 3;
             for (int k = 0; k < nc; k++) {
                 prh_tuning t[2] = {cur[0], cur[1]};
-                int32_t* f = knob == 0 ? &t[c].item_prims
-                           : knob == 1 ? &t[c].raster_wg_per_cu
+                int32_t* f = knob == 1 ? &t[c].raster_wg_per_cu
                            : knob == 2 ? &t[c].shadow_direct_max
                            : knob == 3 ? &t[c].main_direct_max : &t[c].raster_tile;
                 if (*f == cand[k]) continue;
