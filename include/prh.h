@@ -217,8 +217,8 @@ int prh_read_image(prh_renderer* r, uint8_t* rgba, size_t bytes);
 /* Copy one internal buffer to host memory (parity tests, debugging). */
 int prh_read_buffer(prh_renderer* r, int32_t which, void* dst, size_t bytes);
 
-/* Per-kernel device time of the last frame, from HIP events on the
- * renderer's stream. */
+/* Per-pass device time of the last frame, from stamps of the device's clock
+ * its kernels write. */
 typedef struct prh_frame_stats {
     float ms_total;
     float ms_shadow;     /* all shadow passes                               */

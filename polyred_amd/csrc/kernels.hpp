@@ -159,9 +159,16 @@ constexpr int AO_WIN = 448;
 // Third descriptor word of a raw (unstrided, untyped) buffer on gfx9 parts.
 constexpr uint32_t BUF_DWORD3 = 0x00020000u;
 
+// Where a kernel writes the device's clock as it starts or ends (null: not at
+// all), for the passes' times.
+struct Stamp {
+    unsigned long long* start = nullptr;
+    unsigned long long* end = nullptr;
+};
+
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_fill_u64(hipStream_t st, uint64_t* p, size_t n, uint64_t v);
-void launch_frame_clear(hipStream_t st, uint32_t* cnt, int32_t n_cnt, uint64_t* vis, size_t n_vis);
+void launch_frame_clear(hipStream_t st, uint32_t* cnt, int32_t n_cnt, uint64_t* vis, size_t n_vis, Stamp stamp);
 // A frame's start: counters to zero, the visibility buffer emptied.  Each
 // stream's first pass (the vertex passes) does its part before its own
 // work, with k_frame_clear only where that pass has nothing to launch.
@@ -173,9 +180,9 @@ struct FrameClear {
 };
 void launch_vertex_main(hipStream_t st, const DevScene& s, const gm::M4* trans, const gm::M4* normal,
                         const ViewConsts& vc, float4* tv_scr, float4* tv_nor, float4* tv_wp, uint32_t* tv_col,
-                        float2* tv_uv, const FrameClear& clr);
+                        float2* tv_uv, const FrameClear& clr, Stamp stamp);
 void launch_vertex_shadow(hipStream_t st, const DevScene& s, const gm::M4* strans, const ShadowConsts& sc,
-                          float3* ts, const FrameClear& clr);
+                          float3* ts, const FrameClear& clr, Stamp stamp);
 // The setup's workgroups (each writes its unclipped primitives to
 // blk_prims[its index]) and then the clipper's (blk_prims[setup_blocks +
 // its index]: its pieces); blk_prims holds setup_blocks(n_tris) + CLIP_GRID.
@@ -187,7 +194,7 @@ int clip_grid(const Capacities& cap);
 void launch_setup_main(hipStream_t st, const DevScene& s, const ViewConsts& vc, const float4* tv_scr,
                        const float4* tv_nor, const JobQueues& jobs, ClipRec* clips, int32_t* tri_clip_slot,
                        ClipJob* clip_list, int32_t* blk_prims, int32_t* blk_pairs, Counters* cnt, Capacities cap,
-                       unsigned long long* vis, int32_t draw_small, const int4* tri_rec);
+                       unsigned long long* vis, int32_t draw_small, const int4* tri_rec, Stamp stamp);
 void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& sc, const int4* tri_rec,
                          const float3* ts, const JobQueues& jobs, Counters* cnt, uint32_t* smaps);
 // Each global triangle's record, fixed by the scene: its transformed
@@ -196,14 +203,14 @@ void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& 
 void launch_tri_rec(hipStream_t st, const DevScene& s, int4* tri_rec);
 // mode: 0 visibility, 1 visibility in exact order (NaN rule), 2 shadow maps
 void launch_raster(hipStream_t st, int mode, int n_workgroups, const JobQueues& jobs, Counters* cnt,
-                   const RasterTarget& rt);
+                   const RasterTarget& rt, Stamp stamp);
 void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters* cnt, float* depth, const DevScene& s,
-                    int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec);
+                    int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec, Stamp stamp);
 void launch_ao(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b);
-void launch_shade_bg(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b);
-void launch_shade(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b);
+void launch_shade_bg(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b, Stamp stamp);
+void launch_shade(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b, Stamp stamp);
 // false (and nothing launched) without the colour before AO, the AO factors or the triangle records
-bool launch_shade_post(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b);
+bool launch_shade_post(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b, Stamp stamp);
 void launch_shadow_count(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b,
                          uint8_t* out);
 
@@ -218,6 +225,6 @@ int wide_upload(const WideBatch* w, uint8_t* dev);
 void wide_launch(const WideBatch* w, hipStream_t st, const uint8_t* dev);
 // out[y][x] (out_rows x out_w) = 8-bit bilinear filter of row x of `in` at y
 void launch_resize(hipStream_t st, const uint32_t* in, int32_t in_w, uint32_t* out, int32_t out_w, int32_t out_rows,
-                   const int16_t* coeffs, const int32_t* start, int32_t fl);
+                   const int16_t* coeffs, const int32_t* start, int32_t fl, Stamp stamp = {});
 
 }  // namespace prh

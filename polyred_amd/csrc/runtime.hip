@@ -349,6 +349,13 @@ int upload(T** p, const T* src, size_t n) {
 
 }  // namespace
 
+// A frame's stamps (prh_renderer.stamps): where its streams and the uncovered
+// colour's kernel start, and the ends of its passes.
+enum {
+    ST_SHADOW, ST_SHADOW_END, ST_VERTEX, ST_VERTEX_END, ST_SETUP_END, ST_RESOLVED, ST_BG, ST_BG_END, ST_SHADE_END,
+    ST_END, N_STAMPS
+};
+
 struct prh_renderer;
 // prh_render_batch spreads a batch over one stream per hardware queue the
 // process has (GPU_MAX_HW_QUEUES, 4 unless set), at most PRH_BATCH_MAX.
@@ -421,9 +428,9 @@ struct prh_renderer {
     int32_t *blk_prims, *blk_pairs;
     ClipJob* clip_list;
     JobQueues s_jobs;  // the shadow passes' own queues (they run beside the main view's)
-    hipEvent_t ev_fork, ev_join, ev_s[2];
-    // split shading: resolve done, the shadow passes done, the AO's span
-    hipEvent_t ev_res, ev_sdone, ev_sh[2];
+    hipEvent_t ev_fork, ev_join;
+    // split shading: resolve done, the shadow passes done
+    hipEvent_t ev_res, ev_sdone;
     uint32_t* col_pre;            // split shading: the colour before AO
     uint8_t* post_flag;           // and what its second half does per pixel
     int32_t n_cu;
@@ -444,7 +451,8 @@ struct prh_renderer {
     Counters* h_cnt;    // pinned
     Counters* d_h_cnt;  // its device address
     Capacities cap_main, cap_shadow;
-    hipEvent_t ev[8];
+    // the passes' stamps of the device's clock, N_STAMPS of them
+    unsigned long long* stamps;
     prh_frame_stats stats;
     bool has_frame;  // the visibility of a frame is in vis
     int work_gen;    // bumped when the work buffers are reallocated
@@ -461,7 +469,7 @@ struct prh_renderer {
     uint32_t* present_to;  // during prh_surface_render: the acquired surface texture
     prh_tuning tune;       // speed knobs (results do not depend on them)
     bool split_shade_last;  // the last frame split its shading
-    // the last frame's per-pass times wait in its events until the stats are
+    // the last frame's per-pass times wait in its stamps until the stats are
     // read (prh_last_stats): a frame's own host work stays short
     bool times_pending, times_nan_rerun;
     bool counts_pending;  // likewise the primitive and tile counts, in blk_prims and blk_pairs
@@ -1047,6 +1055,7 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     if (!rc) chk(ralloc(r, &r->bg_lin, 4));
     if (!rc) chk(ralloc(r, &r->smaps, (size_t)std::max(1, r->n_slots) * r->SW * r->SH));
     if (!rc) chk(ralloc(r, &r->cnt, 2));
+    if (!rc) chk(ralloc(r, &r->stamps, N_STAMPS));
     if (!rc) chk(alloc_work(r));
     if (!rc) {
         hipError_t e = hipHostMalloc((void**)&r->h_cnt, 2 * sizeof(Counters), hipHostMallocDefault);
@@ -1054,15 +1063,10 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
         else if (hipHostGetDevicePointer((void**)&r->d_h_cnt, r->h_cnt, 0) != hipSuccess)
             rc = fail(PRH_E_HIP, "hipHostGetDevicePointer failed");
     }
-    for (int i = 0; i < 8 && !rc; i++)
-        if (hipEventCreate(&r->ev[i]) != hipSuccess) rc = fail(PRH_E_HIP, "hipEventCreate failed");
-    for (int i = 0; i < 2 && !rc; i++)
-        if (hipEventCreate(&r->ev_s[i]) != hipSuccess) rc = fail(PRH_E_HIP, "hipEventCreate failed");
     if (!rc && (hipEventCreateWithFlags(&r->ev_fork, hipEventDisableTiming) != hipSuccess ||
                 hipEventCreateWithFlags(&r->ev_join, hipEventDisableTiming) != hipSuccess ||
                 hipEventCreateWithFlags(&r->ev_res, hipEventDisableTiming) != hipSuccess ||
-                hipEventCreateWithFlags(&r->ev_sdone, hipEventDisableTiming) != hipSuccess ||
-                hipEventCreate(&r->ev_sh[0]) != hipSuccess || hipEventCreate(&r->ev_sh[1]) != hipSuccess))
+                hipEventCreateWithFlags(&r->ev_sdone, hipEventDisableTiming) != hipSuccess))
         rc = fail(PRH_E_HIP, "hipEventCreate failed");
     if (rc) {
         free_list(r->allocs);
@@ -1072,6 +1076,7 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     // Shadow maps start at zero once, here, as make([]float32) in initShadowMaps
     // (stored as ordered depth bits).
     launch_fill_u32(ctx->stream, r->smaps, (size_t)std::max(1, r->n_slots) * r->SW * r->SH, depth_ord(0.0f));
+    launch_fill_u64(ctx->stream, reinterpret_cast<uint64_t*>(r->stamps), N_STAMPS, 0ull);
     launch_tri_rec(ctx->stream, s->d, r->tri_rec);
     {
         int n_cu = 0;
@@ -1098,18 +1103,12 @@ int prh_renderer_free(prh_renderer* r) {
     if (held) drop_graph(r->ctx);
     free_list(r->allocs);
     if (r->h_cnt) (void)hipHostFree(r->h_cnt);
-    for (int i = 0; i < 8; i++)
-        if (r->ev[i]) (void)hipEventDestroy(r->ev[i]);
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < 2; i++)
         if (r->dev[i]) (void)hipEventDestroy(r->dev[i]);
-        if (r->ev_s[i]) (void)hipEventDestroy(r->ev_s[i]);
-    }
     if (r->ev_fork) (void)hipEventDestroy(r->ev_fork);
     if (r->ev_join) (void)hipEventDestroy(r->ev_join);
     if (r->ev_res) (void)hipEventDestroy(r->ev_res);
     if (r->ev_sdone) (void)hipEventDestroy(r->ev_sdone);
-    for (int i = 0; i < 2; i++)
-        if (r->ev_sh[i]) (void)hipEventDestroy(r->ev_sh[i]);
     r->sc->live_renderers--;
     delete r;
     return PRH_OK;
@@ -1141,8 +1140,8 @@ ShadeBuffers shade_buffers(const prh_renderer* r) {
 }
 
 // Enqueues one frame; nan_mode re-runs the visibility raster in exact order.
-// `timed` records the per-pass events (not while a batch is captured into a
-// graph).  `wide`: the launches are being recorded into a wide batch (the
+// `timed`: the passes stamp the device's clock (not in a recorded or captured
+// batch).  `wide`: the launches are being recorded into a wide batch (the
 // stage numbers order its launches; the persistent rasters take fewer
 // workgroups per view, since every view's run together).  A non-zero
 // status means part of the frame may be enqueued and none of it is valid.
@@ -1152,7 +1151,13 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     Counters* cs = &r->cnt[1].c;
     const int persistent = wide ? std::max(32, r->n_cu * r->tune.raster_wg_per_cu / 16)
                                 : r->n_cu * r->tune.raster_wg_per_cu;
-    if (timed) (void)hipEventRecord(r->ev[0], st);
+    // a stream's first kernel stamps its start `a`, a pass's last its end `b`
+    auto at = [&](int a, int b = -1) {
+        Stamp t;
+        if (timed && a >= 0) t.start = r->stamps + a;
+        if (timed && b >= 0) t.end = r->stamps + b;
+        return t;
+    };
     const size_t P = (size_t)r->W * r->H;
     // counters zeroed, visibility emptied (before the setup, which draws
     // small triangles into it, outside the exact-order pass, whose NaN rule
@@ -1173,40 +1178,37 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
             (void)hipEventRecord(r->ev_fork, st);
             (void)hipStreamWaitEvent(ss, r->ev_fork, 0);
         }
-        if (timed) (void)hipEventRecord(r->ev_s[0], ss);
         wide_stage(2);
-        launch_vertex_shadow(ss, d, r->d_strans, r->shc, r->ts, FrameClear{(uint32_t*)cs, CNT_WORDS, nullptr, 0});
+        launch_vertex_shadow(ss, d, r->d_strans, r->shc, r->ts, FrameClear{(uint32_t*)cs, CNT_WORDS, nullptr, 0},
+                             at(ST_SHADOW));
         wide_stage(3);
         launch_setup_shadow(ss, d, r->shc, r->tri_rec, r->ts, r->s_jobs, cs, r->smaps);
         RasterTarget rt{r->SW, r->SH, nullptr, nullptr, nullptr, r->smaps};
         wide_stage(6);
-        launch_raster(ss, 2, persistent, r->s_jobs, cs, rt);
-        if (timed) (void)hipEventRecord(r->ev_s[1], ss);
+        launch_raster(ss, 2, persistent, r->s_jobs, cs, rt, at(-1, ST_SHADOW_END));
         if (split && !split_shade) (void)hipEventRecord(r->ev_join, ss);
     }
-    if (timed) (void)hipEventRecord(r->ev[1], st);
     wide_stage(7);
     // (both counter blocks where no shadow pass runs)
     launch_vertex_main(st, d, r->d_trans, r->d_normal, r->vc, r->tv_scr, r->tv_nor, r->tv_wp, r->tv_col, r->tv_uv,
-                       FrameClear{(uint32_t*)cm, (shadows ? 1 : 2) * CNT_WORDS, (uint64_t*)r->vis, P});
-    if (timed) (void)hipEventRecord(r->ev[2], st);
+                       FrameClear{(uint32_t*)cm, (shadows ? 1 : 2) * CNT_WORDS, (uint64_t*)r->vis, P},
+                       at(ST_VERTEX, ST_VERTEX_END));
     wide_stage(8);
     // (the exact-order pass keeps the frame's statistics: it draws nothing in
     // the setup, so its raster takes other primitives)
     launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->jobs, r->clips, r->tri_clip_slot, r->clip_list,
                       r->blk_prims, nan_mode ? nullptr : r->blk_pairs, cm, r->cap_main, (unsigned long long*)r->vis,
-                      nan_mode ? 0 : r->tune.main_direct_max, r->tri_rec);
-    if (timed) (void)hipEventRecord(r->ev[3], st);
+                      nan_mode ? 0 : r->tune.main_direct_max, r->tri_rec, at(-1, ST_SETUP_END));
     if (nan_mode) {
         launch_fill_u32(st, r->first_all, P, 0xffffffffu);
         launch_fill_u32(st, r->first_nan, P, 0xffffffffu);
     }
     RasterTarget rt{r->W, r->H, (unsigned long long*)r->vis, r->first_all, r->first_nan, nullptr};
     wide_stage(11);
-    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt);
+    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt, Stamp{});
     wide_stage(12);
-    launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec);
-    if (timed) (void)hipEventRecord(r->ev[4], st);
+    launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec,
+                   at(-1, ST_RESOLVED));
     const ShadeBuffers b = shade_buffers(r);
     // the split shading's buffers: both halves read and write col_pre
     ShadeBuffers bp = b;
@@ -1217,35 +1219,32 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
         (void)hipEventRecord(r->ev_sdone, ss);
         (void)hipEventRecord(r->ev_res, st);
         (void)hipStreamWaitEvent(ss, r->ev_res, 0);
-        if (timed) (void)hipEventRecord(r->ev_sh[0], ss);
         launch_ao(ss, d, r->sh, b);
-        if (timed) (void)hipEventRecord(r->ev_sh[1], ss);
         // the uncovered colour (pixel (0,0)'s shading, its AO factor
         // included) there too, beside the end of the shading's first half
-        launch_shade_bg(ss, d, r->sh, b);
+        launch_shade_bg(ss, d, r->sh, b, at(ST_BG, ST_BG_END));
         (void)hipEventRecord(r->ev_join, ss);
         (void)hipStreamWaitEvent(st, r->ev_sdone, 0);  // the shading reads the shadow maps
-        launch_shade(st, d, r->sh, bp);
+        launch_shade(st, d, r->sh, bp, at(-1, ST_SHADE_END));
     }
     wide_stage(13);
     if (r->sc->any_ao && !split_shade) launch_ao(st, d, r->sh, b);  // else no pixel reads an AO factor
-    if (timed) (void)hipEventRecord(r->ev[5], st);
     if (split) (void)hipStreamWaitEvent(st, r->ev_join, 0);  // the shadow maps (and the AO factors)
     wide_stage(14);
-    if (!split_shade) launch_shade_bg(st, d, r->sh, b);
-    if (timed) (void)hipEventRecord(r->ev[7], st);
+    if (!split_shade) launch_shade_bg(st, d, r->sh, b, at(ST_BG, ST_BG_END));
     wide_stage(15);
-    if (!split_shade) launch_shade(st, d, r->sh, b);
-    else if (!launch_shade_post(st, d, r->sh, bp))
+    const int last = r->msaa > 1 ? -1 : ST_END;
+    if (!split_shade) launch_shade(st, d, r->sh, b, at(-1, last));
+    else if (!launch_shade_post(st, d, r->sh, bp, at(-1, last)))
         return fail(PRH_E_INVALID, "split shading without the AO factors or triangle records");
     if (r->msaa > 1) {
         // passAntialiasing (render/raster.go:361-378): Resize after gamma
         wide_stage(16);
         launch_resize(st, r->image_big, r->W, r->resize_tmp, r->H, r->OW, r->rz_cx, r->rz_ox, r->rz_flx);
         wide_stage(17);
-        launch_resize(st, r->resize_tmp, r->H, final_image(r), r->OW, r->OH, r->rz_cy, r->rz_oy, r->rz_fly);
+        launch_resize(st, r->resize_tmp, r->H, final_image(r), r->OW, r->OH, r->rz_cy, r->rz_oy, r->rz_fly,
+                      at(-1, ST_END));
     }
-    if (timed) (void)hipEventRecord(r->ev[6], st);
     // (k_shade_bg writes the counters into r->h_cnt)
     return PRH_OK;
 }
@@ -1271,7 +1270,7 @@ int regrow(prh_renderer* r) {
 // After a frame's work has completed: after an overflow, grows the work
 // buffers and asks for another attempt (again = true); after a NaN depth,
 // re-runs the visibility in exact order; then fills the statistics (per-pass
-// times only if the frame recorded its events).
+// times only if the frame stamped them).
 int finish_frame(prh_renderer* r, int attempt, bool& again, bool timed = true) {
     again = false;
     hipStream_t st = r->ctx->stream;
@@ -1870,23 +1869,31 @@ int prh_read_buffer(prh_renderer* r, int32_t which, void* dst, size_t bytes) {
     return PRH_OK;
 }
 
-// The last frame's per-pass times from its events (finish_frame left them).
-void fill_times(prh_renderer* r) {
-    if (!r->times_pending) return;
+// The last frame's per-pass times from its stamps (finish_frame left them).
+// A pass starts where the one before it on its stream ended.
+int fill_times(prh_renderer* r) {
+    if (!r->times_pending) return PRH_OK;
     r->times_pending = false;
+    unsigned long long t[N_STAMPS];
+    HIP_TRY(hipMemcpy(t, r->stamps, sizeof t, hipMemcpyDeviceToHost));
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, r->ctx->device) != hipSuccess || khz <= 0) khz = 100000;
+    auto ms = [&](unsigned long long a, unsigned long long b) { return b > a ? (float)(b - a) / (float)khz : 0.0f; };
     prh_frame_stats& S = r->stats;
-    float ms[6] = {0};
-    for (int i = 0; i < 6; i++) (void)hipEventElapsedTime(&ms[i], r->ev[i], r->ev[i + 1]);
-    (void)hipEventElapsedTime(&S.ms_total, r->ev[0], r->ev[6]);
-    // (the shadow passes ran beside the main view's: their own span)
-    S.ms_shadow = 0.0f;
-    if (r->n_slots > 0 && !r->times_nan_rerun) (void)hipEventElapsedTime(&S.ms_shadow, r->ev_s[0], r->ev_s[1]);
-    S.ms_vertex = ms[1], S.ms_setup = ms[2], S.ms_raster = ms[3], S.ms_ao = ms[4];
-    (void)hipEventElapsedTime(&S.ms_shade, r->ev[7], r->ev[6]);  // k_shade alone
-    if (r->split_shade_last) {  // the AO on the second stream; the shading's first half beside it
-        (void)hipEventElapsedTime(&S.ms_ao, r->ev_sh[0], r->ev_sh[1]);
-        S.ms_shade += ms[4];
-    }
+    const bool shadow = r->n_slots > 0 && !r->times_nan_rerun, ao = r->sc->any_ao;
+    const unsigned long long first = shadow ? std::min(t[ST_SHADOW], t[ST_VERTEX]) : t[ST_VERTEX];
+    const unsigned long long setup_end = r->sc->d.n_tris ? t[ST_SETUP_END] : t[ST_VERTEX_END];
+    S.ms_total = ms(first, t[ST_END]);
+    S.ms_shadow = shadow ? ms(t[ST_SHADOW], t[ST_SHADOW_END]) : 0.0f;  // (beside the main view's passes: their own span)
+    S.ms_vertex = ms(t[ST_VERTEX], t[ST_VERTEX_END]);
+    S.ms_setup = ms(t[ST_VERTEX_END], setup_end);
+    S.ms_raster = ms(setup_end, t[ST_RESOLVED]);
+    S.ms_ao = ao ? ms(t[ST_RESOLVED], t[ST_BG]) : 0.0f;
+    // (split shading: the first half beside the AO, and the second)
+    S.ms_shade = r->split_shade_last ? ms(std::max(t[ST_RESOLVED], t[ST_SHADOW_END]), t[ST_SHADE_END]) +
+                                           ms(std::max(t[ST_SHADE_END], t[ST_BG_END]), t[ST_END])
+                                     : ms(t[ST_BG], t[ST_END]);
+    return PRH_OK;
 }
 
 // And its primitive and tile counts, from its workgroups' sums.
@@ -1908,8 +1915,8 @@ int fill_counts(prh_renderer* r) {
 int prh_last_stats(prh_renderer* r, prh_frame_stats* out) {
     if (!r || !out) return fail(PRH_E_INVALID, "prh_last_stats: null argument");
     HIP_TRY(hipSetDevice(r->ctx->device));
-    fill_times(r);
-    int rc = fill_counts(r);
+    int rc = fill_times(r);
+    if (!rc) rc = fill_counts(r);
     if (rc) return rc;
     *out = r->stats;
     return PRH_OK;
@@ -2351,7 +2358,7 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
         std::vector<float> v;
         for (int k = 0; k < frames; k++) {
             if ((rc = prh_render(r))) return rc;
-            fill_times(r);
+            if ((rc = fill_times(r))) return rc;
             v.push_back(r->stats.ms_total);
         }
         std::sort(v.begin(), v.end());
