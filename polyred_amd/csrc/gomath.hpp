@@ -60,12 +60,14 @@ GM_HD double pow64(double x, double y) {
     return std::pow(x, y);
 #endif
 }
-// float32(pow(x, y)) for the shading's x in (0, 1] and y in [2^-8, 2048]
-// (the Blinn-Phong specular term), without the library's double-double pow:
+// float32(pow(x, y)) for the shading's x in (0, 1] and y in [2^-8, 16384]
+// (the Blinn-Phong specular term and the AO's 10000), without the library's
+// double-double pow:
 // t = y log2(x) split as k + f (k an integer, |f| <= 1/2), log2 of the
 // mantissa from the atanh series and 2^f from the exponential series, both
 // in double to a relative error below 2^-40 of the result (the series are
-// truncated below 2^-52; y e is exact; the other roundings are 2^-53 each).
+// truncated below 2^-52; y e is exact; the other roundings are 2^-53 each, of
+// terms of at most 304 where t >= -152, since |y l| <= |y e| / 2 for e < 0).
 // That decides the float32 rounding unless the value lies within 2^-40 of a
 // float32 rounding midpoint; then -- and outside the ranges above -- the
 // library pow decides, so the result is always (float)pow64(x, y).
@@ -76,7 +78,7 @@ GM_HD float pow32_fast(float xf, float yf) {
     uint32_t xb;
     __builtin_memcpy(&xb, &xf, 4);
     if (xb == 0u && yf > 0.0f) return 0.0f;
-    if (!(xf > 0.0f && xf <= 1.0f && yf >= 0.00390625f && yf <= 2048.0f)) return (float)pow64(x, y);
+    if (!(xf > 0.0f && xf <= 1.0f && yf >= 0.00390625f && yf <= 16384.0f)) return (float)pow64(x, y);
     // x = m 2^e, m in [sqrt(1/2), sqrt(2))
     int e;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -157,6 +159,20 @@ GM_HD double atan64(double x) {
 #else
     return std::atan(x);
 #endif
+}
+// float32(atan(r)) for 0 < r <= 2^-5 by the series x - x^3/3 + x^5/5 - ...,
+// in double: truncated below 2^-63 of the result, rounded to within 2^-52 of
+// it, which decides the float32 rounding of every float32 r there (checked for
+// each one from 2^-13 up; below it r^2 / 3 is under 2^-27 and atan(r) rounds
+// to r).
+GM_HD float atan32_small(float r) {
+    const double x = r, x2 = x * x;
+    double p = -1.0 / 11.0;
+    p = __builtin_fma(p, x2, 1.0 / 9.0);
+    p = __builtin_fma(p, x2, -1.0 / 7.0);
+    p = __builtin_fma(p, x2, 1.0 / 5.0);
+    p = __builtin_fma(p, x2, -1.0 / 3.0);
+    return (float)__builtin_fma(x * x2, p, x);
 }
 GM_HD bool isnan32(float x) { return x != x; }
 GM_HD bool isinf64(double x) { return x - x != 0 && x == x; }

@@ -1426,6 +1426,76 @@ __device__ __forceinline__ uint32_t gamma(const ShadeConsts& c, uint32_t col) {
 
 }  // namespace
 
+// The largest depths k_ao's marches compare with: ao_col[q][x] over rows
+// 4q .. 4q+10 of column x, ao_box[q][p] over rows 4q .. 4q+8 of columns
+// 4p .. 4p+8, within the frame.  A thread a column of four rows: each depth is
+// read 2.75 times, all but the first from L2 (6 us at 1920x1080, 10 us at
+// 3840x2160).  Bounds by fours are a sixteenth of the box's exact ones to write
+// and read, and pass over 50 % of the blocks against 57 %.
+struct k_ao_max_args {
+    const float* depth;
+    float *ao_col, *ao_box;
+    int32_t W, H;
+    const Counters* cnt;
+    int32_t gx, gy;  // the grid of this launch
+};
+constexpr int AO_T0 = 4;                       // a march's blocks of eight taps start here
+constexpr int AO_BLOCKS = (100 - AO_T0) / 8;   // and end with tap 99
+static_assert(AO_T0 + 8 * AO_BLOCKS == 100, "the marches' blocks end with tap 99");
+__device__ __forceinline__ float ao_max3(float a, float b, float c) {  // (fmaxf would quiet each operand first)
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// The march tables through the constant address space: uniform loads there are
+// scalar whatever came before (a fence makes the compiler take vector ones for
+// ordinary memory, each a trip to the cache a block has to wait for).
+typedef const __attribute__((address_space(4))) float* ConstF;
+typedef const __attribute__((address_space(4))) double* ConstD;
+template <int N>
+using Int = std::integral_constant<int, N>;
+__device__ __forceinline__ float ao_max8(const float v[8]) {
+    return ao_max3(ao_max3(v[0], v[1], v[2]), ao_max3(v[3], v[4], v[5]), ao_max3(v[6], v[7], v[7]));
+}
+// float32(atan(r)) of a largest quotient, 0 where it is not positive.  The
+// slopes of a rendered depth buffer are small: mostly the whole wave's.
+__device__ __forceinline__ float ao_atan(float r) {
+    if (__ballot(!(r <= 0.03125f)) == 0) return r > 0 ? atan32_small(r) : 0.0f;
+    return r != r ? r : (r > 0 ? (float)atan64((double)r) : 0.0f);
+}
+__device__ __forceinline__ void k_ao_max_body(const k_ao_max_args& a, const VB vb) {
+    __shared__ float s_m[256 + 8];
+    if (a.cnt->overflow) return;
+    const int tid = threadIdx.x, W = a.W, H = a.H, y0 = 4 * vb.by;
+    for (int c = tid; c < 256 + 8; c += 256) {
+        const int x = vb.bx * 256 + c;
+        float v[11];
+#pragma unroll
+        for (int k = 0; k < 11; k++)
+            v[k] = x < W && y0 + k < H ? a.depth[(size_t)(y0 + k) * W + x] : -__builtin_inff();
+        const float m9 = ao_max3(ao_max8(v), v[8], v[8]);
+        s_m[c] = m9;
+        if (c < 256 && x < W) a.ao_col[(size_t)vb.by * W + x] = ao_max3(m9, v[9], v[10]);
+    }
+    __syncthreads();
+    const int bw = (W + 3) / 4, p = vb.bx * 64 + tid;
+    if (tid < 64 && p < bw) {
+        const float* w = s_m + 4 * tid;
+        a.ao_box[(size_t)vb.by * bw + p] = ao_max3(ao_max8(w), w[8], w[8]);
+    }
+}
+__global__ __launch_bounds__(256) void k_ao_max(k_ao_max_args a) {
+    k_ao_max_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
+}
+__global__ __launch_bounds__(256) void k_ao_max_wide(const k_ao_max_args* __restrict__ a,
+        const int32_t* __restrict__ start, int32_t n) {
+    const int v = wide_view(start, n, (int)blockIdx.x);
+    const k_ao_max_args& x = a[v];
+    const int local = (int)blockIdx.x - start[v];
+    if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
+    k_ao_max_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
+}
+
 // Screen-space AO (material/ao.go:20-73) for every pixel whose material has
 // it, plus pixel (0,0) (the uncovered pixels are shaded from it).  One
 // workgroup = 64 consecutive AO pixels of one row (k_resolve's list) x the 8
@@ -1444,12 +1514,19 @@ __device__ __forceinline__ uint32_t gamma(const ShadeConsts& c, uint32_t col) {
 // its rounding to float32 are monotone); a NaN ratio poisons it as math.Max
 // does.  The per-pixel factor pow(total, 10000) (ao.go:31-33) is written for
 // k_shade.
+// What bounds it is vector issue: 83 M instructions at 1920x1080 with every
+// tap taken, 60 M with the blocks of taps that cannot matter passed over, the
+// series for the angles and the power without the library (k_ao and k_ao_max
+// together 193 -> 166 us on one stream; 480x270 51 -> 40, where it waits for
+// loads).  Eight waves a SIMD: 64 registers, without spills.
 struct k_ao_args {
     ShadeConsts c;
     const int32_t* ao_xs;    // k_resolve's lists
     const int32_t* ao_cnt;   // and counts
     const float* depth;
     float* ao;
+    const float* ao_col;  // k_ao_max's
+    const float* ao_box;
     const float* ao_tab;
     int32_t ao_fast;
     const Counters* cnt;
@@ -1473,12 +1550,13 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
     // the row's first pixel (negative outside the buffer) and the distance
     // table's row term
     __shared__ int32_t s_drow[4][100], s_dtab[4][100];
+    __shared__ int32_t s_dbox[4][AO_BLOCKS];  // diagonal marches, block b: byte offset of its row of ao_box
     if (cnt->overflow) return;
     const int W = c.v.W, H = c.v.H;
     const int nbx = (W + 63) / 64, nb = nbx * H;
     const int blk = vb.bx;
     if (blk >= nb) return;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // chunk blk % nbx of row y: the row's AO pixels r0 .. r0+63; past the
     // row's count the workgroup ends here, all its waves alike
     const int y = blk / nbx, r0 = (blk % nbx) * 64;
@@ -1487,191 +1565,259 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
     const int32_t* xs = ao_xs + (size_t)y * W;
     const bool need = r0 + lane < n_row;  // lanes past the row's last AO pixel compute nothing anyone reads
     const int x = xs[min(r0 + lane, n_row - 1)];
-    const int x_first = xs[r0], x_last = xs[min(r0 + 63, n_row - 1)];  // (uniform)
+    const int x_first = __builtin_amdgcn_readfirstlane(x), x_last = __builtin_amdgcn_readlane(x, 63);
     const int li = x - x_first;  // the lane's column counted from the chunk's first pixel
     const int span = x_last - x_first;
     // the x marches read a window of the row staged in LDS when it spans
     // every tap of the chunk (else they take the per-lane path)
     const bool xwin = span + 99 <= AO_WIN;
-    const float dp = need ? depth[(size_t)y * W + x] : -1.0f;
+    // (a lane without a pixel: every elevation -inf)
+    const float dp = need ? depth[(size_t)y * W + x] : __builtin_inff();
     // wave w marches direction 2w (an axis, cheap) then 2w+1 (a diagonal,
-    // costlier): four waves of equal work, none idling at the barrier
-    for (int half = 0; half < 2; half++) {
-    const int wu = __builtin_amdgcn_readfirstlane(2 * wv + half);
-    const int* axis = reinterpret_cast<const int*>(ao_tab + AO_TAB_AXIS) + (wu >> 1) * 4;
-    // Directions 0 and 4 march along x, the major offset exactly +-t.  The
-    // minor one, the float32 cos/sin residue rounded onto the row
-    // coordinate, moves the tap to another row from some t on only near the
-    // frame's bottom rows (it is below half an ulp of Y from Y = 257 up):
-    // tap t is on row y for t < x_t1 and on row x_y2 from there, checked
-    // here for this row (x_rows: every tap on one of the two, both in the
-    // frame).  Where the chunk's taps fit it (xwin), both rows' depths
-    // x_first+1 .. x_last+99 (or x_first-99 .. x_last-1) are staged, 0
-    // outside the row; a wider chunk takes the per-lane path.
-    int x_t1 = 100, x_y2 = y;
-    bool x_rows = false;
-    if (ao_fast && (wu & 3) == 0 && axis[0] && axis[2] != 0x7fffffff) {
-        const float* oy_t = ao_tab + AO_TAB_OFF + wu * 200 + 100;  // fl(dir.y * t)
-        const float Yf = (float)y;
-        const int t_a = lane, t_b = lane + 64;
-        const int iy_a = (int)(Yf + oy_t[t_a]), iy_b = t_b < 100 ? (int)(Yf + oy_t[t_b]) : y;
-        const uint64_t off_a = __ballot(t_a >= 1 && iy_a != y), off_b = __ballot(t_b < 100 && iy_b != y);
-        x_t1 = off_a ? __ffsll((unsigned long long)off_a) - 1 : (off_b ? 64 + __ffsll((unsigned long long)off_b) - 1 : 100);
-        x_y2 = x_t1 < 64 ? __shfl(iy_a, x_t1) : (x_t1 < 100 ? __shfl(iy_b, x_t1 - 64) : y);
-        x_t1 = __builtin_amdgcn_readfirstlane(x_t1), x_y2 = __builtin_amdgcn_readfirstlane(x_y2);
-        const bool bad = (t_a >= x_t1 && iy_a != x_y2) | (t_b >= x_t1 && t_b < 100 && iy_b != x_y2);
-        x_rows = __ballot(bad) == 0 && (unsigned)x_y2 < (unsigned)H;
-        if (x_rows && xwin) {
-            const int ws = axis[1] > 0 ? x_first + 1 : x_first - 99;
-            for (int r = 0; r < (x_t1 < 100 ? 2 : 1); r++) {
-                const size_t row = (size_t)(r ? x_y2 : y) * W;
-                for (int j = lane; j < span + 99; j += 64) {
-                    const int px = ws + j;
-                    s_win[wu >> 2][r][j] = (unsigned)px < (unsigned)W ? depth[row + px] : 0.0f;
+    // costlier): four waves of equal work, none idling at the barrier.  (Each
+    // march is code of its own: as branches of one loop over the two they
+    // shared registers enough to halve the waves in flight.)
+    const int wa = 2 * wv, wd = 2 * wv + 1;
+    const float X = (float)x, Y = (float)y;
+    // the tap with the largest exact elevation/distance quotient; its
+    // rounded quotient is the largest rounded quotient.  The general
+    // path compares exact float64 cross products (e * d_best > e_best * d:
+    // products of two float32 are exact).  The table paths compare
+    // q = e * fl64(1 / d) instead, within 2^-52 of e / d: two distinct
+    // quotients of float32 e and d (d a float32 >= 1) differ relatively by
+    // at least 2^-47, and e / d lies at least 2^-47 (relatively) from any
+    // float32 rounding boundary, so q orders distinct quotients exactly
+    // (equal ones may order either way, and round alike) and float(q)
+    // is the correctly rounded float32 quotient.  (A largest quotient of
+    // at most 0 gives the angle 0: q starts there.)
+    struct Best {
+        double e = -__builtin_inf(), d = 1.0, q = 0.0;
+        bool nan = false;
+    };
+    // depth taps through a buffer descriptor: an out-of-range offset
+    // reads 0 instead of faulting, so a masked lane needs no clamped
+    // address (its value is never used)
+    const __amdgpu_buffer_rsrc_t drs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)depth, (short)0, W * H * 4, BUF_DWORD3);
+    // one tap: the running argmax of elevation / distance, exact
+    // (bitwise & keeps it a select, not a branch that would serialise
+    // the loads of consecutive taps)
+    auto take = [](Best& b, bool v, float e, double d64) {
+        const double e64 = (double)e;
+        const bool better = v & (e64 * b.d > b.e * d64);
+        b.e = better ? e64 : b.e;
+        b.d = better ? d64 : b.d;
+        b.nan |= v & (e != e);
+    };
+    auto take_q = [](Best& b, bool v, float e, double rinv) {
+        const double q = (double)e * rinv;
+        b.q = (v & (q > b.q)) ? q : b.q;
+        b.nan |= v & (e != e);
+    };
+    // every depth finite: no quotient is NaN (an infinite e gives an
+    // infinite q), so the NaN test can go (uniform).  Then a march takes
+    // its taps AO_T0 .. 99 in blocks of eight and passes over a block that
+    // cannot raise any lane's quotient: with M at least every depth of the
+    // block and r at least every 1 / distance, each of its quotients is at
+    // most fl64(fl(M - dp) * r) by the monotony of both roundings (or at
+    // most 0, as is the bound, where M <= dp).  About half of the blocks go
+    // that way on a scene of spheres over a ground plane, and with them their
+    // loads and conversions.
+    const bool finite = cnt->depth_nonfinite == 0;
+    const ConstD rinv_t = (ConstD)(ao_tab + AO_TAB_T64);  // fl64(1 / t) (uniform)
+    auto raises = [&](const Best& b, float e, double r) { return __ballot((double)e * r > b.q) != 0; };
+    auto add = [&](Best& b, float d, double r) { b.q = __builtin_fmax(b.q, (double)(d - dp) * r); };
+    // A march knows its blocks' bounds before it starts (their loads are all
+    // in flight at once) and tests them in the groups {0}, {1}, {2, 3}, {4..7},
+    // {8..11}: each group against the quotients of the groups before it (53 %
+    // of the blocks stay at 1920x1080, against 50 % with a test ahead of each
+    // block, whose loads and scalar work cost more than the blocks it saved).
+    // `test(i)` says if block i can raise a quotient, `eval(i)` takes it.
+    auto blocks = [&](int n, auto test, auto eval) {
+        const uint32_t in = (1u << n) - 1u;
+        uint32_t mask = 0;
+#pragma nounroll
+        for (int g = 0;;) {
+            if (mask == 0) {
+                if (g == 5) break;
+                auto group = [&](auto lo, auto hi) {
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int i = decltype(lo)::value; i < decltype(hi)::value; i++) m |= test(i) ? 1u << i : 0u;
+                    return m & in;
+                };
+                if (g == 0) mask = group(Int<0>(), Int<1>());
+                else if (g == 1) mask = group(Int<1>(), Int<2>());
+                else if (g == 2) mask = group(Int<2>(), Int<4>());
+                else if (g == 3) mask = group(Int<4>(), Int<8>());
+                else mask = group(Int<8>(), Int<AO_BLOCKS>());
+                g++;
+                continue;
+            }
+            const int i = __builtin_ctz(mask);
+            mask &= mask - 1;
+            eval(i);
+        }
+    };
+    // and the march without tables (frames past 4096 pixels a side)
+    auto march_any = [&](Best& b, int wu) {
+        const float dx = c.ao_dir[2 * wu], dy = c.ao_dir[2 * wu + 1];
+        float t = 1.0f;  // t = 0 is the pixel itself: distance 0 < 1, skipped
+#pragma unroll 3
+        for (int ti = 1; ti < 100; ti++, t += 1.0f) {
+            const float cx = X + dx * t, cy = Y + dy * t;
+            const int ix = (int)cx, iy = (int)cy;  // |cx|, |cy| < 2^31: Go's int() truncation
+            const float ex = X - cx, ey = Y - cy;
+            // Len of (ex, ey, 0, 0): FMA(ex,ex, FMA(ey,ey, FMA(0,0,0*0))) where
+            // the inner FMA(ey,ey,+0) is exactly the float32 product ey*ey
+            const float dist = sqrt32_normal(fma64(ex, ex, ey * ey));
+            const bool v = need & ((unsigned)ix < (unsigned)W) & ((unsigned)iy < (unsigned)H) & (dist >= 1.0f);
+            const uint32_t off = (mul_u24((unsigned)iy, (unsigned)W) + (unsigned)ix) * 4u;
+            take(b, v, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp, (double)dist);
+        }
+    };
+    auto ratio = [&](const Best& b) {
+        return b.nan ? __builtin_nanf("") : ao_fast ? (float)b.q : (float)b.e / (float)b.d;
+    };
+    float r_axis, r_diag;
+    {
+        Best b;
+        const int* axis = reinterpret_cast<const int*>(ao_tab + AO_TAB_AXIS) + wv * 4;
+        const ConstF off_x = (ConstF)(ao_tab + AO_TAB_OFF + wa * 200);  // fl(dir.x * t), t = 0..99 (uniform)
+        const ConstF off_y = off_x + 100;                               // fl(dir.y * t)
+        // Directions 0 and 4 march along x, the major offset exactly +-t.  The
+        // minor one, the float32 cos/sin residue rounded onto the row
+        // coordinate, moves the tap to another row from some t on only near the
+        // frame's bottom rows (it is below half an ulp of Y from Y = 257 up):
+        // tap t is on row y for t < x_t1 and on row x_y2 from there, checked
+        // here for this row (x_rows: every tap on one of the two, both in the
+        // frame).  Where the chunk's taps fit it (xwin), both rows' depths
+        // x_first+1 .. x_last+99 (or x_first-99 .. x_last-1) are staged, -inf
+        // outside the row (no elevation, so the march needs no mask there); a
+        // wider chunk takes the per-lane path.
+        int x_t1 = 100, x_y2 = y;
+        bool x_rows = false;
+        if (ao_fast && axis[0] && axis[2] != 0x7fffffff) {
+            const int t_a = lane, t_b = lane + 64;
+            const int iy_a = (int)(Y + off_y[t_a]), iy_b = t_b < 100 ? (int)(Y + off_y[t_b]) : y;
+            const uint64_t off_a = __ballot(t_a >= 1 && iy_a != y), off_b = __ballot(t_b < 100 && iy_b != y);
+            x_t1 = off_a ? __ffsll((unsigned long long)off_a) - 1 : (off_b ? 64 + __ffsll((unsigned long long)off_b) - 1 : 100);
+            x_y2 = x_t1 < 64 ? __shfl(iy_a, x_t1) : (x_t1 < 100 ? __shfl(iy_b, x_t1 - 64) : y);
+            x_t1 = __builtin_amdgcn_readfirstlane(x_t1), x_y2 = __builtin_amdgcn_readfirstlane(x_y2);
+            const bool bad = (t_a >= x_t1 && iy_a != x_y2) | (t_b >= x_t1 && t_b < 100 && iy_b != x_y2);
+            x_rows = __ballot(bad) == 0 && (unsigned)x_y2 < (unsigned)H;
+            if (x_rows && xwin) {
+                const int ws = axis[1] > 0 ? x_first + 1 : x_first - 99;
+                for (int r = 0; r < (x_t1 < 100 ? 2 : 1); r++) {
+                    const int row = (r ? x_y2 : y) * W;
+                    for (int j0 = 0; j0 < span + 99; j0 += 256) {  // (all loads first)
+                        float v[4];
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            v[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                drs, (row + min(max(ws + j0 + 64 * k + lane, 0), W - 1)) * 4, 0, 0));
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const int j = j0 + 64 * k + lane;
+                            if (j < span + 99)
+                                s_win[wv >> 1][r][j] = (unsigned)(ws + j) < (unsigned)W ? v[k] : -__builtin_inff();
+                        }
+                    }
                 }
             }
         }
-    }
-    // Diagonal marches: where the chunk's first and last pixels (so every
-    // lane) put tap t's x in one binade, fl(X + fl(dir.x * t)) - X is the
-    // same for the whole chunk (the table's invariant), so every lane's tap
-    // is the first pixel's shifted by the lane's column, at one distance:
-    // offset and 1/distance per t, and a mask of those t, for the march
-    // below.
-    uint64_t uni_lo = 0, uni_hi = 0;
-    constexpr int ROW_Y = 100 * 8, ROW_X = AO_EXP_N * ROW_Y, BIAS = -AO_EXP_MIN * (ROW_X + ROW_Y);
-    if (ao_fast && (wu & 1)) {
-        const int k = wu >> 1;
-        const float* ox_t = ao_tab + AO_TAB_OFF + wu * 200;
-        const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(ao_tab + AO_TAB_DIST + 2 * k * AO_DIST_PER_DIR), (short)0, AO_DIST_PER_DIR * 8, BUF_DWORD3);
-        const float X0 = (float)x_first, X63 = (float)x_last, Yf = (float)y;
-        bool u0 = false, u1 = false;
-        for (int h = 0; h < 2; h++) {
-            const int t = lane + 64 * h;
-            bool uni = false;
-            if (t < 100) {
-                const float lo = X0 + ox_t[t], hi = X63 + ox_t[t], cy = Yf + ox_t[100 + t];
-                const int kl = __builtin_amdgcn_frexp_expf(lo), kh = __builtin_amdgcn_frexp_expf(hi);
-                uni = (lo > 0.0f) & (kl == kh);
-                const int iy = (int)cy, ky = __builtin_amdgcn_frexp_expf(cy);
-                s_dbase[k][t] = (iy * W + (int)lo) * 4;
-                s_drow[k][t] = (unsigned)iy < (unsigned)H ? iy * W : -(1 << 28);
-                s_dtab[k][t] = ky * ROW_Y + t * 8 + BIAS;
-                const int toff = kl * ROW_X + ky * ROW_Y + t * 8 + BIAS;
-                s_drinv[k][t] =
-                    uni ? __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(trs, toff, 0, 0)) : 0.0;
-            }
-            (h ? u1 : u0) = uni;
-        }
-        uni_lo = __ballot(u0);
-        uni_hi = __ballot(u1);
-    }
-    // the window and the diagonal tables above are this wave's own LDS:
-    // its writes are visible to its lanes past a wave-level fence
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float m = 0.0f;
-    {
-        const float dx = c.ao_dir[2 * wu], dy = c.ao_dir[2 * wu + 1];
-        const float X = (float)x, Y = (float)y;
-        (void)dx;
-        // the tap with the largest exact elevation/distance quotient; its
-        // rounded quotient is the largest rounded quotient.  The general
-        // path compares exact float64 cross products (e * d_best > e_best * d:
-        // products of two float32 are exact).  The table paths compare
-        // q = e * fl64(1 / d) instead, within 2^-52 of e / d: two distinct
-        // quotients of float32 e and d (d a float32 >= 1) differ relatively by
-        // at least 2^-47, and e / d lies at least 2^-47 (relatively) from any
-        // float32 rounding boundary, so q orders distinct quotients exactly
-        // (equal ones may order either way, and round alike) and float(q)
-        // is the correctly rounded float32 quotient.
-        double e_best = -__builtin_inf(), d_best = 1.0, q_best = -__builtin_inf();
-        bool nan = false;
-        // depth taps through a buffer descriptor: an out-of-range offset
-        // reads 0 instead of faulting, so a masked lane needs no clamped
-        // address (its value is never used)
-        const __amdgpu_buffer_rsrc_t drs =
-            __builtin_amdgcn_make_buffer_rsrc((void*)depth, (short)0, W * H * 4, BUF_DWORD3);
-        const float* off_x = ao_tab + AO_TAB_OFF + wu * 200;  // fl(dir.x * t), t = 0..99 (uniform)
-        const float* off_y = off_x + 100;                     // fl(dir.y * t)
-        // one tap: the running argmax of elevation / distance, exact
-        // (bitwise & keeps it a select, not a branch that would serialise
-        // the loads of consecutive taps)
-        auto take = [&](bool v, float e, double d64) {
-            const double e64 = (double)e;
-            const bool better = v & (e64 * d_best > e_best * d64);
-            e_best = better ? e64 : e_best;
-            d_best = better ? d64 : d_best;
-            nan |= v & (e != e);
-        };
-        auto take_q = [&](bool v, float e, double rinv) {
-            const double q = (double)e * rinv;
-            q_best = (v & (q > q_best)) ? q : q_best;
-            nan |= v & (e != e);
-        };
-        // every depth finite: no quotient is NaN (an infinite e gives an
-        // infinite q), so the NaN test can go (uniform)
-        const bool finite = cnt->depth_nonfinite == 0;
-        const double* rinv_t = reinterpret_cast<const double*>(ao_tab + AO_TAB_T64);  // fl64(1 / t) (uniform)
-        // Axis direction, the segment away from the small minor coordinates:
-        // the major offset is exactly +-t and the minor one leaves the tap on
-        // the pixel's row (column), so tap t is the pixel t steps along it,
-        // in the buffer while t < tlim.  Up to the wave's smallest tlim no
-        // lane needs the mask (lanes without AO compute values nobody reads):
-        // a plain running max of q.
-        const bool row_fast = ao_fast && (wu & 1) == 0 && finite && (axis[0] ? y : x_first) >= axis[2];
         if (ao_fast && finite && x_rows && xwin) {  // (directions 0 and 4, whose windows were loaded)
+            // the window is this wave's own LDS: its writes are visible to its
+            // lanes past a wave-level fence
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             // along x: the lane at column li reads tap t at window entry
             // li - 1 + t (li + 99 - t) of its row's window: taps [1, x_t1)
-            // row y's, the rest row x_y2's.  Up to the wave's smallest room
-            // to the border (tmin) no lane needs the mask.
-            const int sgn = axis[1];
-            const int base = sgn > 0 ? li - 1 : li + 99;
-            const int tlim = need ? (sgn > 0 ? W - x : x + 1) : 100;
-            int tl = tlim;  // the wave's smallest
-            for (int k = 32; k >= 1; k >>= 1) tl = min(tl, __shfl_xor(tl, k));
-            const int tmin = min(__builtin_amdgcn_readfirstlane(tl), 100);
-            const int n_rows = x_t1 < 100 ? 2 : 1;
-#pragma nounroll
-            for (int r = 0; r < n_rows; r++) {
-                const int t_lo = r ? x_t1 : 1, t_hi = r ? 100 : x_t1;
-                const int t_mid = min(max(tmin, t_lo), t_hi);
-                const float* win = s_win[wu >> 2][r];
-                // one loop per sign, so each tap's window entry is a constant
-                // offset from the lane's address
-                if (sgn > 0) {
-                    const float* wl = win + li - 1;
-#pragma unroll 4
-                    for (int ti = t_lo; ti < t_mid; ti++)
-                        q_best = __builtin_fmax(q_best, (double)(wl[ti] - dp) * rinv_t[ti]);
+            // row y's, the rest row x_y2's.  A block's largest depth is taken
+            // from its eight entries.  One copy per sign, so each tap's entry
+            // is a constant offset from the lane's address.
+            auto march = [&](auto sign) {
+                constexpr int S = decltype(sign)::value;
+                const float* wl = s_win[wv >> 1][0] + (S > 0 ? li - 1 : li + 99);
+                auto at = [&](int t) { return wl[S * t + (t >= x_t1 ? AO_WIN : 0)]; };
+#pragma unroll
+                for (int t = 1; t < AO_T0; t++) add(b, at(t), rinv_t[t]);
+                auto block = [&](const float* w, int t0) {
+                    float v[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) v[j] = w[S * (t0 + j)];
+                    if (raises(b, ao_max8(v) - dp, rinv_t[t0])) {
+#pragma unroll
+                        for (int j = 0; j < 8; j++) add(b, v[j], rinv_t[t0 + j]);
+                    }
+                };
+                if (x_t1 >= 100) {
+#pragma unroll
+                    for (int i = 0; i < AO_BLOCKS; i++) block(wl, AO_T0 + 8 * i);
                 } else {
-                    const float* wl = win + li + 99;
-#pragma unroll 4
-                    for (int ti = t_lo; ti < t_mid; ti++)
-                        q_best = __builtin_fmax(q_best, (double)(wl[-ti] - dp) * rinv_t[ti]);
+#pragma nounroll
+                    for (int t0 = AO_T0; t0 < 100; t0 += 8) {
+                        if (x_t1 <= t0 || x_t1 >= t0 + 8) {
+                            block(wl + (x_t1 <= t0 ? AO_WIN : 0), t0);
+                        } else {  // the one block on both rows
+#pragma nounroll
+                            for (int t = t0; t < t0 + 8; t++) add(b, at(t), rinv_t[t]);
+                        }
+                    }
                 }
-                for (int ti = t_mid; ti < t_hi; ti++) {
-                    const double q = (double)(win[base + sgn * ti] - dp) * rinv_t[ti];
-                    q_best = (need & (ti < tlim) & (q > q_best)) ? q : q_best;
-                }
-            }
-        } else if (row_fast && !axis[0]) {
-            // along y: tap t is row y +- t, the same for every lane, in the
-            // buffer for t < tl; the march ends there for the whole wave
-            const int sgn = axis[1];
+            };
+            if (axis[1] > 0) march(Int<1>());
+            else march(Int<-1>());
+        } else if (ao_fast && finite && !axis[0] && axis[2] != 0x7fffffff) {
+            // along y: the major offset is exactly +-t, so tap t is row y +- t,
+            // the same for every lane, in the buffer for t < tl; the march
+            // ends there for the whole wave.  The column is the pixel's from
+            // column axis[2] on; left of it the cos/sin residue may move a tap
+            // to the column before (it stays under an ulp of any coordinate
+            // from 1 up, and at 0 truncates to 0).
+            const int sgn = axis[1], step = sgn * W * 4;
             const int tl = min(sgn > 0 ? H - y : y + 1, 100);
+            const __amdgpu_buffer_rsrc_t crs =
+                __builtin_amdgcn_make_buffer_rsrc((void*)a_.ao_col, (short)0, (H + 3) / 4 * W * 4, BUF_DWORD3);
             // the row's offset is uniform (the load's scalar offset), the
             // lane's column its vector offset
-            const int xo = x * 4;
-#pragma unroll 8
-            for (int ti = 1; ti < tl; ti++) {
-                const int row = (y + sgn * ti) * W * 4;
-                const float e = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, xo, row, 0)) - dp;
-                q_best = __builtin_fmax(q_best, (double)e * rinv_t[ti]);
-            }
-        } else if (ao_fast && (wu & 1) == 0) {
+            const int xo = x * 4, xo1 = max(x - 1, 0) * 4, row0 = y * W * 4;
+            auto load = [&](const __amdgpu_buffer_rsrc_t& rs, int vo, int so) {
+                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
+            };
+            auto march = [&](auto own_column) {
+                constexpr bool OWN = decltype(own_column)::value;
+                auto col = [&](int t) { return OWN ? xo : (int)(X + off_x[t]) * 4; };
+                // each block's largest depth (clamped to the frame: a block
+                // past the border is not asked for)
+                float m[AO_BLOCKS];
+#pragma unroll
+                for (int i = 0; i < AO_BLOCKS; i++) {
+                    const int t0 = AO_T0 + 8 * i;
+                    const int row = min(max(sgn > 0 ? y + t0 : y - t0 - 7, 0), H - 1) >> 2;
+                    m[i] = load(crs, xo, row * W * 4);
+                    if (!OWN) m[i] = __builtin_fmaxf(m[i], load(crs, xo1, row * W * 4));
+                }
+                const int n1 = min(AO_T0, tl);
+                for (int t = 1; t < n1; t++) add(b, load(drs, col(t), row0 + t * step), rinv_t[t]);
+                const int n = max(tl - AO_T0, 0) >> 3;
+                blocks(
+                    n, [&](int i) { return raises(b, m[i] - dp, rinv_t[AO_T0 + 8 * i]); },
+                    [&](int i) {
+                        const int t0 = AO_T0 + 8 * i;
+                        float v[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) v[j] = load(drs, col(t0 + j), row0 + (t0 + j) * step);
+#pragma unroll
+                        for (int j = 0; j < 8; j++) add(b, v[j], rinv_t[t0 + j]);
+                    });
+#pragma nounroll
+                for (int t = AO_T0 + 8 * n; t < tl; t++) add(b, load(drs, col(t), row0 + t * step), rinv_t[t]);
+            };
+            if (x_first >= axis[2]) march(std::true_type());
+            else march(std::false_type());
+        } else if (ao_fast) {
             // Axis directions (a = 0, pi/2, pi, 3pi/2 in float32): one offset
             // is exactly +-t, the other the tiny cos/sin residue (<= 8.8e-8 t)
             // rounded onto the coordinate grid, under 2e-5 for coordinates
@@ -1684,16 +1830,69 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
                 const int ix = (int)cx, iy = (int)cy;
                 const bool v = need & ((unsigned)ix < (unsigned)W) & ((unsigned)iy < (unsigned)H);
                 const uint32_t off = (mul_u24((unsigned)iy, (unsigned)W) + (unsigned)ix) * 4u;
-                take_q(v, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp, rinv_t[ti]);
+                take_q(b, v, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp, rinv_t[ti]);
             }
-        } else if (ao_fast) {
+        } else {
+            march_any(b, wa);
+        }
+        r_axis = ratio(b);
+    }
+    {
+        Best b;
+        const float dx = c.ao_dir[2 * wd], dy = c.ao_dir[2 * wd + 1];
+        const ConstF off_x = (ConstF)(ao_tab + AO_TAB_OFF + wd * 200);
+        const ConstF off_y = off_x + 100;
+        // Diagonal marches: where the chunk's first and last pixels (so every
+        // lane) put tap t's x in one binade, fl(X + fl(dir.x * t)) - X is the
+        // same for the whole chunk (the table's invariant), so every lane's tap
+        // is the first pixel's shifted by the lane's column, at one distance:
+        // offset and 1/distance per t, and a mask of those t, for the march
+        // below.
+        uint64_t uni_lo = 0, uni_hi = 0;
+        constexpr int ROW_Y = 100 * 8, ROW_X = AO_EXP_N * ROW_Y, BIAS = -AO_EXP_MIN * (ROW_X + ROW_Y);
+        if (ao_fast) {
+            const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc(
+                (void*)(ao_tab + AO_TAB_DIST + 2 * wv * AO_DIST_PER_DIR), (short)0, AO_DIST_PER_DIR * 8, BUF_DWORD3);
+            const float X0 = (float)x_first, X63 = (float)x_last;
+            bool u0 = false, u1 = false;
+            for (int h = 0; h < 2; h++) {
+                const int t = lane + 64 * h;
+                bool uni = false;
+                if (t < 100) {
+                    const float lo = X0 + off_x[t], hi = X63 + off_x[t], cy = Y + off_y[t];
+                    const int kl = __builtin_amdgcn_frexp_expf(lo), kh = __builtin_amdgcn_frexp_expf(hi);
+                    uni = (lo > 0.0f) & (kl == kh);
+                    const int iy = (int)cy, ky = __builtin_amdgcn_frexp_expf(cy);
+                    s_dbase[wv][t] = (iy * W + (int)lo) * 4;
+                    s_drow[wv][t] = (unsigned)iy < (unsigned)H ? iy * W : -(1 << 28);
+                    s_dtab[wv][t] = ky * ROW_Y + t * 8 + BIAS;
+                    const int toff = kl * ROW_X + ky * ROW_Y + t * 8 + BIAS;
+                    s_drinv[wv][t] =
+                        uni ? __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(trs, toff, 0, 0)) : 0.0;
+                }
+                (h ? u1 : u0) = uni;
+            }
+            if (lane < AO_BLOCKS) {
+                const int t = AO_T0 + 8 * lane;
+                const int iy = (int)(Y + off_y[dy > 0 ? t : t + 7]);
+                s_dbox[wv][lane] = (min(max(iy, 0), H - 1) >> 2) * ((W + 3) / 4) * 4;
+            }
+            uni_lo = __ballot(u0);
+            uni_hi = __ballot(u1);
+        }
+        // the tables above are this wave's own LDS:
+        // its writes are visible to its lanes past a wave-level fence
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (ao_fast) {
             // Diagonal directions: X - fl(X + fl(dir.x * t)) is fixed by t and
             // the binade of the tap coordinate (checked when the table is
             // built, for every coordinate below 4096), so the distance
             // Len = sqrt32(fma64(ex, ex, ey * ey)) is fixed by (binade of cx,
             // binade of cy, t); the table holds fl64(1 / Len).
             const double* dtab =
-                reinterpret_cast<const double*>(ao_tab + AO_TAB_DIST) + ((wu - 1) >> 1) * AO_DIST_PER_DIR;
+                reinterpret_cast<const double*>(ao_tab + AO_TAB_DIST) + wv * AO_DIST_PER_DIR;
             const __amdgpu_buffer_rsrc_t trs =
                 __builtin_amdgcn_make_buffer_rsrc((void*)dtab, (short)0, AO_DIST_PER_DIR * 8, BUF_DWORD3);
             // byte offset of (kx, ky, t) = kx * ROW_X + ky * ROW_Y + t * 8 + BIAS
@@ -1702,7 +1901,6 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
                 float e;
                 bool in;  // in the buffer
             };
-            const int kd = wu >> 1;
             auto tap = [&](int ti) {
                 const float cx = X + off_x[ti];
                 const int ix = (int)cx;
@@ -1712,8 +1910,8 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
                 // (iy = (int)(Y + fl(dir.y * t)), its exponent) is the chunk's,
                 // from the tables above.
                 const int kx = __builtin_amdgcn_frexp_expf(cx);
-                const int row = s_drow[kd][ti];
-                const int toff = mul_i24(kx, ROW_X) + s_dtab[kd][ti];
+                const int row = s_drow[wv][ti];
+                const int toff = mul_i24(kx, ROW_X) + s_dtab[wv][ti];
                 Tap r;
                 r.rinv = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(trs, toff, 0, 0));
                 r.in = ((unsigned)ix < (unsigned)W) & (row >= 0);
@@ -1721,98 +1919,120 @@ __device__ __forceinline__ void k_ao_body(const k_ao_args& a_, const VB vb) {
                 r.e = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp;
                 return r;
             };
-            {
+            auto first = [&]() {
                 const Tap a = tap(1);
-                take_q(need & a.in & (a.rinv <= 1.0), a.e, a.rinv);  // distance < 1 only occurs at t = 1
-            }
-            int ti = 2;
+                take_q(b, need & a.in & (a.rinv <= 1.0), a.e, a.rinv);  // distance < 1 only occurs at t = 1
+            };
             if (finite) {
-                // Taps with t <= r / (|dir| * 1.001), r the room to the border
+                // Taps with t <= 0.999 r / |dir|, r the room to the border
                 // the direction heads for, stay in the buffer whatever the
                 // rounding of fl(X + fl(dir * t)) (off by far less than the
                 // 0.1 % margin): up to the wave's smallest such bound no lane
                 // needs the mask.
-                // And from t >= (r + 2) / (|dir| * 0.999) + 2 on, a lane's tap
+                // And from t >= 1.0011 (r + 2) / |dir| + 2 on, a lane's tap
                 // lies more than a pixel past the border (far beyond the
                 // rounding), where its march has ended: past the wave's
                 // largest such bound no lane has a tap left.
                 int tl = 100, tu = 0;
                 if (need) {
                     const float rx = dx > 0 ? (float)(W - 1 - x) : X, ry = dy > 0 ? (float)(H - 1 - y) : Y;
-                    const float ax = __builtin_fabsf(dx), ay = __builtin_fabsf(dy);
-                    const float lim = fminf(rx / (ax * 1.001f), ry / (ay * 1.001f));
-                    tl = min((int)lim + 1, 100);
-                    const float out = fminf((rx + 2.0f) / (ax * 0.999f), (ry + 2.0f) / (ay * 0.999f));
-                    tu = min((int)out + 2, 100);
+                    // (the reciprocals are within an ulp: nothing to the margin)
+                    const float ax = __builtin_amdgcn_rcpf(__builtin_fabsf(dx));
+                    const float ay = __builtin_amdgcn_rcpf(__builtin_fabsf(dy));
+                    tl = min((int)(fminf(rx * ax, ry * ay) * 0.999f) + 1, 100);
+                    tu = min((int)(fminf((rx + 2.0f) * ax, (ry + 2.0f) * ay) * 1.0011f) + 2, 100);
                 }
                 for (int k = 32; k >= 1; k >>= 1) tl = min(tl, __shfl_xor(tl, k)), tu = max(tu, __shfl_xor(tu, k));
                 const int tmin = __builtin_amdgcn_readfirstlane(tl), tmax = __builtin_amdgcn_readfirstlane(tu);
                 const uint32_t lane4 = (uint32_t)li * 4u;
-                for (; ti + 7 < tmin; ti += 8) {
-                    const uint64_t bits = ti < 64 ? (uni_lo >> ti) | (ti > 56 ? uni_hi << (64 - ti) : 0ull)
-                                                  : uni_hi >> (ti - 64);
-                    if ((bits & 0xFFull) == 0xFFull) {  // eight taps of one shape across the wave
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            const uint32_t off = (uint32_t)s_dbase[kd][ti + j] + lane4;
-                            const float e =
-                                __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp;
-                            q_best = __builtin_fmax(q_best, (double)e * s_drinv[kd][ti + j]);
-                        }
-                    } else {
-#pragma unroll 4
-                        for (int j = 0; j < 8; j++) {
-                            const Tap a = tap(ti + j);
-                            q_best = __builtin_fmax(q_best, (double)a.e * a.rinv);
-                        }
-                    }
-                }
-                for (; ti < tmin; ti++) {
-                    const Tap a = tap(ti);
-                    q_best = __builtin_fmax(q_best, (double)a.e * a.rinv);
-                }
-#pragma unroll 2
-                for (; ti < tmax; ti++) {
-                    const Tap a = tap(ti);
+                auto masked = [&](int t) {
+                    const Tap a = tap(t);
                     const double q = (double)a.e * a.rinv;
-                    q_best = (need & a.in & (q > q_best)) ? q : q_best;
+                    b.q = (need & a.in & (q > b.q)) ? q : b.q;
+                };
+                // The eight taps of a block from t0 lie in the six columns
+                // and six rows from its least ones (7 * 0.7072 < 5 apart, far
+                // beyond the rounding), and those in the buffer in the ones
+                // from there clamped to it: ao_box's nine by nine from that
+                // column and row rounded down to fours hold them.  Their
+                // distances are at least 0.9991 t0 (each offset is within 3e-4
+                // of dir * t for coordinates below 4096).
+                const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
+                    (void*)a_.ao_box, (short)0, (H + 3) / 4 * ((W + 3) / 4) * 4, BUF_DWORD3);
+                const ConstF off_c = off_x + (dx > 0 ? 0 : 7);
+                float m[AO_BLOCKS];
+#pragma unroll
+                for (int i = 0; i < AO_BLOCKS; i++) {
+                    const int ix = min(max((int)(X + off_c[AO_T0 + 8 * i]), 0), W - 1);
+                    m[i] = __uint_as_float(
+                        __builtin_amdgcn_raw_buffer_load_b32(brs, (ix & ~3) + s_dbox[wv][i], 0, 0));
                 }
-            } else {
+                // (distance < 1 only occurs at t = 1)
+                if (tmin >= AO_T0 && ((uni_lo >> 1) & ((1u << (AO_T0 - 1)) - 1u)) == (1u << (AO_T0 - 1)) - 1u) {
+#pragma unroll
+                    for (int t = 1; t < AO_T0; t++) {
+                        const float d = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            drs, (int)((uint32_t)s_dbase[wv][t] + lane4), 0, 0));
+                        if (t > 1 || s_drinv[wv][t] <= 1.0) add(b, d, s_drinv[wv][t]);
+                    }
+                } else {
+                    first();
+#pragma unroll
+                    for (int t = 2; t < AO_T0; t++) masked(t);
+                }
+                blocks(
+                    max(tmax - AO_T0 + 7, 0) >> 3,  // (the blocks with a tap before tmax)
+                    [&](int i) { return raises(b, (m[i] - dp) * 1.001f, rinv_t[AO_T0 + 8 * i]); },
+                    [&](int i) {
+                        const int t0 = AO_T0 + 8 * i;
+                        const uint64_t bits = t0 < 64 ? (uni_lo >> t0) | (t0 > 56 ? uni_hi << (64 - t0) : 0ull)
+                                                      : uni_hi >> (t0 - 64);
+                        if (t0 + 7 >= tmin) {
 #pragma unroll 2
-                for (; ti < 100; ti++) {
+                            for (int j = 0; j < 8; j++) masked(t0 + j);
+                        } else if ((bits & 0xFFull) == 0xFFull) {  // eight taps of one shape across the wave
+                            float v[8];
+#pragma unroll
+                            for (int j = 0; j < 8; j++)
+                                v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                    drs, (int)((uint32_t)s_dbase[wv][t0 + j] + lane4), 0, 0));
+#pragma unroll
+                            for (int j = 0; j < 8; j++) add(b, v[j], s_drinv[wv][t0 + j]);
+                        } else {
+#pragma unroll 4
+                            for (int j = 0; j < 8; j++) {
+                                const Tap a = tap(t0 + j);
+                                b.q = __builtin_fmax(b.q, (double)a.e * a.rinv);
+                            }
+                        }
+                    });
+            } else {
+                first();
+#pragma unroll 2
+                for (int ti = 2; ti < 100; ti++) {
                     const Tap a = tap(ti);
-                    take_q(need & a.in, a.e, a.rinv);
+                    take_q(b, need & a.in, a.e, a.rinv);
                 }
             }
         } else {
-            float t = 1.0f;  // t = 0 is the pixel itself: distance 0 < 1, skipped
-#pragma unroll 3
-            for (int ti = 1; ti < 100; ti++, t += 1.0f) {
-                const float cx = X + dx * t, cy = Y + dy * t;
-                const int ix = (int)cx, iy = (int)cy;  // |cx|, |cy| < 2^31: Go's int() truncation
-                const float ex = X - cx, ey = Y - cy;
-                // Len of (ex, ey, 0, 0): FMA(ex,ex, FMA(ey,ey, FMA(0,0,0*0))) where
-                // the inner FMA(ey,ey,+0) is exactly the float32 product ey*ey
-                const float dist = sqrt32_normal(fma64(ex, ex, ey * ey));
-                const bool v = need & ((unsigned)ix < (unsigned)W) & ((unsigned)iy < (unsigned)H) & (dist >= 1.0f);
-                const uint32_t off = (mul_u24((unsigned)iy, (unsigned)W) + (unsigned)ix) * 4u;
-                take(v, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(drs, (int)off, 0, 0)) - dp, (double)dist);
-            }
+            march_any(b, wd);
         }
-        const float maxr = ao_fast ? (float)q_best : (float)e_best / (float)d_best;
-        m = nan ? __builtin_nanf("") : (maxr > 0 ? (float)atan64((double)maxr) : 0.0f);
+        r_diag = ratio(b);
     }
-    s_m[wu][lane] = m;
+#pragma nounroll
+    for (int h = 0; h < 2; h++) {
+        const float r = h ? r_diag : r_axis;
+        s_m[2 * wv + h][lane] = ao_atan(r);
     }
     __syncthreads();
     if (wv == 0 && need) {
         float total = 0.0f;
         for (int k = 0; k < 8; k++) total += 1.57079632679489661923f - s_m[k][lane];
         total /= 12.5663706143591729539f;
-        ao[(size_t)y * W + x] = (float)pow64((double)total, 10000.0);
+        ao[(size_t)y * W + x] = pow32_fast(total, 10000.0f);
     }
 }
-__global__ __launch_bounds__(256) void k_ao(k_ao_args a) {
+__global__ __launch_bounds__(256, 8) void k_ao(k_ao_args a) {
     k_ao_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
 }
 __global__ __launch_bounds__(256) void k_ao_wide(const k_ao_args* __restrict__ a, const int32_t* __restrict__ start,
@@ -2250,9 +2470,14 @@ void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters
     else go(k_resolve<false>, k_resolve_wide<false>, dim3(rt.H), 256, st, a);
 }
 void launch_ao(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b) {
+    if (c.v.W <= 0 || c.v.H <= 0) return;
+    if (b.ao_fast)
+        go(k_ao_max, k_ao_max_wide, dim3(blocks_for(c.v.W, 256), (c.v.H + 3) / 4), 256, st,
+           k_ao_max_args{b.depth, b.ao_col, b.ao_box, c.v.W, c.v.H, &b.cnt->c, 0, 0});
+    else if (g_wide) g_wide->sub++;  // (its place in the recorded batch stays empty)
     const int nb = ((c.v.W + 63) / 64) * c.v.H;
     go(k_ao, k_ao_wide, dim3(((nb + 7) / 8) * 8), 256, st,
-       k_ao_args{c, b.ao_xs, b.ao_cnt, b.depth, b.ao, b.ao_tab, b.ao_fast, &b.cnt->c, 0, 0});
+       k_ao_args{c, b.ao_xs, b.ao_cnt, b.depth, b.ao, b.ao_col, b.ao_box, b.ao_tab, b.ao_fast, &b.cnt->c, 0, 0});
 }
 void launch_shade_bg(hipStream_t st, const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b, Stamp stamp) {
     go(k_shade_bg, k_shade_bg_wide, dim3(1), 64, st, k_shade_bg_args{s, c, b, stamp, 0, 0});

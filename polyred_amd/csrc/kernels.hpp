@@ -59,6 +59,7 @@ struct ShadeBuffers {
     float* ao;                 // [H][W] AO factor of the pixels that need it
     int32_t* ao_xs;            // [H][W] per row, the columns of the pixels k_ao computes, left to right (k_resolve)
     int32_t* ao_cnt;           // [H] and their count
+    float *ao_col, *ao_box;    // [(H+3)/4][W] and [(H+3)/4][(W+3)/4], the marches' depth bounds (k_ao_max)
     const float* ao_tab;       // AO march tables (tap offsets, diagonal distances)
     int32_t ao_fast;           // the tables hold for this frame size
     uint32_t* col_pre;         // set: k_shade is the first half of a split shading (colour before AO)

@@ -445,6 +445,7 @@ struct prh_renderer {
     int rz_flx, rz_fly;
     float *linear, *bg_lin, *ao;
     int32_t *ao_xs, *ao_cnt;  // scenes with AO only: the rows' lists of AO pixels
+    float *ao_col, *ao_box;   // and the marches' depth bounds
     float* ao_tab;   // AO march tables (ao_tables)
     int32_t ao_fast; // the tables hold for this frame size
     PassCounters* cnt;  // [2]: main, shadow
@@ -1027,6 +1028,8 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     if (!rc) chk(ralloc(r, &r->ao, P));
     if (!rc && s->any_ao) chk(ralloc(r, &r->ao_xs, P));
     if (!rc && s->any_ao) chk(ralloc(r, &r->ao_cnt, (size_t)r->H));
+    if (!rc && s->any_ao) chk(ralloc(r, &r->ao_col, (size_t)((r->H + 3) / 4) * r->W));
+    if (!rc && s->any_ao) chk(ralloc(r, &r->ao_box, (size_t)((r->H + 3) / 4) * ((r->W + 3) / 4)));
     if (!rc && s->any_ao && r->n_slots > 0) chk(ralloc(r, &r->col_pre, P));
     if (!rc && s->any_ao && r->n_slots > 0) chk(ralloc(r, &r->post_flag, P));
     if (!rc && msaa == 1) chk(ralloc(r, &r->image, P));
@@ -1133,7 +1136,7 @@ ShadeBuffers shade_buffers(const prh_renderer* r) {
     b.cnt = r->cnt;
     b.cnt_host = r->d_h_cnt;
     b.ao = r->ao;
-    b.ao_xs = r->ao_xs, b.ao_cnt = r->ao_cnt;
+    b.ao_xs = r->ao_xs, b.ao_cnt = r->ao_cnt, b.ao_col = r->ao_col, b.ao_box = r->ao_box;
     b.ao_tab = r->ao_tab, b.ao_fast = r->ao_fast;
     b.col_pre = nullptr, b.post_flag = nullptr;
     return b;
