@@ -2044,11 +2044,24 @@ __global__ __launch_bounds__(256) void k_ao_wide(const k_ao_args* __restrict__ a
     k_ao_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
 }
 
+// The frame's counters are final before the shading: one workgroup hands them
+// to the host's pinned copy (main then shadow), in place of a copy after the
+// frame.
+__device__ __forceinline__ void counters_to_host(const ShadeBuffers& b) {
+    constexpr int CW = sizeof(Counters) / 4;
+    if (b.cnt_host && threadIdx.x < 2 * CW)
+        reinterpret_cast<int32_t*>(b.cnt_host)[threadIdx.x] =
+            reinterpret_cast<const int32_t*>(&b.cnt[threadIdx.x / CW].c)[threadIdx.x % CW];
+}
+
 // The colour of every uncovered pixel (render/raster.go:324-328 with
 // raster_screen.go:75-87): DrawFragment hands `shade` the zero fragment, whose
 // X = Y = 0 and MaterialID = 0, so it is shaded from pixel (0,0)'s stored
 // fragment with material table[0]; if pixel (0,0) is uncovered it is the
 // Background.  With no material 0 the colour is pixel (0,0)'s own final one.
+// One thread's latency: the fragment is shaded once (shading it with its own
+// material too, which nobody reads where there is a material 0, took 25 us of
+// a 1600x1200 textured frame in place of 12).
 struct k_shade_bg_args {
     DevScene s;
     ShadeConsts c;
@@ -2063,27 +2076,17 @@ __device__ __forceinline__ void k_shade_bg_body(const k_shade_bg_args& a_, const
     const ShadeBuffers& b = a_.b;
 
     if (vb.bx != 0) return;
-    // the frame's counters are final here: hand them to the host's pinned
-    // copy (main then shadow), in place of a copy after the frame
-    constexpr int CW = sizeof(Counters) / 4;
-    if (b.cnt_host && threadIdx.x < 2 * CW)
-        reinterpret_cast<int32_t*>(b.cnt_host)[threadIdx.x] =
-            reinterpret_cast<const int32_t*>(&b.cnt[threadIdx.x / CW].c)[threadIdx.x % CW];
+    counters_to_host(b);
     if (threadIdx.x != 0 || b.cnt->c.overflow) return;
     const uint64_t k00 = b.vis[0];
     float lin[3] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
     uint32_t col = c.background;
     if (k00 != VIS_EMPTY) {
-        GFrag f = fetch_fragment(s, c, b, 0, 0, k00);
+        const GFrag f = fetch_fragment(s, c, b, 0, 0, k00);
         bool hl;
-        float own_lin[3];
-        uint32_t own = shade_fragment(s, c, b, f, 0, 0, f.mat, f.col, own_lin, hl);
-        if (s.n_materials > 0) {
-            col = shade_fragment(s, c, b, f, 0, 0, 0, f.col, lin, hl);
-            if (!hl) lin[0] = lin[1] = lin[2] = __builtin_nanf("");
-        } else {
-            col = own;
-        }
+        // (without materials f.mat is -1: pixel (0,0)'s vertex colour)
+        col = shade_fragment(s, c, b, f, 0, 0, s.n_materials > 0 ? 0 : f.mat, f.col, lin, hl);
+        if (!hl) lin[0] = lin[1] = lin[2] = __builtin_nanf("");
     }
     b.bg[0] = col;
     b.bg_lin[0] = lin[0], b.bg_lin[1] = lin[1], b.bg_lin[2] = lin[2];
@@ -2120,7 +2123,10 @@ __device__ __forceinline__ void shade_tile(const DevScene& s, const ShadeConsts&
     const int y = (tile / tiles_x) * TILE + (wv >> 1) * 8 + (lane >> 3);
     if (x >= c.v.W || y >= c.v.H) return;
     const size_t o = (size_t)y * c.v.W + x;
-    const uint64_t key = b.vis[o];
+    const uint64_t own_key = b.vis[o];
+    // an uncovered pixel as pixel (0,0) with material 0 (k_shade_bg's colour)
+    const bool as_origin = own_key == VIS_EMPTY && b.bg_inline;
+    const uint64_t key = as_origin ? b.vis[0] : own_key;
     uint32_t col;
     float lin[3] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
     bool hl = false;
@@ -2130,12 +2136,16 @@ __device__ __forceinline__ void shade_tile(const DevScene& s, const ShadeConsts&
             b.post_flag[o] = 2;
             return;
         }
-        col = b.bg[0];
-        lin[0] = b.bg_lin[0], lin[1] = b.bg_lin[1], lin[2] = b.bg_lin[2];
+        col = c.background;
+        if (!b.bg_inline) {
+            col = b.bg[0];
+            lin[0] = b.bg_lin[0], lin[1] = b.bg_lin[1], lin[2] = b.bg_lin[2];
+        }
         hl = true;
     } else {
-        GFrag f = fetch_fragment(s, c, b, x, y, key);
-        col = shade_fragment(s, c, b, f, x, y, f.mat, f.col, lin, hl);
+        const int fx = as_origin ? 0 : x, fy = as_origin ? 0 : y;
+        const GFrag f = fetch_fragment(s, c, b, fx, fy, key);
+        col = shade_fragment(s, c, b, f, fx, fy, as_origin && s.n_materials > 0 ? 0 : f.mat, f.col, lin, hl);
         if (b.col_pre) flag = f.mat >= 0 && s.mats[f.mat].ambient_occlusion;
     }
     if (b.col_pre) {
@@ -2158,20 +2168,26 @@ __device__ __forceinline__ void shade_tile(const DevScene& s, const ShadeConsts&
         b.linear[3 * o + 2] = hl ? lin[2] : __builtin_nanf("");
     }
     b.image[(size_t)(c.v.H - 1 - y) * c.v.W + x] = gamma(c, col);
+    // (stores only after the loads: ahead of them they would make the uniform
+    // ones vector loads)
+    if (b.depth_out) {
+        const uint32_t hi = (uint32_t)(own_key >> 32);
+        b.depth_out[o] = own_key == VIS_EMPTY ? -1.0f : (hi == KEY_HI_NAN ? __builtin_nanf("") : depth_from_key_hi(hi));
+    }
 }
 __device__ __forceinline__ void k_shade_body(const k_shade_args& a_, const VB vb) {
     const DevScene& s = a_.s;
     const ShadeConsts& c = a_.c;
     const ShadeBuffers& b = a_.b;
 
-    if (b.cnt->c.overflow) return;
     const int tiles_x = c.v.tiles_x, tiles_y = c.v.tiles_y;
     // workgroup i shades tile i: the dispatcher deals consecutive
     // workgroups round-robin to the 8 XCDs, so every XCD gets a share of
     // every part of the frame (the covered pixels, whose shading is the
     // work, crowd where the ground is)
     const int tile = vb.bx;
-    if (tile < tiles_x * tiles_y) shade_tile(s, c, b, tile);
+    if (tile < tiles_x * tiles_y && !b.cnt->c.overflow) shade_tile(s, c, b, tile);
+    if (b.bg_inline && tile == 0) counters_to_host(b);
     stamp_end(a_.stamp, vb);
 }
 __global__ __launch_bounds__(256) void k_shade(k_shade_args a) {

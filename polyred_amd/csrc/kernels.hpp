@@ -62,6 +62,8 @@ struct ShadeBuffers {
     float *ao_col, *ao_box;    // [(H+3)/4][W] and [(H+3)/4][(W+3)/4], the marches' depth bounds (k_ao_max)
     const float* ao_tab;       // AO march tables (tap offsets, diagonal distances)
     int32_t ao_fast;           // the tables hold for this frame size
+    int32_t bg_inline;         // k_shade shades the uncovered pixels itself: no k_shade_bg ran
+    float* depth_out;          // set: no k_resolve ran, and k_shade writes the depth
     uint32_t* col_pre;         // set: k_shade is the first half of a split shading (colour before AO)
     uint8_t* post_flag;        // and per pixel what the second half does: 0 colour as is, 1 with the AO
                                // factor, 2 uncovered (the uncovered colour)

@@ -355,6 +355,13 @@ enum {
     ST_SHADOW, ST_SHADOW_END, ST_VERTEX, ST_VERTEX_END, ST_SETUP_END, ST_RESOLVED, ST_BG, ST_BG_END, ST_SHADE_END,
     ST_END, N_STAMPS
 };
+// Frames without AO of up to this many pixels have their uncovered pixels
+// shade pixel (0,0) each for itself, instead of reading the colour a kernel of
+// one workgroup computed before: at most two waves a SIMD, so the chip has the
+// room, and the frame is a kernel shorter.  256x256: 81 -> 73 us; at 512x512
+// and 1001x701 no difference (436 and 220 us either way), nor with AO at
+// 480x270.
+constexpr size_t BG_INLINE_PIXELS = 1 << 17;
 
 struct prh_renderer;
 // prh_render_batch spreads a batch over one stream per hardware queue the
@@ -470,6 +477,7 @@ struct prh_renderer {
     uint32_t* present_to;  // during prh_surface_render: the acquired surface texture
     prh_tuning tune;       // speed knobs (results do not depend on them)
     bool split_shade_last;  // the last frame split its shading
+    int raster_end_last;    // the stamp its raster pass ends at
     // the last frame's per-pass times wait in its stamps until the stats are
     // read (prh_last_stats): a frame's own host work stays short
     bool times_pending, times_nan_rerun;
@@ -1126,7 +1134,7 @@ namespace {
 uint32_t* final_image(const prh_renderer* r) { return r->present_to ? r->present_to : r->image; }
 
 ShadeBuffers shade_buffers(const prh_renderer* r) {
-    ShadeBuffers b;
+    ShadeBuffers b{};
     b.vis = r->vis, b.depth = r->depth, b.tv_scr = r->tv_scr, b.tv_nor = r->tv_nor, b.tv_wp = r->tv_wp;
     b.tri_rec = r->tri_rec, b.tv_col = r->tv_col, b.tv_uv = r->tv_uv;
     b.clips = r->clips, b.tri_clip_slot = r->tri_clip_slot, b.smaps = r->smaps;
@@ -1208,11 +1216,22 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     }
     RasterTarget rt{r->W, r->H, (unsigned long long*)r->vis, r->first_all, r->first_nan, nullptr};
     wide_stage(11);
-    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt, Stamp{});
+    // the depth buffer: by the resolve where the AO reads it (or the exact
+    // pass settles it), else by the shading, a kernel less (4 to 7 us of a
+    // frame)
+    const bool resolve = r->sc->any_ao || nan_mode;
+    // without AO and up to BG_INLINE_PIXELS no k_shade_bg runs either
+    const bool bg_inline = !r->sc->any_ao && !wide && P <= BG_INLINE_PIXELS;
+    // (the pass ends with the resolve, else where k_shade_bg starts, else with
+    // the raster: of its unequal workgroups a stamp sees a few)
+    r->raster_end_last = resolve || bg_inline ? ST_RESOLVED : ST_BG;
+    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt, at(-1, !resolve && bg_inline ? ST_RESOLVED : -1));
     wide_stage(12);
-    launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec,
-                   at(-1, ST_RESOLVED));
-    const ShadeBuffers b = shade_buffers(r);
+    if (resolve)
+        launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec,
+                       at(-1, ST_RESOLVED));
+    ShadeBuffers b = shade_buffers(r);
+    if (!resolve) b.depth_out = r->depth;
     // the split shading's buffers: both halves read and write col_pre
     ShadeBuffers bp = b;
     bp.col_pre = r->col_pre, bp.post_flag = r->post_flag;
@@ -1234,7 +1253,8 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     if (r->sc->any_ao && !split_shade) launch_ao(st, d, r->sh, b);  // else no pixel reads an AO factor
     if (split) (void)hipStreamWaitEvent(st, r->ev_join, 0);  // the shadow maps (and the AO factors)
     wide_stage(14);
-    if (!split_shade) launch_shade_bg(st, d, r->sh, b, at(ST_BG, ST_BG_END));
+    b.bg_inline = bg_inline;
+    if (!split_shade && !bg_inline) launch_shade_bg(st, d, r->sh, b, at(ST_BG, ST_BG_END));
     wide_stage(15);
     const int last = r->msaa > 1 ? -1 : ST_END;
     if (!split_shade) launch_shade(st, d, r->sh, b, at(-1, last));
@@ -1890,12 +1910,14 @@ int fill_times(prh_renderer* r) {
     S.ms_shadow = shadow ? ms(t[ST_SHADOW], t[ST_SHADOW_END]) : 0.0f;  // (beside the main view's passes: their own span)
     S.ms_vertex = ms(t[ST_VERTEX], t[ST_VERTEX_END]);
     S.ms_setup = ms(t[ST_VERTEX_END], setup_end);
-    S.ms_raster = ms(setup_end, t[ST_RESOLVED]);
-    S.ms_ao = ao ? ms(t[ST_RESOLVED], t[ST_BG]) : 0.0f;
+    const unsigned long long raster_end = t[r->raster_end_last], shadow_end = shadow ? t[ST_SHADOW_END] : 0;
+    S.ms_raster = ms(setup_end, raster_end);
+    S.ms_ao = ao ? ms(raster_end, t[ST_BG]) : 0.0f;
     // (split shading: the first half beside the AO, and the second)
-    S.ms_shade = r->split_shade_last ? ms(std::max(t[ST_RESOLVED], t[ST_SHADOW_END]), t[ST_SHADE_END]) +
+    const unsigned long long ready = std::max(ao ? t[ST_BG] : raster_end, shadow_end);
+    S.ms_shade = r->split_shade_last ? ms(std::max(raster_end, shadow_end), t[ST_SHADE_END]) +
                                            ms(std::max(t[ST_SHADE_END], t[ST_BG_END]), t[ST_END])
-                                     : ms(t[ST_BG], t[ST_END]);
+                                     : ms(ready, t[ST_END]);
     return PRH_OK;
 }
 
