@@ -2244,6 +2244,66 @@ __global__ __launch_bounds__(256) void k_shade_post(DevScene s, ShadeConsts c, S
     stamp_end(stamp, VB{(int)blockIdx.x, 0, (int)gridDim.x, 1});
 }
 
+// ------------------------------------------------------------- host copies
+// n bytes by all the launch's threads, `part` of `parts` workgroups, in the
+// widest unit the addresses allow.  OUT: to host memory, in stores of system
+// scope (no cache holds them back, so a wait for them is all that the flag
+// below needs: a fence writes the caches back, once a wave, and took a third
+// of the copy's time).
+template <bool OUT, class T>
+__device__ __forceinline__ size_t copy_units(uint8_t* dst, const uint8_t* src, size_t n, size_t i0, size_t step) {
+    T* d = reinterpret_cast<T*>(dst);
+    const T* s = reinterpret_cast<const T*>(src);
+    for (size_t i = i0; i < n / sizeof(T); i += 4 * step) {
+        T v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i + k * step < n / sizeof(T)) v[k] = s[i + k * step];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i + k * step < n / sizeof(T)) {
+                if (OUT) __hip_atomic_store(&d[i + k * step], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                else d[i + k * step] = v[k];
+            }
+    }
+    return n / sizeof(T) * sizeof(T);
+}
+template <bool OUT>
+__device__ __forceinline__ void copy_part(uint8_t* dst, const uint8_t* src, size_t n, int part, int parts) {
+    const size_t i0 = part * (size_t)blockDim.x + threadIdx.x, step = parts * (size_t)blockDim.x;
+    const uintptr_t a = (uintptr_t)dst | (uintptr_t)src;
+    size_t done = 0;
+    if ((a & 7) == 0) done = copy_units<OUT, unsigned long long>(dst, src, n, i0, step);
+    else if ((a & 3) == 0) done = copy_units<OUT, uint32_t>(dst, src, n, i0, step);
+    copy_units<OUT, uint8_t>(dst + done, src + done, n - done, i0, step);
+}
+// Page-locked host memory to the device, read over the link.
+__global__ __launch_bounds__(256) void k_pull(uint8_t* dst, const uint8_t* src, size_t n) {
+    copy_part<false>(dst, src, n, (int)blockIdx.x, (int)gridDim.x);
+}
+// Device memory into page-locked host memory, chunk by chunk: once a chunk is
+// whole its flag is set to `serial`, so that the host takes it from there
+// while the next ones cross the link.  Even and odd chunks by different
+// workgroups (`sets`): one half writes while the other waits for its last
+// writes to arrive.
+__global__ __launch_bounds__(256) void k_push(PushArgs a) {
+    const int set = (int)blockIdx.x % a.sets, part = (int)blockIdx.x / a.sets, parts = (int)gridDim.x / a.sets;
+    for (int k = set; k < a.n_chunks; k += a.sets) {
+        const uint32_t c0 = (uint32_t)k * a.chunk, c1 = c0 + a.chunk;
+        for (int i = 0; i < a.n_segs; i++) {
+            const PushSeg& s = a.seg[i];
+            const uint32_t lo = max(c0, s.off), hi = min(c1, s.off + s.n);
+            if (lo < hi) copy_part<true>(a.dst + lo, s.src + (lo - s.off), hi - lo, part, parts);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's stores have arrived
+        __syncthreads();
+        if (threadIdx.x == 0 && atomicAdd(&a.done[k], 1u) == (uint32_t)parts - 1u) {
+            a.done[k] = 0u;
+            __hip_atomic_store(&a.flags[k], a.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
 // ------------------------------------------------------------- launchers
 static inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -2403,6 +2463,19 @@ void launch_frame_clear(hipStream_t st, uint32_t* cnt, int32_t n_cnt, uint64_t* 
 void launch_fill_u64(hipStream_t st, uint64_t* p, size_t n, uint64_t v) {
     if (!n) return;
     hipLaunchKernelGGL(k_fill_u64, dim3(std::min<size_t>(blocks_for(n, 256), 4096)), dim3(256), 0, st, p, n, v);
+}
+void launch_pull(hipStream_t st, uint8_t* dst, const uint8_t* src, size_t n) {
+    // (a few loads in flight a thread: 1 MB of them is more than the link's
+    // latency holds)
+    const unsigned wg = std::min<size_t>(blocks_for(n, 256 * 16), 256);
+    if (n) hipLaunchKernelGGL(k_pull, dim3(wg), dim3(256), 0, st, dst, src, n);
+}
+void launch_push(hipStream_t st, PushArgs a) {
+    a.sets = a.n_chunks > 1 ? 2 : 1;
+    uint32_t n = 0;
+    for (int i = 0; i < a.n_segs; i++) n += a.seg[i].n;
+    const unsigned parts = std::min<size_t>(blocks_for(std::min(n, a.chunk), 256 * 32), 64);
+    hipLaunchKernelGGL(k_push, dim3(std::max(parts, 1u) * a.sets), dim3(256), 0, st, a);
 }
 // The clear on its own where the vertex pass has nothing to launch (a group
 // of its own in a recorded batch, beside the views' vertex passes).

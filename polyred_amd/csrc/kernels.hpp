@@ -169,6 +169,25 @@ struct Stamp {
     unsigned long long* end = nullptr;
 };
 
+// Host copies (k_push, k_pull): device memory src[0, n) to dst[off, off + n).
+constexpr int PUSH_SEGS = 4, PUSH_CHUNKS = 32;
+struct PushSeg {
+    const uint8_t* src;
+    uint32_t off, n;
+};
+struct PushArgs {
+    PushSeg seg[PUSH_SEGS];
+    int32_t n_segs;
+    uint8_t* dst;  // page-locked host memory, as the device sees it
+    uint32_t chunk;  // a multiple of 16
+    int32_t n_chunks, sets;
+    uint32_t* done;   // [PUSH_CHUNKS] zero before and after
+    uint32_t* flags;  // [PUSH_CHUNKS] page-locked host memory
+    uint32_t serial;
+};
+void launch_pull(hipStream_t st, uint8_t* dst, const uint8_t* src, size_t n);
+void launch_push(hipStream_t st, PushArgs a);
+
 void launch_fill_u32(hipStream_t st, uint32_t* p, size_t n, uint32_t v);
 void launch_fill_u64(hipStream_t st, uint64_t* p, size_t n, uint64_t v);
 void launch_frame_clear(hipStream_t st, uint32_t* cnt, int32_t n_cnt, uint64_t* vis, size_t n_vis, Stamp stamp);
