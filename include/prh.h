@@ -294,10 +294,9 @@ int prh_diff_backward_noalloc(prh_renderer* r, const prh_diff_params* p, const f
  * as the reference scales the shaded colour (render/raster.go:339-347).  One
  * step is one launch of the adjoint over every view (gradients summed over
  * views) and one Adam update (Kingma & Ba 2015) of the chosen parameter
- * groups, parametrised as p = start * (1 + theta), theta starting at 0; the
- * steps of a run are one captured HIP graph replayed.  The loss is the sum
- * over views of prh_diff_backward's loss.  kd, ks, shininess, light
- * intensities and albedo are kept >= 0. */
+ * groups, parametrised as p = start * (1 + theta), theta starting at 0.  The
+ * loss is the sum over views of prh_diff_backward's loss.  kd, ks, shininess,
+ * light intensities and albedo are kept >= 0. */
 typedef struct prh_fit prh_fit;
 #define PRH_FIT_ALBEDO 1 /* (normals are not fitted) */
 #define PRH_FIT_KD 4

@@ -815,6 +815,20 @@ __global__ __launch_bounds__(256) void k_diff_clear(float* __restrict__ grad, si
     if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
 }
 
+// A fit's start: the parameters kept as the base, the Adam state and what the
+// steps accumulate at zero (one kernel in place of a copy and five fills).
+__global__ __launch_bounds__(256) void k_fit_start(const float* __restrict__ par, float* __restrict__ base,
+                                                   float* __restrict__ theta, float* __restrict__ m,
+                                                   float* __restrict__ v, size_t n, float* __restrict__ grad,
+                                                   size_t n_grad, double* __restrict__ loss, int32_t* count,
+                                                   int32_t* step) {
+    const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = i0; i < n; i += stride) base[i] = par[i], theta[i] = m[i] = v[i] = 0.0f;
+    for (size_t i = i0; i < n_grad; i += stride) grad[i] = 0.0f;
+    if (i0 < DIFF_REPS) loss[i0] = 0.0;
+    if (i0 == 0) *count = 0, *step = 0;
+}
+
 __global__ __launch_bounds__(256) void k_diff_gbuffer(DevScene s, ViewConsts v, DiffBuffers b, float4* __restrict__ g) {
     const size_t P = (size_t)v.W * v.H;
     const size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
@@ -906,6 +920,12 @@ void launch_diff_forward_views(hipStream_t st, const DevScene& s, const DiffView
 void launch_diff_clear(hipStream_t st, float* grad, size_t n, double* loss, int32_t* count) {
     const unsigned grid = (unsigned)std::min<size_t>((n + 255) / 256 + 1, 1024);
     hipLaunchKernelGGL(k_diff_clear, dim3(grid), dim3(256), 0, st, grad, n, loss, count);
+}
+void launch_fit_start(hipStream_t st, const float* par, float* base, float* theta, float* m, float* v, size_t n,
+                      float* grad, size_t n_grad, double* loss, int32_t* count, int32_t* step) {
+    const unsigned grid = (unsigned)std::min<size_t>((std::max(n, n_grad) + 255) / 256 + 1, 1024);
+    hipLaunchKernelGGL(k_fit_start, dim3(grid), dim3(256), 0, st, par, base, theta, m, v, n, grad, n_grad, loss, count,
+                       step);
 }
 void launch_diff_list(hipStream_t st, const DiffView& w, uint2* chunks, int32_t* count) {
     const int n = n_strips(w.v);

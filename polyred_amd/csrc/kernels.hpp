@@ -117,6 +117,8 @@ void launch_diff_forward_views(hipStream_t st, const DevScene& s, const DiffView
 // The adjoint: the gradients (n floats), the loss and the count of chunks
 // zeroed, the views' shaded pixels listed, then the adjoint over the list.
 void launch_diff_clear(hipStream_t st, float* grad, size_t n, double* loss, int32_t* count);
+void launch_fit_start(hipStream_t st, const float* par, float* base, float* theta, float* m, float* v, size_t n,
+                      float* grad, size_t n_grad, double* loss, int32_t* count, int32_t* step);
 void launch_diff_list(hipStream_t st, const DiffView& w, uint2* chunks, int32_t* count);
 void launch_diff_list_views(hipStream_t st, const DiffView* views, int32_t n, int32_t strips, uint2* chunks,
                             int32_t* count);

@@ -630,11 +630,11 @@ int stage_wait(volatile uint32_t* flag, uint32_t serial, hipStream_t st) {
     for (uint32_t k = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != serial; k++) {
         __builtin_ia32_pause();
         if (k % 4096) continue;
-        const hipError_t e = hipStreamQuery(st);
-        if (e == hipErrorNotReady) {
+        if (hipStreamQuery(st) == hipErrorNotReady) {
             (void)hipGetLastError();
             continue;
         }
+        const hipError_t e = hipStreamSynchronize(st);
         if (e != hipSuccess) return fail(PRH_E_HIP, std::string("copy to the host: ") + hipGetErrorString(e));
         if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != serial) return fail(PRH_E_HIP, "copy to the host: not completed");
     }
@@ -1915,9 +1915,9 @@ int fit_views(prh_fit* f, bool backward, uint32_t want, hipStream_t st) {
         strip += diff_strips(r->vc);
     }
     f->total_blocks = blk, f->total_strips = strip;
-    HIP_TRY(hipMemcpyAsync(f->d_views, h.data(), h.size() * sizeof(DiffView), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));  // h is a local
-    return PRH_OK;
+    const int rc = stage_up(f->ctx, f->d_views, h.data(), h.size() * sizeof(DiffView), st);
+    if (!rc && f->ctx->stage_failed) HIP_TRY(hipStreamSynchronize(st));  // h is a local
+    return rc;
 }
 
 // The optimised indices of the parameter block and their lower bounds.
@@ -2329,7 +2329,6 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     const DiffLayout& l = f->l;
     // parameters and the Adam state
     if ((rc = upload_params(f->views[0], l, start, f->par, st))) return rc;
-    HIP_TRY(hipMemcpyAsync(f->base, f->par, l.total * 4, hipMemcpyDeviceToDevice, st));
     std::vector<int32_t> idx;
     std::vector<float> lower;
     fit_groups(f, o->groups, idx, lower);
@@ -2338,12 +2337,9 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
         if ((rc = stage_up(f->ctx, f->idx, idx.data(), idx.size() * 4, st))) return rc;
         if ((rc = stage_up(f->ctx, f->lower, lower.data(), lower.size() * 4, st))) return rc;
     }
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->theta), l.total, 0u);
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->m), l.total, 0u);
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->v), l.total, 0u);
-    launch_fill_u32(st, reinterpret_cast<uint32_t*>(f->step), 1, 0u);
     // (each step's Adam pass leaves the gradients it read, and the loss, at zero)
-    launch_diff_clear(st, f->grad, l.grad_total(), f->loss, f->n_chunks);
+    launch_fit_start(st, f->par, f->base, f->theta, f->m, f->v, l.total, f->grad, l.grad_total(), f->loss, f->n_chunks,
+                     f->step);
     if (f->ctx->stage_failed) HIP_TRY(hipStreamSynchronize(st));  // idx and lower are locals
     if (o->steps > f->hist_cap) {
         if (f->hist) {
@@ -2370,29 +2366,20 @@ int prh_fit_run(prh_fit* f, const prh_diff_params* start, const prh_fit_options*
     launch_diff_list_views(st, f->d_views, (int32_t)f->views.size(), f->total_strips, f->chunks, f->n_chunks);
     HIP_TRY(hipGetLastError());
     const AdamConsts a{o->lr, o->beta1, o->beta2, o->eps, n_idx, f->hist_cap, l.reps, (int32_t)l.kd, (int32_t)l.tail()};
-    // one step: the adjoint over every view, Adam; captured once, replayed
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    if (o->steps > 0) {
-        HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
+    // one step: the adjoint over every view, Adam.  Two plain launches, queued
+    // faster than any step runs: a graph of the step, instantiated for each
+    // call and launched per step, took 6 us a step more (1195 us against 1060
+    // for 20 steps of six small views, 1335 against 1260 for 10 of four)
+    hipError_t e = hipEventRecord(f->ev[0], st);
+    for (int32_t k = 0; k < o->steps && e == hipSuccess; k++) {
         launch_adjoint_views(st, f->sc->d, f->d_views, f->max_chunks, f->chunks, f->n_chunks,
                              (o->groups & PRH_FIT_ALBEDO) != 0, f->step);
         launch_adam(st, f->par, f->grad, f->base, f->theta, f->m, f->v, f->idx, f->lower, a, f->step, f->loss,
                     f->hist);
-        const hipError_t e = hipStreamEndCapture(st, &g);
-        if (e != hipSuccess) return fail(PRH_E_HIP, std::string("prh_fit_run capture: ") + hipGetErrorString(e));
-        const hipError_t e2 = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-        if (e2 != hipSuccess) {
-            (void)hipGraphDestroy(g);
-            return fail(PRH_E_HIP, std::string("prh_fit_run instantiate: ") + hipGetErrorString(e2));
-        }
+        e = hipGetLastError();
     }
-    hipError_t e = hipEventRecord(f->ev[0], st);
-    for (int32_t k = 0; k < o->steps && e == hipSuccess; k++) e = hipGraphLaunch(ge, st);
     if (e == hipSuccess) e = hipEventRecord(f->ev[1], st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (ge) (void)hipGraphExecDestroy(ge);
-    if (g) (void)hipGraphDestroy(g);
     if (e != hipSuccess) return fail(PRH_E_HIP, std::string("prh_fit_run: ") + hipGetErrorString(e));
     f->stats.steps = o->steps;
     (void)hipEventElapsedTime(&f->stats.ms_steps, f->ev[0], f->ev[1]);
