@@ -436,9 +436,12 @@ __device__ __forceinline__ void draw_small_tris(bool mine, V4 p1, V4 p2, V4 p3, 
 // A larger primitive is handed to the raster pass as jobs: rectangles of at
 // most `side` pixels a side of its pixel box, each a record of its own (the
 // vertices, the order key or the map, the rectangle) in one of RASTER_QUEUES
-// queues, the workgroup's, at a place its wave takes with one atomic.  The
-// wave's jobs are spread over its lanes, so a triangle that covers the screen
-// costs its wave a few rounds.  (They were counted into 16x16 tiles, scanned,
+// queues, at places its wave takes with one atomic.  The wave's jobs are spread
+// over its lanes, so a triangle that covers the screen costs its wave a few
+// rounds, and each round's sixty-four over the queues, so that all the raster's
+// waves draw it (in the workgroup's one queue they were a sixteenth of the
+// waves' work: k_raster 56 us of a 1600x1200 frame with a large ground quad, 17
+// over the queues).  (They were counted into 16x16 tiles, scanned,
 // listed by tile and rasterised tile by tile: two triangles covering 1600x1200
 // held their wave's lane for 1.4 ms, and a frame of small ones paid 15-25 us
 // for the three passes.)
@@ -450,16 +453,22 @@ __device__ __forceinline__ void emit_jobs(bool mine, V4 p1, V4 p2, V4 p3, uint32
     const int nx = mine ? (x1 - x0 + side) >> shift : 0, c = mine ? nx * ((y1 - y0 + side) >> shift) : 0;
     const int lane = threadIdx.x & 63;
     const int total = __builtin_amdgcn_readlane(wave_scan_incl<false>(c), 63);
-    const int qi = block & (RASTER_QUEUES - 1);
-    int base = 0;
-    if (lane == 0) base = atomicAdd(&q.n[qi * JOB_COUNT_STRIDE], total);
-    base = __builtin_amdgcn_readfirstlane(base);
-    if (base + total > q.cap) {  // the host grows the queues and draws the frame again
-        if (lane == 0) atomicMax(&cnt->need_jobs, base + total), atomicOr(&cnt->overflow, 1);
+    // the wave's jobs in sixty-fours, one to a queue from the workgroup's on:
+    // lane k takes queue k's places, all with one atomic
+    const int qi = block & (RASTER_QUEUES - 1), rel = (lane - qi) & (RASTER_QUEUES - 1);
+    const int rounds = (total + 63) >> 6;
+    int mineq = 0, base = 0;
+    if (lane < RASTER_QUEUES && rel < rounds) {
+        mineq = 64 * ((rounds - rel + RASTER_QUEUES - 1) / RASTER_QUEUES);
+        if (((rounds - 1 - rel) & (RASTER_QUEUES - 1)) == 0) mineq -= 64 * rounds - total;  // (the last, in part)
+        base = atomicAdd(&q.n[lane * JOB_COUNT_STRIDE], mineq);
+    }
+    const bool full = base + mineq > q.cap;
+    if (__ballot(full) != 0) {  // the host grows the queues and draws the frame again
+        if (full) atomicMax(&cnt->need_jobs, base + mineq), atomicOr(&cnt->overflow, 1);
         return;
     }
-    Prim* out = q.jobs + (size_t)qi * q.cap + base;
-    int done = 0;
+    int round = 0;
     wave_spread(c, wmark, [&](int o, int l, bool valid) {
         Prim j;
         j.p0 = make_float4(__shfl(p1.x, o), __shfl(p1.y, o), __shfl(p1.z, o), __shfl(p2.x, o));
@@ -468,14 +477,16 @@ __device__ __forceinline__ void emit_jobs(bool mine, V4 p1, V4 p2, V4 p3, uint32
                   oy1 = __shfl(y1, o);
         const float cz = __shfl(p3.z, o);
         const uint32_t okey = (uint32_t)__shfl((int)key, o);
+        const int to = (qi + round) & (RASTER_QUEUES - 1);
+        Prim* out = q.jobs + (size_t)to * q.cap + __builtin_amdgcn_readlane(base, to) + 64 * (round / RASTER_QUEUES);
         if (valid) {
             const int jy = l / onx, jx = l - jy * onx;
             const int ax = ox0 + (jx << shift), ay = oy0 + (jy << shift);
             j.p2 = make_float4(cz, bitsf(okey), bitsf(pack_bbox(ax, ay)),
                                bitsf(pack_bbox(min(ax + side - 1, ox1), min(ay + side - 1, oy1))));
-            out[done + lane] = j;
+            out[lane] = j;
         }
-        done += 64;
+        round++;
     });
 }
 // The raster tiles a pixel box touches (the frame statistics' pairs).
