@@ -2426,10 +2426,19 @@ __global__ __launch_bounds__(256) void k_push(PushArgs a) {
 static inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // ------------------------------------------------------------- resize
-// resizeRGBA (internal/imageutil/resize.go:76-118), one output pixel per
-// thread: out[y][x] filters row x of `in` (rows of in_w RGBA8 pixels) at
-// output position y with createWeights8's 8-bit weights.  Two launches make
-// imageutil.Resize: the first writes its result transposed.
+// resizeRGBA (internal/imageutil/resize.go:76-118): out[y][x] filters row x of
+// `in` (rows of in_w RGBA8 pixels) at output position y with createWeights8's
+// 8-bit weights.  Two launches make imageutil.Resize: the first writes its
+// result transposed.
+// TILE: a workgroup makes 64 positions of 32 rows, a lane a position, so a
+// row's taps are read along it, eight rows at once; the tile turns in LDS, so
+// the output is written along its rows as well.  (A thread an output pixel
+// reads 64 rows a load: the two passes of a 1600x1200 frame to 800x600 took 23
+// and 13 us, now 8.5 and 6.)  Few outputs, or a long filter (a texture's
+// pyramid), leave too few tiles and keep the thread a pixel: 65536 outputs of
+// 4 taps take 4 us against 6, the pyramids of two textures 680 us against 1030
+// with tiles alone.
+constexpr int RESIZE_ROWS = 32, RESIZE_TILE_TAPS = 8, RESIZE_TILE_OUTPUTS = 1 << 17;
 struct k_resize_args {
     const uint32_t* in;
     int32_t in_w;
@@ -2442,6 +2451,7 @@ struct k_resize_args {
     Stamp stamp;
     int32_t gx, gy;  // the grid of this launch
 };
+template <bool TILE>
 __device__ __forceinline__ void k_resize_body(const k_resize_args& a_, const VB vb) {
     const uint32_t* __restrict__ in = a_.in;
     const int32_t in_w = a_.in_w;
@@ -2452,38 +2462,89 @@ __device__ __forceinline__ void k_resize_body(const k_resize_args& a_, const VB 
     const int32_t* __restrict__ start = a_.start;
     const int32_t fl = a_.fl;
 
-    const int x = vb.bx * blockDim.x + threadIdx.x, y = vb.by;
-    if (x >= out_w || y >= out_rows) return;
-    const uint32_t* row = in + (size_t)x * in_w;
-    const int maxX = in_w - 1;
-    int32_t acc[4] = {0, 0, 0, 0}, sum = 0;
+    if (!TILE) {
+        const int x = vb.bx * blockDim.x + threadIdx.x, y = vb.by;
+        if (x < out_w && y < out_rows) {
+            const uint32_t* row = in + (size_t)x * in_w;
+            const int maxX = in_w - 1;
+            int32_t acc[4] = {0, 0, 0, 0}, sum = 0;
+            for (int i = 0; i < fl; i++) {
+                const int32_t coeff = coeffs[y * fl + i];
+                if (coeff == 0) continue;
+                int xi = start[y] + i;
+                xi = (unsigned)xi < (unsigned)maxX ? xi : (xi >= maxX ? maxX : 0);
+                const uint32_t p = row[xi];
+                for (int k = 0; k < 4; k++) acc[k] += coeff * (int32_t)((p >> (8 * k)) & 0xffu);
+                sum += coeff;
+            }
+            uint32_t o = 0;
+            for (int k = 0; k < 4; k++) {
+                const int v = acc[k] / sum;  // truncating division, as Go's
+                o |= (uint32_t)(v < 0 ? 0 : (v > 255 ? 255 : v)) << (8 * k);
+            }
+            out[(size_t)y * out_w + x] = o;
+        }
+        return stamp_end(a_.stamp, vb);
+    }
+    __shared__ uint32_t s_out[64][RESIZE_ROWS + 1];
+    constexpr int PER = RESIZE_ROWS / 4;  // a wave's rows
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int x0 = vb.bx * RESIZE_ROWS, y0 = vb.by * 64, y = min(y0 + lane, out_rows - 1);
+    const int maxX = in_w - 1, from = start[y];
+    const uint32_t* row = in + (size_t)x0 * in_w;
+    int32_t acc[PER][4] = {}, sum = 0;
     for (int i = 0; i < fl; i++) {
         const int32_t coeff = coeffs[y * fl + i];
-        if (coeff == 0) continue;
-        int xi = start[y] + i;
+        int xi = from + i;
         xi = (unsigned)xi < (unsigned)maxX ? xi : (xi >= maxX ? maxX : 0);
-        const uint32_t p = row[xi];
-        for (int k = 0; k < 4; k++) acc[k] += coeff * (int32_t)((p >> (8 * k)) & 0xffu);
+        uint32_t p[PER];
+#pragma unroll
+        for (int r = 0; r < PER; r++) p[r] = row[(size_t)min(PER * wv + r, out_w - 1 - x0) * in_w + xi];
+#pragma unroll
+        for (int r = 0; r < PER; r++)
+            for (int k = 0; k < 4; k++) acc[r][k] += mul_i24(coeff, (int32_t)((p[r] >> (8 * k)) & 0xffu));
         sum += coeff;
     }
-    uint32_t o = 0;
-    for (int k = 0; k < 4; k++) {
-        const int v = acc[k] / sum;  // truncating division, as Go's
-        o |= (uint32_t)(v < 0 ? 0 : (v > 255 ? 255 : v)) << (8 * k);
+    // truncating division by the position's sum, as Go's: below 2^24 by the
+    // float reciprocal, put right by its remainder
+    const bool small = sum > 0 && sum < (1 << 16);
+    const float inv = __builtin_amdgcn_rcpf((float)sum);
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        uint32_t o = 0;
+        for (int k = 0; k < 4; k++) {
+            const int a = acc[r][k];
+            int v;
+            if (small) {  // (0 <= a <= 255 sum)
+                v = (int)((float)a * inv);
+                const int rem = a - v * sum;
+                v += rem >= sum ? 1 : (rem < 0 ? -1 : 0);
+            } else {
+                v = a / sum;
+            }
+            o |= (uint32_t)(v < 0 ? 0 : (v > 255 ? 255 : v)) << (8 * k);
+        }
+        s_out[lane][PER * wv + r] = o;
     }
-    out[(size_t)y * out_w + x] = o;
+    __syncthreads();
+    for (int t = threadIdx.x; t < 64 * RESIZE_ROWS; t += 256) {
+        const int ty = t / RESIZE_ROWS, tx = t % RESIZE_ROWS;
+        if (y0 + ty < out_rows && x0 + tx < out_w) out[(size_t)(y0 + ty) * out_w + x0 + tx] = s_out[ty][tx];
+    }
     stamp_end(a_.stamp, vb);
 }
+template <bool TILE>
 __global__ __launch_bounds__(256) void k_resize(k_resize_args a) {
-    k_resize_body(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
+    k_resize_body<TILE>(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
 }
+template <bool TILE>
 __global__ __launch_bounds__(256) void k_resize_wide(const k_resize_args* __restrict__ a, const int32_t* __restrict__ start,
         int32_t n) {
     const int v = wide_view(start, n, (int)blockIdx.x);
     const k_resize_args& x = a[v];
     const int local = (int)blockIdx.x - start[v];
     if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_resize_body(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
+    k_resize_body<TILE>(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
 }
 
 // ------------------------------------------------------------- wide launches
@@ -2708,8 +2769,13 @@ void launch_shadow_count(hipStream_t st, const DevScene& s, const ShadeConsts& c
 void launch_resize(hipStream_t st, const uint32_t* in, int32_t in_w, uint32_t* out, int32_t out_w, int32_t out_rows,
                    const int16_t* coeffs, const int32_t* start, int32_t fl, Stamp stamp) {
     if (out_w <= 0 || out_rows <= 0) return;
-    go(k_resize, k_resize_wide, dim3(blocks_for(out_w, 256), out_rows), 256, st,
-       k_resize_args{in, in_w, out, out_w, out_rows, coeffs, start, fl, stamp, 0, 0});
+    const k_resize_args a{in, in_w, out, out_w, out_rows, coeffs, start, fl, stamp, 0, 0};
+    if (fl <= RESIZE_TILE_TAPS && (int64_t)out_w * out_rows >= RESIZE_TILE_OUTPUTS)
+        go(k_resize<true>, k_resize_wide<true>, dim3(blocks_for(out_w, RESIZE_ROWS), blocks_for(out_rows, 64)), 256, st, a);
+    else {
+        if (g_wide) g_wide->sub = 1;  // (beside the views' tiles in a recorded batch)
+        go(k_resize<false>, k_resize_wide<false>, dim3(blocks_for(out_w, 256), out_rows), 256, st, a);
+    }
 }
 
 }  // namespace prh
