@@ -69,16 +69,31 @@ __device__ bool pixel_box(float ax, float ay, float az, float bx, float by, floa
     float mnx = gmin3(ax, bx, cx), mny = gmin3(ay, by, cy);
     float mxx = gmax3(ax, bx, cx), mxy = gmax3(ay, by, cy);
     (void)az, (void)bz, (void)cz;
-    int64_t xmin = f2i(round32(mnx) - 1), xmax = f2i(round32(mxx) + 1);
-    int64_t ymin = f2i(round32(mny) - 1), ymax = f2i(round32(mxy) + 1);
     const float wmax = fmaxf(mxx - mnx, mxy - mny);
+    bool narrow = false;
     if (wmax <= 64.0f && wmax >= 0x1p-20f) {  // false for NaN / Inf
         const float sabc = tri_setup(ax, ay, bx, by, cx, cy).sabc;
-        if (fabsf(sabc) >= 0.25f * wmax * wmax) {
+        narrow = fabsf(sabc) >= 0.25f * wmax * wmax;
+    }
+    // Go's int is 64 bits wide; within 2^30 (every lane, mostly) 32 hold the
+    // same values at a third of the instructions: k_setup_shadow 47.4 -> 39.4 M
+    // of them with 1.04 M triangles into five 2048x2048 maps, 77 -> 70 us
+    if ((fabsf(mnx) < 0x1p30f) & (fabsf(mxx) < 0x1p30f) & (fabsf(mny) < 0x1p30f) & (fabsf(mxy) < 0x1p30f)) {
+        int xmin = (int)(round32(mnx) - 1), xmax = (int)(round32(mxx) + 1);
+        int ymin = (int)(round32(mny) - 1), ymax = (int)(round32(mxy) + 1);
+        if (narrow) {
             // centres x + 0.5 in [min - 0.24, max + 0.24]
-            xmin = max(xmin, (int64_t)ceilf(mnx - 0.74f)), xmax = min(xmax, (int64_t)floorf(mxx - 0.26f));
-            ymin = max(ymin, (int64_t)ceilf(mny - 0.74f)), ymax = min(ymax, (int64_t)floorf(mxy - 0.26f));
+            xmin = max(xmin, (int)ceilf(mnx - 0.74f)), xmax = min(xmax, (int)floorf(mxx - 0.26f));
+            ymin = max(ymin, (int)ceilf(mny - 0.74f)), ymax = min(ymax, (int)floorf(mxy - 0.26f));
         }
+        x0 = max(xmin, 0), y0 = max(ymin, 0), x1 = min(xmax, W - 1), y1 = min(ymax, H - 1);
+        return x0 <= x1 && y0 <= y1;
+    }
+    int64_t xmin = f2i(round32(mnx) - 1), xmax = f2i(round32(mxx) + 1);
+    int64_t ymin = f2i(round32(mny) - 1), ymax = f2i(round32(mxy) + 1);
+    if (narrow) {
+        xmin = max(xmin, (int64_t)ceilf(mnx - 0.74f)), xmax = min(xmax, (int64_t)floorf(mxx - 0.26f));
+        ymin = max(ymin, (int64_t)ceilf(mny - 0.74f)), ymax = min(ymax, (int64_t)floorf(mxy - 0.26f));
     }
     if (xmin < 0) xmin = 0;
     if (ymin < 0) ymin = 0;

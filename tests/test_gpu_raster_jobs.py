@@ -107,3 +107,25 @@ def test_exact_order_pass_outgrows_the_queues(device, orc):
     render.render_batch([r])
     _same(r, fr)
     r.free()
+
+
+@pytest.mark.parametrize("far", [1e4, 3e8, 3e9, 1e12, 1e30])
+def test_boxes_past_32_bits(device, orc, far):
+    """Triangles whose screen coordinates in the view and in the shadow maps
+    lie within and beyond what 32-bit pixel boxes hold."""
+    s = cases.shadow_footprint()
+    for m in s.meshes:
+        p = m.pos[:, :2]
+        p[np.abs(p) >= np.abs(p).max() * 0.99] *= np.float32(far)  # the ground's corners
+    fr = orc.render(s)
+    r = render.renderer_for(s, device)
+    try:
+        r.render_device()
+    except abi.PrhError as e:  # (areas that overflow: a NaN depth in a shadow pass is refused)
+        assert e.code == abi.PRH_E_UNSUPPORTED and far in (3e9, 1e12)
+        r.free()
+        return
+    _same(r, fr)
+    got = r.read(abi.PRH_BUF_SHADOW).reshape(-1)
+    assert np.array_equal(got.view(np.uint32), fr.shadow_maps[: got.size].view(np.uint32))
+    r.free()
