@@ -121,7 +121,7 @@ PASSES = ("total", "shadow", "vertex", "setup", "raster", "ao", "shade")
 
 def run_frames(r, steps: int):
     """`steps` synchronous frames timed by the wall clock, then `steps` more
-    whose per-pass times are read from each frame's own HIP events (reading
+    whose per-pass times are read from each frame's own clock stamps (reading
     them is host work the timed frames leave out): (wall seconds, mean
     per-pass ms)."""
     t0 = time.perf_counter()
@@ -140,7 +140,7 @@ def run_frames(r, steps: int):
 def adjoint_bench(dev, steps: int) -> dict:
     """Forward + adjoint against a plain single view: the 512x512 ~100k-
     triangle 4-light scene, target rendered from seed parameters, gradients
-    at a 10 % Gaussian perturbation.  Device times from HIP events: one
+    at a 10 % Gaussian perturbation.  Device times from the frames' clock stamps and HIP events: one
     frame (prh_render), one adjoint launch (loss + all gradients)."""
     from polyred_amd import diff, render, scenes
 
@@ -405,7 +405,7 @@ def main() -> int:
         return out
 
     pmc_note = (f"traffic and VALU instruction counts per launch from {pmc_path} (rocprofv3 --pmc, recorded on "
-                f"commit {pmc.get('_commit', '?')}); times from this run's HIP events with every pass on one stream")
+                f"commit {pmc.get('_commit', '?')}); times from this run's clock stamps with every pass on one stream")
     # the dominant kernel: the longest of the frame's kernels run alone
     ao_roof = dict(roof("k_ao", ab, ms1["ao"]), standalone=True, source=pmc_note)
     shade_roof = dict(roof("k_shade", sb["bytes"], ms1["shade"]), standalone=True, covered_px=sb["covered"],

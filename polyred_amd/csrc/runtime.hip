@@ -486,6 +486,7 @@ struct prh_renderer {
     prh_tuning tune;       // speed knobs (results do not depend on them)
     bool split_shade_last;  // the last frame split its shading
     int raster_end_last;    // the stamp its raster pass ends at
+    bool bg_last;           // k_shade_bg ran
     // the last frame's per-pass times wait in its stamps until the stats are
     // read (prh_last_stats): a frame's own host work stays short
     bool times_pending, times_nan_rerun;
@@ -1398,7 +1399,7 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     const bool bg_inline = !r->sc->any_ao && !wide && P <= BG_INLINE_PIXELS;
     // (the pass ends with the resolve, else where k_shade_bg starts, else with
     // the raster: of its unequal workgroups a stamp sees a few)
-    r->raster_end_last = resolve || bg_inline ? ST_RESOLVED : ST_BG;
+    r->raster_end_last = resolve || bg_inline ? ST_RESOLVED : ST_BG, r->bg_last = !bg_inline;
     launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt, at(-1, !resolve && bg_inline ? ST_RESOLVED : -1));
     wide_stage(12);
     if (resolve)
@@ -2088,7 +2089,8 @@ int fill_times(prh_renderer* r) {
     S.ms_raster = ms(setup_end, raster_end);
     S.ms_ao = ao ? ms(raster_end, t[ST_BG]) : 0.0f;
     // (split shading: the first half beside the AO, and the second)
-    const unsigned long long ready = std::max(ao ? t[ST_BG] : raster_end, shadow_end);
+    // (the uncovered colour of its own kernel in none of them)
+    const unsigned long long ready = std::max(r->bg_last ? t[ST_BG_END] : raster_end, shadow_end);
     S.ms_shade = r->split_shade_last ? ms(std::max(raster_end, shadow_end), t[ST_SHADE_END]) +
                                            ms(std::max(t[ST_SHADE_END], t[ST_BG_END]), t[ST_END])
                                      : ms(ready, t[ST_END]);
