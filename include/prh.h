@@ -231,7 +231,7 @@ typedef struct prh_frame_stats {
                             plus the clipper's pieces                       */
     int32_t n_clipped;   /* triangles that went through the clipper         */
     int32_t n_bin_pairs; /* (primitive, raster tile) pairs of the primitives
-                            the setup does not draw itself                  */
+                            of more than main_direct_max pixel centres      */
     int32_t nan_rerun;   /* 1 if the NaN-depth exact-order pass ran         */
     float ms_diff;       /* the last prh_diff_forward / _backward kernel    */
 } prh_frame_stats;
@@ -376,7 +376,8 @@ typedef struct prh_tuning {
                                   the raster has no per-tile lists whose capacity it was                   */
     int32_t shadow_direct_max; /* shadow-map triangles of at most this many texel centres are drawn by
                                   the setup, 0..256; default 64                                            */
-    int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise; 48  */
+    int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise; 48
+                                  (left there, 16 in a frame of its own of at most 2^19 triangles)        */
     int32_t overlap_shadows;   /* 1: a frame's shadow passes run on a second stream beside the main
                                   view's passes; default 1 from 2^19 framebuffer pixels, else 0          */
     int32_t raster_tile;       /* side of the raster tiles (main view and shadow maps): 8, 16 or 32

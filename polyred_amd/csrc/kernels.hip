@@ -528,6 +528,7 @@ struct k_setup_main_args {
     Capacities cap;
     unsigned long long* vis;
     int32_t draw_small;
+    int32_t count_small;  // the statistics' pairs are of primitives of more pixel centres
     const int4* tri_rec;
     int32_t gx, gy;  // the grid of this launch
 };
@@ -599,8 +600,9 @@ __device__ __forceinline__ void k_setup_main_body(const k_setup_main_args& a_, c
     __shared__ int32_t s_pairs;
     if (threadIdx.x == 0) s_pairs = 0;
     const int nd = __syncthreads_count(direct);
-    const int nb = __syncthreads_count(big);
-    if (nb && big) atomicAdd(&s_pairs, box_tiles(x0, y0, x1, y1, vc.rt_shift));
+    const bool counted = direct && (x1 - x0 + 1) * (y1 - y0 + 1) > a_.count_small;
+    const int nb = __syncthreads_count(counted);
+    if (nb && counted) atomicAdd(&s_pairs, box_tiles(x0, y0, x1, y1, vc.rt_shift));
     if (nb) __syncthreads();
     if (threadIdx.x == 0) {
         blk_prims[vb.bx] = nd;
@@ -2699,11 +2701,13 @@ int clip_grid(const Capacities& cap) { return (int)std::min<size_t>(blocks_for(c
 void launch_setup_main(hipStream_t st, const DevScene& s, const ViewConsts& vc, const float4* tv_scr,
                        const float4* tv_nor, const JobQueues& jobs, ClipRec* clips, int32_t* tri_clip_slot,
                        ClipJob* clip_list, int32_t* blk_prims, int32_t* blk_pairs, Counters* cnt, Capacities cap,
-                       unsigned long long* vis, int32_t draw_small, const int4* tri_rec, Stamp stamp) {
+                       unsigned long long* vis, int32_t draw_small, int32_t count_small, const int4* tri_rec,
+                       Stamp stamp) {
     if (!s.n_tris) return;
     const int nb = setup_blocks(s.n_tris);
     go(k_setup_main, k_setup_main_wide, dim3(nb), 256, st,
-       k_setup_main_args{s, vc, tv_scr, clip_list, jobs, blk_prims, blk_pairs, cnt, cap, vis, draw_small, tri_rec,
+       k_setup_main_args{s, vc, tv_scr, clip_list, jobs, blk_prims, blk_pairs, cnt, cap, vis, draw_small,
+                         count_small, tri_rec,
                          0, 0});
     go(k_clip, k_clip_wide, dim3(clip_grid(cap)), CLIP_WAVES * 64, st,
        k_clip_args{s, vc, tv_scr, tv_nor, clip_list, jobs, clips, tri_clip_slot, blk_prims + nb,

@@ -218,7 +218,8 @@ int clip_grid(const Capacities& cap);
 void launch_setup_main(hipStream_t st, const DevScene& s, const ViewConsts& vc, const float4* tv_scr,
                        const float4* tv_nor, const JobQueues& jobs, ClipRec* clips, int32_t* tri_clip_slot,
                        ClipJob* clip_list, int32_t* blk_prims, int32_t* blk_pairs, Counters* cnt, Capacities cap,
-                       unsigned long long* vis, int32_t draw_small, const int4* tri_rec, Stamp stamp);
+                       unsigned long long* vis, int32_t draw_small, int32_t count_small, const int4* tri_rec,
+                       Stamp stamp);
 void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& sc, const int4* tri_rec,
                          const float3* ts, const JobQueues& jobs, Counters* cnt, uint32_t* smaps);
 // Each global triangle's record, fixed by the scene: its transformed

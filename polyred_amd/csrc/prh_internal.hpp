@@ -157,6 +157,7 @@ struct Capacities {
 };
 
 constexpr int ITEM_PRIMS = 2048;    // prh_tuning.item_prims' default
+constexpr int MAIN_DIRECT_MAX = 48; // and main_direct_max'
 
 // Where a raster pass writes.
 struct RasterTarget {

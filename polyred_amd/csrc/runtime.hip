@@ -362,6 +362,13 @@ enum {
 // and 1001x701 no difference (436 and 220 us either way), nor with AO at
 // 480x270.
 constexpr size_t BG_INLINE_PIXELS = 1 << 17;
+// The main view's triangles of at most so many pixel centres are drawn by the
+// setup (prh_tuning.main_direct_max); 16 in a frame of its own of at most 2^19
+// triangles (2048 workgroups, 8 a CU) with the knob at its default.  48 -> 16:
+// 480x270 of 197 k triangles 148 -> 138 us on the device and back, 1001x701 of
+// 310 k 147 -> 134, 512x512 of 104 k 69 -> 64; 1.04 M triangles 414 -> 422 and
+// a 64-view batch 2254 -> 2457, which are bound by the work and keep 48.
+constexpr int32_t MAIN_DIRECT_FEW = 16, LATENCY_TRIS = 1 << 19;
 
 struct prh_renderer;
 // prh_render_batch spreads a batch over one stream per hardware queue the
@@ -1054,7 +1061,7 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     HIP_TRY(hipSetDevice(ctx->device));
     prh_renderer* r = new prh_renderer();
     r->ctx = ctx, r->sc = s, r->cam = *cam, r->opt = *o;
-    r->tune = prh_tuning{8, ITEM_PRIMS, 64, 48, (size_t)o->width * o->height * msaa * msaa >= (1u << 19) ? 1 : 0,
+    r->tune = prh_tuning{8, ITEM_PRIMS, 64, MAIN_DIRECT_MAX, (size_t)o->width * o->height * msaa * msaa >= (1u << 19) ? 1 : 0,
                          TILE, 0.0f};
     // every pass renders the MSAA-sized buffer (render/raster.go:149-150)
     r->msaa = msaa, r->OW = o->width, r->OH = o->height;
@@ -1380,11 +1387,15 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
                        FrameClear{(uint32_t*)cm, (shadows ? 1 : 2) * CNT_WORDS, (uint64_t*)r->vis, P},
                        at(ST_VERTEX, ST_VERTEX_END));
     wide_stage(8);
+    // a frame whose setup fits the chip at once waits for the setup's longest
+    // wave: left at its default, the knob hands the raster more of them there
+    const int32_t draw_small = r->tune.main_direct_max == MAIN_DIRECT_MAX && !wide && d.n_tris <= LATENCY_TRIS
+                                   ? MAIN_DIRECT_FEW : r->tune.main_direct_max;
     // (the exact-order pass keeps the frame's statistics: it draws nothing in
     // the setup, so its raster takes other primitives)
     launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->jobs, r->clips, r->tri_clip_slot, r->clip_list,
                       r->blk_prims, nan_mode ? nullptr : r->blk_pairs, cm, r->cap_main, (unsigned long long*)r->vis,
-                      nan_mode ? 0 : r->tune.main_direct_max, r->tri_rec, at(-1, ST_SETUP_END));
+                      nan_mode ? 0 : draw_small, r->tune.main_direct_max, r->tri_rec, at(-1, ST_SETUP_END));
     if (nan_mode) {
         launch_fill_u32(st, r->first_all, P, 0xffffffffu);
         launch_fill_u32(st, r->first_nan, P, 0xffffffffu);

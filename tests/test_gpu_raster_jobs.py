@@ -129,3 +129,22 @@ def test_boxes_past_32_bits(device, orc, far):
     got = r.read(abi.PRH_BUF_SHADOW).reshape(-1)
     assert np.array_equal(got.view(np.uint32), fr.shadow_maps[: got.size].view(np.uint32))
     r.free()
+
+
+@pytest.mark.parametrize("knob", [0, 15, 16, 47, 48, 49, 256])
+def test_threshold_by_frame_size(device, orc, knob):
+    """The setup's threshold in a small frame (16 with the knob at its default,
+    else the knob's) and in a batch: the same frame, and the same statistics,
+    which go by the knob."""
+    s = scenes.c2_scale(seed=3, width=200, height=150, n_spheres=20, grid=6, shadow_size=64, ao=False)
+    fr = orc.render(s)
+    r = render.renderer_for(s, device)
+    r.set_tuning(main_direct_max=knob)
+    r.render_device()
+    _same(r, fr)
+    a = r.stats()
+    render.render_batch([r])
+    _same(r, fr)
+    b = r.stats()
+    assert (a.n_prims, a.n_bin_pairs, a.n_clipped) == (b.n_prims, b.n_bin_pairs, b.n_clipped)
+    r.free()
