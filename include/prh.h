@@ -379,7 +379,9 @@ typedef struct prh_tuning {
     int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise; 48
                                   (left there, 16 in a frame of its own of at most 2^19 triangles)        */
     int32_t overlap_shadows;   /* 1: a frame's shadow passes run on a second stream beside the main
-                                  view's passes; default 1 from 2^19 framebuffer pixels, else 0          */
+                                  view's passes; default 1 from 2^19 framebuffer pixels, else 0 (from
+                                  there on only where it pays: more than 2^19 triangles, or AO and at
+                                  least 2^22 pixels)                                                      */
     int32_t raster_tile;       /* side of the raster tiles (main view and shadow maps): 8, 16 or 32
                                   pixels, a raster job being at most 2 x 2 of them; default 16            */
     float ms;                  /* prh_autotune: the chosen configuration's median frame time             */

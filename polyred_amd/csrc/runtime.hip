@@ -369,6 +369,15 @@ constexpr size_t BG_INLINE_PIXELS = 1 << 17;
 // 310 k 147 -> 134, 512x512 of 104 k 69 -> 64; 1.04 M triangles 414 -> 422 and
 // a 64-view batch 2254 -> 2457, which are bound by the work and keep 48.
 constexpr int32_t MAIN_DIRECT_FEW = 16, LATENCY_TRIS = 1 << 19;
+// prh_tuning.overlap_shadows is 1 from so many pixels.  A frame that has it so
+// by default still takes one stream with at most LATENCY_TRIS triangles, whose
+// setups leave the chip room and whose fork and joins cost more than they
+// hide: 1001x701 of 310 k triangles 131 -> 122 us on the device and back,
+// 1600x900 146 -> 135, 3840x2160 314 -> 302, a textured 1600x1200 one 235 ->
+// 224; 1.04 M triangles 1001x701 195 against 200 on one stream, 1920x1080 with
+// AO 400 against 417.  With AO and 2^22 pixels the AO beside the shading is
+// worth the fork (3840x2160 of 116 k triangles 602 against 614).
+constexpr size_t OVERLAP_PIXELS = 1 << 19, OVERLAP_AO_PIXELS = 1 << 22;
 
 struct prh_renderer;
 // prh_render_batch spreads a batch over one stream per hardware queue the
@@ -1061,7 +1070,7 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     HIP_TRY(hipSetDevice(ctx->device));
     prh_renderer* r = new prh_renderer();
     r->ctx = ctx, r->sc = s, r->cam = *cam, r->opt = *o;
-    r->tune = prh_tuning{8, ITEM_PRIMS, 64, MAIN_DIRECT_MAX, (size_t)o->width * o->height * msaa * msaa >= (1u << 19) ? 1 : 0,
+    r->tune = prh_tuning{8, ITEM_PRIMS, 64, MAIN_DIRECT_MAX, (size_t)o->width * o->height * msaa * msaa >= OVERLAP_PIXELS ? 1 : 0,
                          TILE, 0.0f};
     // every pass renders the MSAA-sized buffer (render/raster.go:149-150)
     r->msaa = msaa, r->OW = o->width, r->OH = o->height;
@@ -1360,7 +1369,9 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     // a plain frame runs its shadow passes on the context's second stream,
     // beside the main view's passes (they meet at the shading); a batch
     // keeps them on its own stream
-    const bool split = shadows && !wide && st == r->ctx->stream && r->tune.overlap_shadows;
+    // (a knob at its default for the frame's size: only where it pays)
+    const bool pays = P < OVERLAP_PIXELS || d.n_tris > LATENCY_TRIS || (r->sc->any_ao && P >= OVERLAP_AO_PIXELS);
+    const bool split = shadows && !wide && st == r->ctx->stream && r->tune.overlap_shadows && pays;
     const hipStream_t ss = split ? r->ctx->stream2 : st;
     // with AO as well, the AO runs on the second stream (after the shadow
     // passes) beside the shading's first half (everything but the AO factor)
