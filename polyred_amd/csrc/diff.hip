@@ -525,7 +525,8 @@ __device__ __forceinline__ void diff_adjoint(const DFwd<NLMAX>& f, const DevScen
             // d(nH^s)/dnH = s Ls / nH (below 2^-100 it is taken as 0)
             const bool in = u.nH > 0x1p-100f && u.nH < 1.0f;
             const float nH = in ? u.nH : 1.0f, z = in ? gS * I * q.Ls : 0.0f;
-            gshin = fma1(z, q.lg, gshin);
+            // (outside, the logarithm may be infinite: of 0, at a shininess of 0)
+            gshin = fma1(z, in ? q.lg : 0.0f, gshin);
             Ops<false> unused;
             const float gLs = z * shin * unused.rcp(nH);
             if (VTX) gn = fma3(gLd, u.L, fma3(gLs * q.rh, u.h, gn));
