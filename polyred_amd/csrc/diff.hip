@@ -91,11 +91,6 @@ __device__ __forceinline__ float div255(float x) {
     constexpr float hi = (float)(1.0 / 255.0), lo = (float)(1.0 / 255.0 - (double)hi);
     return fma1(x, hi, x * lo);
 }
-// a b - c d, to about an ulp of the result (Kahan): a pixel's areas cancel
-__device__ __forceinline__ float diff_of_products(float a, float b, float c, float d) {
-    const float w = c * d, e = fma1(-c, d, w);
-    return fma1(a, b, -w) + e;
-}
 // x^y and log2(x) for x in [0, 1] (x = 0: log2 is not used), within 0.57 and
 // 0.51 ulp for x in (0, 1] and y in [2^-8, 2048] (the library's powf is within
 // 1 ulp, and its logf came on top): log2 of the mantissa from the atanh
@@ -235,16 +230,16 @@ __device__ __forceinline__ DPix diff_pixel(Ops<SAFE>& op, const DTri& t, const i
     DPix p;
     p.mat = rec.w;
     p.vid[0] = rec.x, p.vid[1] = rec.y, p.vid[2] = rec.z;
-    // screen barycentrics at the pixel centre
+    // The geometry is the forward pass's, to the bit: barycentrics at the pixel
+    // centre from its rounded areas (a needle's are far below the products
+    // they are the differences of, so better ones would be other ones: 1e-4 of
+    // its colour), perspective weights, world position.
     const float4(&P)[3] = t.P;
-    const float abx = P[1].x - P[0].x, aby = P[1].y - P[0].y, acx = P[2].x - P[0].x, acy = P[2].y - P[0].y;
-    const float bcx = P[2].x - P[1].x, bcy = P[2].y - P[1].y;
-    const float apx = (float)x + 0.5f - P[0].x, apy = (float)y + 0.5f - P[0].y;
-    const float bpx = (float)x + 0.5f - P[1].x, bpy = (float)y + 0.5f - P[1].y;
-    const float sabc = diff_of_products(abx, acy, aby, acx), rs = op.rcp(sabc);
-    p.bc[2] = op.quot(diff_of_products(abx, apy, aby, apx), sabc, rs);
-    p.bc[1] = op.quot(diff_of_products(apx, acy, apy, acx), sabc, rs);
-    p.bc[0] = op.quot(diff_of_products(bcx, bpy, bcy, bpx), sabc, rs);
+    const TriSetup ts = tri_setup(P[0].x, P[0].y, P[1].x, P[1].y, P[2].x, P[2].y);
+    float area[3];
+    tri_areas(ts, (float)x + 0.5f, (float)y + 0.5f, area);
+    const float rs = op.rcp(ts.sabc);
+    for (int k = 0; k < 3; k++) p.bc[k] = op.quot(area[k], ts.sabc, rs);
     const float wc[3] = {P[0].w * p.bc[0], P[1].w * p.bc[1], P[2].w * p.bc[2]};
     const float norm = perspect ? op.rcp(wc[0] + wc[1] + wc[2]) : 1.0f;
     F3 nraw = f3(0, 0, 0);
@@ -253,7 +248,7 @@ __device__ __forceinline__ DPix diff_pixel(Ops<SAFE>& op, const DTri& t, const i
         p.w[k] = wc[k] * norm;
         p.a = fma3(p.w[k], t.A[k], p.a);
         nraw = fma3(p.bc[k], t.N[k], nraw);
-        p.x = fma3(p.bc[k], t.M[k], p.x);
+        p.x = p.x + p.bc[k] * t.M[k];
     }
     p.flat = t.flat;
     if (p.flat) {  // the face normal: fixed
