@@ -336,7 +336,10 @@ int dalloc(T** p, size_t n) {
     *p = nullptr;
     if (n == 0) n = 1;
     hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-    if (e != hipSuccess) return fail(PRH_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (reported here: not by the next call's launches)
+        return fail(PRH_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     return PRH_OK;
 }
 template <class T>
@@ -487,7 +490,8 @@ struct prh_renderer {
     unsigned long long* stamps;
     prh_frame_stats stats;
     bool has_frame;  // the visibility of a frame is in vis
-    int work_gen;    // bumped when the work buffers are reallocated
+    bool work;       // the work buffers are there (a growth that fails leaves none)
+    int work_gen;    // bumped when they are reallocated
     // differentiable shading, allocated on first use: parameters and
     // gradients in one block each (albedo, normal, kd, ks, shininess,
     // light_pos, light_int), the target, the forward output, the loss
@@ -531,18 +535,7 @@ void raster_tile(prh_renderer* r) {
     r->vc.rt_shift = r->sh.v.rt_shift = r->shc.rt_shift = shift;
 }
 
-int alloc_work(prh_renderer* r) {
-    int rc;
-    if ((rc = ralloc(r, &r->jobs.jobs, (size_t)RASTER_QUEUES * r->cap_main.jobs))) return rc;
-    if ((rc = ralloc(r, &r->clips, (size_t)r->cap_main.clip_subs))) return rc;
-    if ((rc = ralloc(r, &r->clip_list, (size_t)r->cap_main.clip_tris))) return rc;
-    r->jobs.cap = r->cap_main.jobs, r->jobs.n = r->cnt[0].jobs;
-    if (r->n_slots > 0) {
-        if ((rc = ralloc(r, &r->s_jobs.jobs, (size_t)RASTER_QUEUES * r->cap_shadow.jobs))) return rc;
-        r->s_jobs.cap = r->cap_shadow.jobs, r->s_jobs.n = r->cnt[1].jobs;
-    }
-    return PRH_OK;
-}
+// The work buffers: all of them (r->work), or none.
 void free_work(prh_renderer* r) {
     for (void* p : {(void*)r->jobs.jobs, (void*)r->clips, (void*)r->clip_list, (void*)r->s_jobs.jobs}) {
         if (!p) continue;
@@ -553,7 +546,25 @@ void free_work(prh_renderer* r) {
         }
     }
     r->jobs.jobs = nullptr, r->clips = nullptr, r->clip_list = nullptr, r->s_jobs.jobs = nullptr;
+    r->jobs.cap = r->s_jobs.cap = 0;
+    r->work = false;
 }
+int alloc_work(prh_renderer* r) {
+    int rc = ralloc(r, &r->jobs.jobs, (size_t)RASTER_QUEUES * r->cap_main.jobs);
+    if (!rc) rc = ralloc(r, &r->clips, (size_t)r->cap_main.clip_subs);
+    if (!rc) rc = ralloc(r, &r->clip_list, (size_t)r->cap_main.clip_tris);
+    if (!rc && r->n_slots > 0) rc = ralloc(r, &r->s_jobs.jobs, (size_t)RASTER_QUEUES * r->cap_shadow.jobs);
+    if (rc) {
+        free_work(r);
+        return rc;
+    }
+    r->jobs.cap = r->cap_main.jobs, r->jobs.n = r->cnt[0].jobs;
+    if (r->n_slots > 0) r->s_jobs.cap = r->cap_shadow.jobs, r->s_jobs.n = r->cnt[1].jobs;
+    r->work = true;
+    return PRH_OK;
+}
+// Before a frame is enqueued: the buffers again, after a growth that failed.
+int work_ready(prh_renderer* r) { return r->work ? PRH_OK : alloc_work(r); }
 
 }  // namespace
 
@@ -1469,22 +1480,24 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     return PRH_OK;
 }
 
-// The work capacities a frame's counters ask for; false if it had enough.
-bool grow_work(prh_renderer* r, const Counters& cm, const Counters& cs) {
-    if (!cm.overflow && !cs.overflow) return false;
+bool overflowed(const Counters& cm, const Counters& cs) { return cm.overflow || cs.overflow; }
+// Work buffers of the capacities an overflowed frame's counters ask for.  If
+// they cannot be had, the renderer is left with the capacities it had and no
+// buffers, until its next frame's work_ready.
+int regrow(prh_renderer* r, const Counters& cm, const Counters& cs) {
+    const Capacities main0 = r->cap_main, shadow0 = r->cap_shadow;
     auto up = [](int32_t& cap, int32_t need) {
-        if (need > cap) cap = need + need / 4 + 16;
+        if (need > cap) cap = (int32_t)std::min<int64_t>(INT32_MAX, (int64_t)need + need / 4 + 16);
     };
     up(r->cap_shadow.jobs, cs.need_jobs);
     up(r->cap_main.jobs, cm.need_jobs);
     up(r->cap_main.clip_tris, cm.n_clipped);
     r->cap_main.clip_subs = CLIP_PIECES * r->cap_main.clip_tris;
-    return true;
-}
-int regrow(prh_renderer* r) {
     free_work(r);
     r->work_gen++;
-    return alloc_work(r);
+    const int rc = alloc_work(r);
+    if (rc) r->cap_main = main0, r->cap_shadow = shadow0;
+    return rc;
 }
 
 // After a frame's work has completed: after an overflow, grows the work
@@ -1495,9 +1508,9 @@ int finish_frame(prh_renderer* r, int attempt, bool& again, bool timed = true) {
     again = false;
     hipStream_t st = r->ctx->stream;
     const Counters cm = r->h_cnt[0], cs = r->h_cnt[1];
-    if (grow_work(r, cm, cs)) {
+    if (overflowed(cm, cs)) {
         if (attempt >= 3) return fail(PRH_E_NOMEM, "work buffers keep overflowing");
-        int rc = regrow(r);
+        int rc = regrow(r, cm, cs);
         if (rc) return rc;
         again = true;
         return PRH_OK;
@@ -1511,9 +1524,10 @@ int finish_frame(prh_renderer* r, int attempt, bool& again, bool timed = true) {
             int rc = enqueue_frame(r, true, st, timed);
             HIP_TRY(hipStreamSynchronize(st));
             if (rc) return rc;
-            if (!grow_work(r, r->h_cnt[0], Counters{})) break;
+            const Counters cn = r->h_cnt[0];
+            if (!overflowed(cn, Counters{})) break;
             if (k >= 3) return fail(PRH_E_NOMEM, "work buffers keep overflowing");
-            if ((rc = regrow(r))) return rc;
+            if ((rc = regrow(r, cn, Counters{}))) return rc;
         }
         nan_rerun = true;
     }
@@ -1969,6 +1983,7 @@ int prh_render(prh_renderer* r) {
     r->has_frame = false;
     HIP_TRY(hipSetDevice(r->ctx->device));
     hipStream_t st = r->ctx->stream;
+    if (int rc = work_ready(r)) return rc;
     for (int attempt = 0;; attempt++) {
         const int rc0 = enqueue_frame(r, false, st, true);
         HIP_TRY(hipStreamSynchronize(st));
@@ -1993,6 +2008,8 @@ int prh_render_batch(prh_renderer* const* rs, int32_t n, int32_t flags, float* m
     const bool graph = (flags & PRH_BATCH_GRAPH) != 0;
     const bool wide = (flags & PRH_BATCH_STREAMS) == 0;
     hipStream_t s0 = ctx->bst[0];
+    for (int i = 0; i < n; i++)
+        if ((rc = work_ready(rs[i]))) return rc;
     if (graph) rc = batch_graph(ctx, rs, n, wide);
     else if (wide) rc = batch_wide(ctx, rs, n);
     if (rc) return rc;
