@@ -472,17 +472,24 @@ __device__ __forceinline__ void emit_jobs(bool mine, V4 p1, V4 p2, V4 p3, uint32
     // lane k takes queue k's places, all with one atomic
     const int qi = block & (RASTER_QUEUES - 1), rel = (lane - qi) & (RASTER_QUEUES - 1);
     const int rounds = (total + 63) >> 6;
-    int mineq = 0, base = 0;
+    int mineq = 0;
+    unsigned long long at = 0;
     if (lane < RASTER_QUEUES && rel < rounds) {
         mineq = 64 * ((rounds - rel + RASTER_QUEUES - 1) / RASTER_QUEUES);
         if (((rounds - 1 - rel) & (RASTER_QUEUES - 1)) == 0) mineq -= 64 * rounds - total;  // (the last, in part)
-        base = atomicAdd(&q.n[lane * JOB_COUNT_STRIDE], mineq);
+        at = atomicAdd(&q.n[lane * JOB_COUNT_STRIDE], (unsigned long long)mineq);
     }
-    const bool full = base + mineq > q.cap;
+    // (64 bits: a frame's jobs are counted past any capacity, and a count that
+    // wrapped would pass for a place)
+    const bool full = at + mineq > (unsigned long long)q.cap;
     if (__ballot(full) != 0) {  // the host grows the queues and draws the frame again
-        if (full) atomicMax(&cnt->need_jobs, base + mineq), atomicOr(&cnt->overflow, 1);
+        if (full) {
+            atomicMax(&cnt->need_jobs, (int32_t)min(at + mineq, 0x7fffffffull));
+            atomicOr(&cnt->overflow, 1);
+        }
         return;
     }
+    const int base = (int)at;
     int round = 0;
     wave_spread(c, wmark, [&](int o, int l, bool valid) {
         Prim j;
@@ -941,7 +948,7 @@ __device__ __forceinline__ void k_raster_body(const k_raster_args& a_, const VB 
     const int lane = threadIdx.x & 63;
     const int w0 = __builtin_amdgcn_readfirstlane(vb.bx * 4 + (threadIdx.x >> 6)), nw = vb.gx * 4;
     const int qi = w0 & (RASTER_QUEUES - 1);
-    const int n = cnt->overflow ? 0 : __builtin_amdgcn_readfirstlane(min(jq.n[qi * JOB_COUNT_STRIDE], jq.cap));
+    const int n = cnt->overflow ? 0 : __builtin_amdgcn_readfirstlane((int)min(jq.n[qi * JOB_COUNT_STRIDE], (unsigned long long)jq.cap));
     const Prim* jobs = jq.jobs + (size_t)qi * jq.cap;
     bool saw_nan = false;
     // (nw is a multiple of RASTER_QUEUES: the launches see to it)

@@ -18,7 +18,7 @@ constexpr int TILE_PX = TILE * TILE;     // 256 pixels = 4 wave64s
 // counts a cache line apart (a power of two, and a multiple of a workgroup's
 // four waves): with one counter the waves' atomics to it, 8 ns each, took as
 // long as the setup.
-constexpr int RASTER_QUEUES = 16, JOB_COUNT_STRIDE = 16;
+constexpr int RASTER_QUEUES = 16, JOB_COUNT_STRIDE = 8;
 constexpr uint32_t SUB_DIRECT = 7;       // key sub-index of an unclipped triangle
 constexpr uint64_t VIS_EMPTY = ~0ull;    // no fragment
 constexpr uint32_t KEY_HI_NAN = 0u;      // NaN-depth winner (exact-order pass only)
@@ -112,8 +112,8 @@ struct Prim {
     float4 p2;  // cz key bbox_lo bbox_hi (bit patterns)
 };
 struct JobQueues {
-    Prim* jobs;   // [RASTER_QUEUES][cap]
-    int32_t* n;   // [RASTER_QUEUES * JOB_COUNT_STRIDE], zeroed at the frame's start
+    Prim* jobs;             // [RASTER_QUEUES][cap]
+    unsigned long long* n;  // [RASTER_QUEUES * JOB_COUNT_STRIDE], zeroed at the frame's start
     int32_t cap;
 };
 
@@ -140,14 +140,14 @@ struct Counters {
     int32_t nan_flag;
     int32_t overflow;
     int32_t shadow_nan;
-    int32_t need_jobs;      // after an overflow: the most jobs one queue was asked for
+    int32_t need_jobs;      // after an overflow: the most jobs one queue was asked for (2^31 - 1: that or more)
     int32_t depth_nonfinite;  // some pixel's resolved depth is NaN or infinite
     int32_t pad[10];
 };
 // A pass's counters and its queues' job counts, zeroed together.
 struct PassCounters {
     Counters c;
-    int32_t jobs[RASTER_QUEUES * JOB_COUNT_STRIDE];
+    unsigned long long jobs[RASTER_QUEUES * JOB_COUNT_STRIDE];
 };
 
 struct Capacities {

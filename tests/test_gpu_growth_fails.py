@@ -46,3 +46,15 @@ def test_growth_past_the_memory(device, orc):
     assert np.array_equal(r.read(abi.PRH_BUF_VIS), vis)
     for x in (r, one, q):
         x.free()
+
+
+def test_counts_past_31_bits(device):
+    """2.3 million triangles of 16384 jobs: 2.36e9 a queue, past what 32-bit
+    counts tell from a place in the queue."""
+    r = render.renderer_for(_needle(2_300_000), device)
+    r.set_tuning(raster_tile=8, main_direct_max=0)
+    for draw in (r.render_device, lambda: render.render_batch([r])):
+        with pytest.raises(abi.PrhError) as e:
+            draw()
+        assert e.value.code == abi.PRH_E_NOMEM
+    r.free()
