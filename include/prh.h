@@ -376,25 +376,28 @@ typedef struct prh_tuning {
                                   the raster has no per-tile lists whose capacity it was                   */
     int32_t shadow_direct_max; /* shadow-map triangles of at most this many texel centres are drawn by
                                   the setup, 0..256; default 64                                            */
-    int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise; 48
-                                  (left there, 16 in a frame of its own of at most 2^19 triangles)        */
+    int32_t main_direct_max;   /* main-view triangles of at most this many pixel centres, likewise;
+                                  default 48 (while nobody set it, 16 in a frame of its own of at most
+                                  2^19 triangles)                                                         */
     int32_t overlap_shadows;   /* 1: a frame's shadow passes run on a second stream beside the main
-                                  view's passes; default 1 from 2^19 framebuffer pixels, else 0 (from
-                                  there on only where it pays: more than 2^19 triangles, or AO and at
-                                  least 2^22 pixels)                                                      */
+                                  view's passes; default 1 from 2^19 framebuffer pixels, else 0 (while
+                                  nobody set it, only where it pays: more than 2^19 triangles, or AO and
+                                  at least 2^22 pixels)                                                   */
     int32_t raster_tile;       /* side of the raster tiles (main view and shadow maps): 8, 16 or 32
                                   pixels, a raster job being at most 2 x 2 of them; default 16            */
     float ms;                  /* prh_autotune: the chosen configuration's median frame time             */
 } prh_tuning;
 int prh_get_tuning(prh_renderer* r, prh_tuning* out);
+/* Sets every knob but `ms`; from then on each is taken at its value. */
 int prh_set_tuning(prh_renderer* r, const prh_tuning* t);
 /* Coordinate descent over raster_wg_per_cu {1, 2, 4, 8}, shadow_direct_max {0, 16, 32, 64, 128, 256}, main_direct_max {0, 24,
  * 48, 96, 192}, overlap_shadows {0, 1} and raster_tile {8, 16, 32}: each
  * configuration timed as the median of
  * `frames` frames (HIP events, after one warm-up frame); the winner is timed
  * again against the starting knobs over twice the frames and the faster of
- * the two stays on r and goes to *out (may be NULL).  r holds a frame of it
- * on return. */
+ * the two stays on r and goes to *out (may be NULL).  A knob nobody set
+ * starts from its rule and keeps it, reported at its default, where no
+ * candidate is faster.  r holds a frame of the winner on return. */
 int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out);
 /* The same search for a batch (no counterpart in polyred): the views of a
  * prh_render_batch of wide launches, split into two size classes (class 0

@@ -156,9 +156,6 @@ struct Capacities {
     int32_t jobs;  // per raster queue
 };
 
-constexpr int ITEM_PRIMS = 2048;    // prh_tuning.item_prims' default
-constexpr int MAIN_DIRECT_MAX = 48; // and main_direct_max'
-
 // Where a raster pass writes.
 struct RasterTarget {
     int32_t W, H;

@@ -21,6 +21,7 @@
 
 #include "../../include/prh.h"
 #include "kernels.hpp"
+#include "knobs.hpp"
 
 using namespace gm;
 using namespace prh;
@@ -365,22 +366,6 @@ enum {
 // and 1001x701 no difference (436 and 220 us either way), nor with AO at
 // 480x270.
 constexpr size_t BG_INLINE_PIXELS = 1 << 17;
-// The main view's triangles of at most so many pixel centres are drawn by the
-// setup (prh_tuning.main_direct_max); 16 in a frame of its own of at most 2^19
-// triangles (2048 workgroups, 8 a CU) with the knob at its default.  48 -> 16:
-// 480x270 of 197 k triangles 148 -> 138 us on the device and back, 1001x701 of
-// 310 k 147 -> 134, 512x512 of 104 k 69 -> 64; 1.04 M triangles 414 -> 422 and
-// a 64-view batch 2254 -> 2457, which are bound by the work and keep 48.
-constexpr int32_t MAIN_DIRECT_FEW = 16, LATENCY_TRIS = 1 << 19;
-// prh_tuning.overlap_shadows is 1 from so many pixels.  A frame that has it so
-// by default still takes one stream with at most LATENCY_TRIS triangles, whose
-// setups leave the chip room and whose fork and joins cost more than they
-// hide: 1001x701 of 310 k triangles 131 -> 122 us on the device and back,
-// 1600x900 146 -> 135, 3840x2160 314 -> 302, a textured 1600x1200 one 235 ->
-// 224; 1.04 M triangles 1001x701 195 against 200 on one stream, 1920x1080 with
-// AO 400 against 417.  With AO and 2^22 pixels the AO beside the shading is
-// worth the fork (3840x2160 of 116 k triangles 602 against 614).
-constexpr size_t OVERLAP_PIXELS = 1 << 19, OVERLAP_AO_PIXELS = 1 << 22;
 
 struct prh_renderer;
 // prh_render_batch spreads a batch over one stream per hardware queue the
@@ -503,7 +488,7 @@ struct prh_renderer {
     uint32_t count_serial;
     int live_fits;  // a renderer outlives every prh_fit holding it as a view
     uint32_t* present_to;  // during prh_surface_render: the acquired surface texture
-    prh_tuning tune;       // speed knobs (results do not depend on them)
+    Knobs tune;            // speed knobs (results do not depend on them)
     bool split_shade_last;  // the last frame split its shading
     int raster_end_last;    // the stamp its raster pass ends at
     bool bg_last;           // k_shade_bg ran
@@ -1081,8 +1066,7 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     HIP_TRY(hipSetDevice(ctx->device));
     prh_renderer* r = new prh_renderer();
     r->ctx = ctx, r->sc = s, r->cam = *cam, r->opt = *o;
-    r->tune = prh_tuning{8, ITEM_PRIMS, 64, MAIN_DIRECT_MAX, (size_t)o->width * o->height * msaa * msaa >= OVERLAP_PIXELS ? 1 : 0,
-                         TILE, 0.0f};
+    r->tune = default_knobs((size_t)o->width * o->height * msaa * msaa);
     // every pass renders the MSAA-sized buffer (render/raster.go:149-150)
     r->msaa = msaa, r->OW = o->width, r->OH = o->height;
     r->W = o->width * msaa, r->H = o->height * msaa;
@@ -1380,9 +1364,7 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     // a plain frame runs its shadow passes on the context's second stream,
     // beside the main view's passes (they meet at the shading); a batch
     // keeps them on its own stream
-    // (a knob at its default for the frame's size: only where it pays)
-    const bool pays = P < OVERLAP_PIXELS || d.n_tris > LATENCY_TRIS || (r->sc->any_ao && P >= OVERLAP_AO_PIXELS);
-    const bool split = shadows && !wide && st == r->ctx->stream && r->tune.overlap_shadows && pays;
+    const bool split = shadows && !wide && st == r->ctx->stream && two_streams(r->tune, P, d.n_tris, r->sc->any_ao);
     const hipStream_t ss = split ? r->ctx->stream2 : st;
     // with AO as well, the AO runs on the second stream (after the shadow
     // passes) beside the shading's first half (everything but the AO factor)
@@ -1409,10 +1391,9 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
                        FrameClear{(uint32_t*)cm, (shadows ? 1 : 2) * CNT_WORDS, (uint64_t*)r->vis, P},
                        at(ST_VERTEX, ST_VERTEX_END));
     wide_stage(8);
-    // a frame whose setup fits the chip at once waits for the setup's longest
-    // wave: left at its default, the knob hands the raster more of them there
-    const int32_t draw_small = r->tune.main_direct_max == MAIN_DIRECT_MAX && !wide && d.n_tris <= LATENCY_TRIS
-                                   ? MAIN_DIRECT_FEW : r->tune.main_direct_max;
+    // (a frame whose setup fits the chip at once waits for the setup's longest
+    // wave: by default it hands the raster more triangles)
+    const int32_t draw_small = direct_centres(r->tune, d.n_tris, wide);
     // (the exact-order pass keeps the frame's statistics: it draws nothing in
     // the setup, so its raster takes other primitives)
     launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->jobs, r->clips, r->tri_clip_slot, r->clip_list,
@@ -2553,31 +2534,37 @@ int prh_get_tuning(prh_renderer* r, prh_tuning* out) {
     return PRH_OK;
 }
 
-int prh_set_tuning(prh_renderer* r, const prh_tuning* t) {
-    if (!r || !t) return fail(PRH_E_INVALID, "prh_set_tuning: null argument");
-    const bool pow2 = t->item_prims > 0 && (t->item_prims & (t->item_prims - 1)) == 0;
-    if (t->raster_wg_per_cu < 1 || t->raster_wg_per_cu > 16 || !pow2 || t->item_prims < 64 ||
-        t->item_prims > 8192 || t->shadow_direct_max < 0 || t->shadow_direct_max > 256 || t->main_direct_max < 0 ||
-        t->main_direct_max > 256 || (t->overlap_shadows != 0 && t->overlap_shadows != 1) ||
-        (t->raster_tile != 8 && t->raster_tile != 16 && t->raster_tile != 32))
-        return fail(PRH_E_INVALID, "prh_set_tuning: a knob out of range");
+}  // extern "C" (the helper below is the library's own)
+
+namespace {
+
+int put_knobs(prh_renderer* r, const Knobs& k) {
     HIP_TRY(hipSetDevice(r->ctx->device));
     HIP_TRY(hipStreamSynchronize(r->ctx->stream));
-    r->tune.raster_wg_per_cu = t->raster_wg_per_cu, r->tune.item_prims = t->item_prims;
-    r->tune.shadow_direct_max = t->shadow_direct_max, r->tune.main_direct_max = t->main_direct_max;
-    r->tune.overlap_shadows = t->overlap_shadows;
-    r->tune.raster_tile = t->raster_tile;
-    r->shc.direct_max = t->shadow_direct_max;
+    r->tune = k;
+    r->shc.direct_max = k.shadow_direct_max;
     raster_tile(r);
     r->work_gen++;  // a cached batch recorded the old values
     return PRH_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+int prh_set_tuning(prh_renderer* r, const prh_tuning* t) {
+    if (!r || !t) return fail(PRH_E_INVALID, "prh_set_tuning: null argument");
+    if (!valid_knobs(*t)) return fail(PRH_E_INVALID, "prh_set_tuning: a knob out of range");
+    Knobs k = r->tune;
+    set_knobs(k, *t);
+    return put_knobs(r, k);
+}
+
 int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
     if (!r) return fail(PRH_E_INVALID, "prh_autotune: null renderer");
     if (frames < 1) frames = 5;
-    auto time = [&](const prh_tuning& t, float* ms) -> int {
-        int rc = prh_set_tuning(r, &t);
+    auto time = [&](const Knobs& t, float* ms) -> int {
+        int rc = put_knobs(r, t);
         if (rc) return rc;
         if ((rc = prh_render(r))) return rc;  // warm-up (and any regrowth)
         std::vector<float> v;
@@ -2595,23 +2582,29 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
     static const int32_t c_md[] = {0, 24, 48, 96, 192};
     static const int32_t c_ov[] = {0, 1};
     static const int32_t c_rt[] = {8, 16, 32};
-    const prh_tuning start = r->tune;
-    prh_tuning best = start;
+    const size_t P = (size_t)r->W * r->H;
+    const int64_t n_tris = r->sc->d.n_tris;
+    const Knobs start = r->tune;
+    Knobs best = start;
     float best_ms = 0.0f;
     int rc = time(best, &best_ms);
     if (rc) return rc;
-    // coordinate descent: each knob over its candidates, the others at their best
+    // coordinate descent: each knob over its candidates, the others at their
+    // best; one never set is first timed by its rule
     for (int knob = 1; knob < 6; knob++) {
         const int32_t* c = knob == 1 ? c_wg : knob == 2 ? c_sd : knob == 3 ? c_md : knob == 4 ? c_ov : c_rt;
         const int n = knob == 1 ? 4 : knob == 2 ? 6 : knob == 3 ? 5 : knob == 4 ? 2 : 3;
         for (int k = 0; k < n; k++) {
-            prh_tuning t = best;
+            Knobs t = best;
             int32_t* f = knob == 1 ? &t.raster_wg_per_cu
                        : knob == 2 ? &t.shadow_direct_max
                        : knob == 3 ? &t.main_direct_max
                        : knob == 4 ? &t.overlap_shadows : &t.raster_tile;
-            if (*f == c[k]) continue;
+            const int32_t now = knob == 3 ? direct_centres(best, n_tris, false)
+                              : knob == 4 ? two_streams(best, P, n_tris, r->sc->any_ao) : *f;
+            if (now == c[k]) continue;
             *f = c[k];
+            t.direct_set |= knob == 3, t.overlap_set |= knob == 4;
             float ms = 0.0f;
             if ((rc = time(t, &ms))) return rc;
             if (ms < best_ms) best = t, best_ms = ms;
@@ -2619,7 +2612,8 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
     }
     // a second look at the winner against the starting point, over twice the
     // frames, so that one noisy median does not move the knobs
-    if (std::memcmp(&best, &start, offsetof(prh_tuning, ms)) != 0) {
+    if (std::memcmp(&best, &start, offsetof(prh_tuning, ms)) != 0 || best.direct_set != start.direct_set ||
+        best.overlap_set != start.overlap_set) {
         frames *= 2;
         float ms_best = 0.0f, ms_start = 0.0f;
         if ((rc = time(start, &ms_start)) || (rc = time(best, &ms_best))) return rc;
@@ -2627,8 +2621,7 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
         else best_ms = ms_best;
     }
     best.ms = best_ms;
-    if ((rc = prh_set_tuning(r, &best))) return rc;
-    r->tune.ms = best_ms;
+    if ((rc = put_knobs(r, best))) return rc;
     if ((rc = prh_render(r))) return rc;  // leave a frame of the chosen configuration
     if (out) *out = r->tune;
     return PRH_OK;
@@ -2641,7 +2634,7 @@ int prh_autotune_batch(prh_renderer* const* rs, int32_t n, int32_t frames, prh_t
     if (frames < 1) frames = 5;
     std::vector<int> cls(n);
     for (int i = 0; i < n; i++) cls[i] = (int64_t)rs[i]->W * rs[i]->H >= (1 << 19) ? 1 : 0;
-    std::vector<prh_tuning> start(n);
+    std::vector<Knobs> start(n);
     for (int i = 0; i < n; i++) start[i] = rs[i]->tune;
     // the classes start from the knobs of their first view
     prh_tuning cur[2];
@@ -2655,9 +2648,13 @@ int prh_autotune_batch(prh_renderer* const* rs, int32_t n, int32_t frames, prh_t
     }
     auto apply = [&](const prh_tuning* t) -> int {
         for (int i = 0; i < n; i++) {
-            prh_tuning v = t[cls[i]];
-            v.overlap_shadows = rs[i]->tune.overlap_shadows;  // (not used by a wide batch)
-            int rc = prh_set_tuning(rs[i], &v);
+            Knobs v = start[i];
+            static_cast<prh_tuning&>(v) = t[cls[i]];
+            // (a wide batch does not use the overlap, nor a rule for the
+            // threshold: the view's own frames keep theirs where it stays)
+            v.overlap_shadows = start[i].overlap_shadows;
+            v.direct_set |= v.main_direct_max != start[i].main_direct_max;
+            int rc = put_knobs(rs[i], v);
             if (rc) return rc;
         }
         return PRH_OK;
