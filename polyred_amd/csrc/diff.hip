@@ -27,6 +27,7 @@
 // frame that fixed the visibility.  A view's pixel state is either rebuilt
 // from the visibility buffer at every launch or read from a stored G-buffer.
 #include "kernels.hpp"
+#include "roots.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -51,10 +52,10 @@ __device__ __forceinline__ F3 fma3(float s, F3 a, F3 c) { return f3(fma1(s, a.x,
 __device__ __forceinline__ float dot(F3 a, F3 b) { return fma1(a.x, b.x, fma1(a.y, b.y, a.z * b.z)); }
 __device__ __forceinline__ F3 ld3(const float* p) { return f3(p[0], p[1], p[2]); }
 __device__ __forceinline__ F3 xyz(float4 a) { return f3(a.x, a.y, a.z); }
-// 1 / sqrt(x), 1 / x and x / y within 0.51 ulp from the hardware estimates (1
-// ulp) and one Newton step each, with the residual 1 - x r^2 to both halves of
-// x r: a third of the instructions of the correctly rounded expansions (1 /
-// sqrtf(x) rounds twice).  They hold for 2^-100 <= |x| < 2^100; `off` collects
+// 1 / x and x / y by the steps of roots.hpp, and 1 / sqrt(x) within 0.51 ulp from
+// the hardware estimate (1 ulp) and one Newton step, with the residual 1 - x r^2
+// to both halves of x r: a third of the instructions of the compiler's
+// expansions (1 / sqrtf(x) rounds twice).  They hold for 2^-100 <= |x| < 2^100; `off` collects
 // the inputs outside, and a pixel that had one is computed again with SAFE,
 // the library's.
 template <bool SAFE>
@@ -75,14 +76,12 @@ struct Ops {
     __device__ __forceinline__ float rcp(float x) {
         if (SAFE) return 1.0f / x;
         note(x);
-        const float r = __builtin_amdgcn_rcpf(x);
-        return fma1(fma1(-x, r, 1.0f), r, r);
+        return rcp_exact(x);
     }
     // x / y with r = rcp(y)
     __device__ __forceinline__ float quot(float x, float y, float r) {
         if (SAFE) return x / y;
-        const float q = x * r;
-        return fma1(fma1(-q, y, x), r, q);
+        return quot_exact(x, y, r);
     }
 };
 // x / 255: a product with the rounded 1 / 255 alone would scale every colour

@@ -5,6 +5,7 @@
 // (render/raster.go, render/clipping.go, render/shadow.go,
 // shader/blinn_cpu.go, material/ao.go, shader/gamma.go) through gomath.hpp.
 #include "kernels.hpp"
+#include "roots.hpp"
 
 #include <functional>
 #include <map>
@@ -1123,31 +1124,14 @@ struct GFrag {
     float u, v, du, dv;  // texture coordinates and their screen derivatives (scenes with textures)
 };
 
-// The shading's roots and quotients without the compiler's scaling and special
-// cases, where every lane's operand is in a range in which no step over- or
-// underflows; a wave with a lane outside takes the plain ones.  Each is the
-// correctly rounded result, as the plain one: the reciprocal and the root by
-// the hardware's estimate and one residual step (Markstein 1990) -- from this
-// hardware's estimates that step is exact for every float32 mantissa, at even
-// and odd exponents alike -- and the quotient by a residual step from the
-// correctly rounded reciprocal.  A length and its reciprocal take 8
+// The shading's lengths and barycentrics take the steps of roots.hpp where every
+// lane's operand is in their range; a wave with a lane outside takes the plain
+// ones.  A length and its reciprocal take 8
 // instructions in place of 25; with the pow's series in fused steps and the
 // vertex colour and face normal only where they are read, k_shade went from
 // 37.3 to 30 M vector instructions at 1920x1080, 84.5 -> 80.5 us on one stream
 // (what is left there is waiting: 4 waves a SIMD at 128 registers, and loads
 // by triangle and by shadow texel).
-__device__ __forceinline__ float rcp_exact(float x) {  // 1 / x, 2^-64 <= |x| < 2^64
-    const float y = __builtin_amdgcn_rcpf(x);
-    return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
-}
-__device__ __forceinline__ float quot_exact(float a, float x, float r) {  // a / x with r = rcp_exact(x)
-    const float q = a * r;
-    return __builtin_fmaf(__builtin_fmaf(-x, q, a), r, q);
-}
-__device__ __forceinline__ float sqrt_exact(float d) {  // sqrt(d), 2^-64 <= d < 2^64
-    const float r = __builtin_amdgcn_rsqf(d), g = d * r;
-    return __builtin_fmaf(__builtin_fmaf(-g, g, d), 0.5f * r, g);
-}
 __device__ __forceinline__ bool mid_range(float x) {  // 2^-63 <= x < 2^63
     return __float_as_uint(x) - 0x20000000u < 0x5f000000u - 0x20000000u;
 }
