@@ -218,7 +218,9 @@ int prh_read_image(prh_renderer* r, uint8_t* rgba, size_t bytes);
 int prh_read_buffer(prh_renderer* r, int32_t which, void* dst, size_t bytes);
 
 /* Per-pass device time of the last frame, from stamps of the device's clock
- * its kernels write. */
+ * its kernels write.  The end of a pass is the latest end among its last
+ * kernel's every 64th workgroup and its last one, so a time leaves out what
+ * others take past those: it is a lower bound. */
 typedef struct prh_frame_stats {
     float ms_total;
     float ms_shadow;     /* all shadow passes                               */
@@ -385,17 +387,17 @@ typedef struct prh_tuning {
                                   at least 2^22 pixels)                                                   */
     int32_t raster_tile;       /* side of the raster tiles (main view and shadow maps): 8, 16 or 32
                                   pixels, a raster job being at most 2 x 2 of them; default 16            */
-    float ms;                  /* prh_autotune: the chosen configuration's median frame time             */
+    float ms;                  /* prh_autotune: the chosen configuration's median time of a prh_render    */
 } prh_tuning;
 int prh_get_tuning(prh_renderer* r, prh_tuning* out);
 /* Sets every knob but `ms`; from then on each is taken at its value. */
 int prh_set_tuning(prh_renderer* r, const prh_tuning* t);
-/* Coordinate descent over raster_wg_per_cu {1, 2, 4, 8}, shadow_direct_max {0, 16, 32, 64, 128, 256}, main_direct_max {0, 24,
- * 48, 96, 192}, overlap_shadows {0, 1} and raster_tile {8, 16, 32}: each
- * configuration timed as the median of
- * `frames` frames (HIP events, after one warm-up frame); the winner is timed
- * again against the starting knobs over twice the frames and the faster of
- * the two stays on r and goes to *out (may be NULL).  A knob nobody set
+/* Coordinate descent over raster_wg_per_cu {1, 2, 4, 8}, shadow_direct_max
+ * {0, 16, 32, 64, 128, 256}, main_direct_max {0, 24, 48, 96, 192},
+ * overlap_shadows {0, 1} and raster_tile {8, 16, 32}: each configuration timed
+ * as the median of `frames` prh_render calls (the host's clock, after one more
+ * call); the winner is timed again against the starting knobs over twice the
+ * frames and the faster of the two stays on r and goes to *out (may be NULL).  A knob nobody set
  * starts from its rule and keeps it, reported at its default, where no
  * candidate is faster.  r holds a frame of the winner on return. */
 int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out);

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -2569,9 +2570,11 @@ int prh_autotune(prh_renderer* r, int32_t frames, prh_tuning* out) {
         if ((rc = prh_render(r))) return rc;  // warm-up (and any regrowth)
         std::vector<float> v;
         for (int k = 0; k < frames; k++) {
+            // (the whole call: the passes' stamps sample workgroups, other ones
+            // for other grids)
+            const auto t0 = std::chrono::steady_clock::now();
             if ((rc = prh_render(r))) return rc;
-            if ((rc = fill_times(r))) return rc;
-            v.push_back(r->stats.ms_total);
+            v.push_back(std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count());
         }
         std::sort(v.begin(), v.end());
         *ms = v[v.size() / 2];
