@@ -140,8 +140,8 @@ def run_frames(r, steps: int):
 def adjoint_bench(dev, steps: int) -> dict:
     """Forward + adjoint against a plain single view: the 512x512 ~100k-
     triangle 4-light scene, target rendered from seed parameters, gradients
-    at a 10 % Gaussian perturbation.  Device times from the frames' clock stamps and HIP events: one
-    frame (prh_render), one adjoint launch (loss + all gradients)."""
+    at a 10 % Gaussian perturbation.  Device times: one frame (prh_render) by
+    its clock stamps, one adjoint launch (loss + all gradients) by HIP events."""
     from polyred_amd import diff, render, scenes
 
     s = scenes.c4_adjoint()
@@ -227,9 +227,9 @@ def fit_bench(dev, steps: int = 200) -> dict:
     (1024^2 maps) at fixed visibility.  Targets from the scene's own
     materials and lights; start 30 % off (Gaussian, per value); 200 Adam
     steps at lr 1e-2 on Kd, Ks, shininess, light positions and intensities,
-    each step the adjoint of all 32 views in one launch plus the update (a
-    replayed HIP graph).  Run twice: per-pixel state rebuilt from the
-    visibility buffer at every step, and read from a stored G-buffer."""
+    each step the adjoint of all 32 views in one launch plus the update.
+    Run twice: per-pixel state rebuilt from the visibility buffer at every
+    step, and read from a stored G-buffer."""
     from polyred_amd import diff, render, scenes
 
     s, cams = scenes.c5_inverse()
@@ -351,7 +351,7 @@ def main() -> int:
     r = render.renderer_for(scene, dev)
     tuned = None
     if not args.no_autotune:
-        t = r.Autotune(frames=5)  # occupancy, bin capacity, small-triangle thresholds; results unchanged
+        t = r.Autotune(frames=5)  # occupancy, small-triangle thresholds, streams, tile; results unchanged
         tuned = {"raster_wg_per_cu": t.raster_wg_per_cu, "item_prims": t.item_prims,
                  "shadow_direct_max": t.shadow_direct_max, "main_direct_max": t.main_direct_max,
                  "overlap_shadows": t.overlap_shadows, "raster_tile": t.raster_tile}

@@ -1168,8 +1168,8 @@ int prh_renderer_new(prh_ctx* ctx, prh_scene* s, const prh_camera* cam, const pr
     const int clip_tris = std::min(Tg, 1 << 16) + 16;
     // A raster queue's first capacity (grown when a frame overflows it): its
     // share of every triangle at one job (of a quarter of them for the maps,
-    // whose triangles are mostly drawn by the setup), and the jobs of a few
-    // triangles that cover the screen, which their workgroup sends to one queue
+    // whose triangles are mostly drawn by the setup), and the jobs of some
+    // triangles that cover the screen, 64 of 32 x 32 pixel centres each
     r->cap_main = Capacities{CLIP_PIECES * clip_tris, clip_tris, (int32_t)(Tg / RASTER_QUEUES + P / 256 + 1024)};
     r->cap_shadow = Capacities{0, 0, (int32_t)((int64_t)r->n_slots * Tg / (4 * RASTER_QUEUES) +
                                                (int64_t)r->SW * r->SH / 256 + 1024)};
@@ -1458,7 +1458,8 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
         launch_resize(st, r->resize_tmp, r->H, final_image(r), r->OW, r->OH, r->rz_cy, r->rz_oy, r->rz_fly,
                       at(-1, ST_END));
     }
-    // (k_shade_bg writes the counters into r->h_cnt)
+    // (k_shade_bg wrote the counters into r->h_cnt, or k_shade where that one
+    // does not run)
     return PRH_OK;
 }
 

@@ -142,7 +142,7 @@ class Fit:
     """Gradient descent on the shading parameters over many views of one
     scene (prh_fit_*): each view's last frame fixes its visibility and its
     shadow visibility; one step is the adjoint of every view in one launch
-    plus an Adam update on the device, the steps one replayed HIP graph.
+    plus an Adam update on the device.
 
         gs, views = render.views_of(scene, cams, dev)
         for r in views: r.render_device()
