@@ -935,9 +935,7 @@ __global__ __launch_bounds__(CLIP_WAVES * 64) void k_clip_wide(const k_clip_args
 // that still beats the tiles' merge in LDS which this replaced (prh_render at
 // 1920x1080, per-tile lists -> jobs: 1000 triangles across the view 38.3 -> 4.9
 // ms, 50 k of some 200 pixels 13.2 -> 9.9, 100 k of 50 1.65 -> 1.49, 1 M of 16
-// 1.71 -> 1.61).  Where not even the smallest triangles are drawn by the setup
-// (shadow_direct_max = 0, 1.04 M of them into five maps) a wave a job is the
-// slower way, 0.65 -> 0.93 ms; from 16 on any threshold is faster.
+// 1.71 -> 1.61).
 enum { MODE_VIS = 0, MODE_EXACT = 1, MODE_SHADOW = 2 };
 
 struct k_raster_args {
@@ -947,7 +945,11 @@ struct k_raster_args {
     Stamp stamp;
     int32_t gx, gy;  // the grid of this launch
 };
-template <int MODE>
+// PACK, where the setup leaves the smallest triangles to the raster (launch_raster):
+// a wave reads sixty-four of its jobs at once, and those of at most 64 centres,
+// one round of a wave of their own, it spreads over its lanes together, as the
+// setups do.
+template <int MODE, bool PACK>
 __device__ __forceinline__ void k_raster_body(const k_raster_args& a_, const VB vb) {
     constexpr bool SHADOW = MODE == MODE_SHADOW, EXACT = MODE == MODE_EXACT;
     const JobQueues& jq = a_.jobs;
@@ -959,8 +961,19 @@ __device__ __forceinline__ void k_raster_body(const k_raster_args& a_, const VB 
     const int n = cnt->overflow ? 0 : __builtin_amdgcn_readfirstlane((int)min(jq.n[qi * JOB_COUNT_STRIDE], (unsigned long long)jq.cap));
     const Prim* jobs = jq.jobs + (size_t)qi * jq.cap;
     bool saw_nan = false;
-    // (nw is a multiple of RASTER_QUEUES: the launches see to it)
-    for (int j = w0 / RASTER_QUEUES; j < n; j += nw / RASTER_QUEUES) {
+    auto merge = [&](int px, int py, float z, uint32_t key) {
+        const size_t o = (size_t)py * rt.W + px;
+        if (EXACT) atomicMin(&rt.first_all[o], key);
+        if (z != z) {
+            saw_nan = true;
+            if (EXACT) atomicMin(&rt.first_nan[o], key);
+        } else if (SHADOW) {
+            if (z > 0.0f) atomicMax(&rt.smap_ord[(size_t)key * rt.W * rt.H + o], depth_ord(z));  // the map starts at 0
+        } else {
+            atomicMin(&rt.vis[o], ((unsigned long long)depth_key_hi(z) << 32) | key);
+        }
+    };
+    auto draw = [&](int j) {  // one job, uniform over the wave
         const Prim* p = jobs + j;
         auto u = [](float f) { return bitsf(__builtin_amdgcn_readfirstlane(fbits(f))); };
         const float4 q0 = p->p0, q1 = p->p1, q2 = p->p2;
@@ -976,37 +989,55 @@ __device__ __forceinline__ void k_raster_body(const k_raster_args& a_, const VB 
         while (ly < h) {
             const int px = x0 + lx, py = y0 + ly;
             float z;
-            if (cover_z(t, (float)px + 0.5f, (float)py + 0.5f, az, bz, cz, z)) {  // raster.go:487-496
-                const size_t o = (size_t)py * rt.W + px;
-                if (EXACT) atomicMin(&rt.first_all[o], key);
-                if (z != z) {
-                    saw_nan = true;
-                    if (EXACT) atomicMin(&rt.first_nan[o], key);
-                } else if (SHADOW) {
-                    if (z > 0.0f) atomicMax(&rt.smap_ord[(size_t)key * rt.W * rt.H + o], depth_ord(z));  // the map starts at 0
-                } else {
-                    atomicMin(&rt.vis[o], ((unsigned long long)depth_key_hi(z) << 32) | key);
-                }
-            }
+            if (cover_z(t, (float)px + 0.5f, (float)py + 0.5f, az, bz, cz, z)) merge(px, py, z, key);  // raster.go:487-496
             lx += r64, ly += q64;
             if (lx >= w) lx -= w, ly++;
+        }
+    };
+    // the wave's jobs: every nq-th from its own place in the queue on (nw is a
+    // multiple of RASTER_QUEUES: the launches see to it)
+    const int first = w0 / RASTER_QUEUES, nq = nw / RASTER_QUEUES;
+    if constexpr (!PACK) {
+        for (int j = first; j < n; j += nq) draw(j);
+    } else {
+        __shared__ DPrim sp[256];
+        __shared__ int32_t mark[256];
+        __shared__ uint32_t s_key[256];
+        uint32_t* wkey = s_key + (threadIdx.x & ~63);
+        for (int64_t j0 = first; j0 < n; j0 += 64 * nq) {
+            const int64_t j = j0 + lane * nq;
+            const bool have = j < n;
+            const Prim* p = jobs + j;
+            uint32_t lo = 0, hi = 0;
+            float4 q2 = make_float4(0, 0, 0, 0);
+            if (have) q2 = p->p2, lo = fbits(q2.z), hi = fbits(q2.w);
+            const int x0 = (int)(lo & 0xffff), y0 = (int)(lo >> 16), x1 = (int)(hi & 0xffff), y1 = (int)(hi >> 16);
+            const bool small = have && (x1 - x0 + 1) * (y1 - y0 + 1) <= 64;
+            if (__ballot(small) != 0) {
+                float4 q0 = make_float4(0, 0, 0, 0), q1 = q0;
+                if (small) q0 = p->p0, q1 = p->p1, wkey[lane] = fbits(q2.y);
+                draw_small_tris(small, v4(q0.x, q0.y, q0.z, 1), v4(q0.w, q1.x, q1.y, 1), v4(q1.z, q1.w, q2.x, 1), x0, y0,
+                                x1, y1, sp, mark, [&](int px, int py, float z, int o) { merge(px, py, z, wkey[o]); });
+            }
+            for (uint64_t big = __ballot(have && !small); big; big &= big - 1)
+                draw((int)j0 + __builtin_ctzll(big) * nq);
         }
     }
     if (saw_nan) atomicOr(SHADOW ? &cnt->shadow_nan : &cnt->nan_flag, 1);
     stamp_end(a_.stamp, vb);
 }
-template <int MODE>
+template <int MODE, bool PACK>
 __global__ __launch_bounds__(256) void k_raster(k_raster_args a) {
-    k_raster_body<MODE>(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
+    k_raster_body<MODE, PACK>(a, VB{(int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y});
 }
-template <int MODE>
+template <int MODE, bool PACK>
 __global__ __launch_bounds__(256) void k_raster_wide(const k_raster_args* __restrict__ a, const int32_t* __restrict__ start,
         int32_t n) {
     const int v = wide_view(start, n, (int)blockIdx.x);
     const k_raster_args& x = a[v];
     const int local = (int)blockIdx.x - start[v];
     if (local >= x.gx * x.gy) return;  // padding to a multiple of 8 workgroups
-    k_raster_body<MODE>(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
+    k_raster_body<MODE, PACK>(x, VB{local % x.gx, local / x.gx, x.gx, x.gy});
 }
 
 // Fragment depth per pixel from the visibility key (-1 where uncovered, as
@@ -2742,14 +2773,28 @@ __global__ __launch_bounds__(256) void k_tri_rec(DevScene s, int4* tri_rec) {
 void launch_tri_rec(hipStream_t st, const DevScene& s, int4* tri_rec) {
     if (s.n_tris) hipLaunchKernelGGL(k_tri_rec, dim3(blocks_for(s.n_tris, 256)), dim3(256), 0, st, s, tri_rec);
 }
-void launch_raster(hipStream_t st, int mode, int n_workgroups, const JobQueues& jobs, Counters* cnt,
+template <int MODE>
+static void launch_raster_t(hipStream_t st, const dim3& grid, const k_raster_args& a, bool pack) {
+    // (in a recorded batch each is a group of its own in the stage)
+    if (g_wide) g_wide->sub = pack;
+    if (pack) go(k_raster<MODE, true>, k_raster_wide<MODE, true>, grid, 256, st, a);
+    else go(k_raster<MODE, false>, k_raster_wide<MODE, false>, grid, 256, st, a);
+}
+// `direct`: the setup drew triangles of at most so many centres.  Below 16 the
+// small jobs are many: packed, 1.04 M triangles into five maps take a frame of
+// 480 us at shadow_direct_max = 0 (918 a wave a job, 641 with per-tile lists),
+// 452 at 8 (596, 586); a 64-view batch 2.94 ms at 0 (6.4, 3.8), 2.7 at 4 (4.1,
+// 3.5).  From 16 on it gains little (the batch at 16: 2.31 against 2.34 ms) and
+// the larger kernel costs small frames a microsecond.
+void launch_raster(hipStream_t st, int mode, int direct, int n_workgroups, const JobQueues& jobs, Counters* cnt,
                    const RasterTarget& rt, Stamp stamp) {
+    const bool pack = direct < 16;
     const k_raster_args a{jobs, cnt, rt, stamp, 0, 0};
     // (four waves a workgroup: every queue gets the same number of waves)
     const dim3 grid((n_workgroups + RASTER_QUEUES / 4 - 1) / (RASTER_QUEUES / 4) * (RASTER_QUEUES / 4));
-    if (mode == MODE_SHADOW) go(k_raster<MODE_SHADOW>, k_raster_wide<MODE_SHADOW>, grid, 256, st, a);
-    else if (mode == MODE_EXACT) go(k_raster<MODE_EXACT>, k_raster_wide<MODE_EXACT>, grid, 256, st, a);
-    else go(k_raster<MODE_VIS>, k_raster_wide<MODE_VIS>, grid, 256, st, a);
+    if (mode == MODE_SHADOW) launch_raster_t<MODE_SHADOW>(st, grid, a, pack);
+    else if (mode == MODE_EXACT) launch_raster_t<MODE_EXACT>(st, grid, a, pack);
+    else launch_raster_t<MODE_VIS>(st, grid, a, pack);
 }
 void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters* cnt, float* depth, const DevScene& s,
                     int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec, Stamp stamp) {

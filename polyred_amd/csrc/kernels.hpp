@@ -226,8 +226,9 @@ void launch_setup_shadow(hipStream_t st, const DevScene& s, const ShadowConsts& 
 // vertices and its material in the flat table (-1: vertex colour, matAt's
 // rule), or x = -1 when Triangle.IsValid is false.  Once per renderer.
 void launch_tri_rec(hipStream_t st, const DevScene& s, int4* tri_rec);
-// mode: 0 visibility, 1 visibility in exact order (NaN rule), 2 shadow maps
-void launch_raster(hipStream_t st, int mode, int n_workgroups, const JobQueues& jobs, Counters* cnt,
+// mode: 0 visibility, 1 visibility in exact order (NaN rule), 2 shadow maps;
+// direct: the setup drew the triangles of at most so many centres
+void launch_raster(hipStream_t st, int mode, int direct, int n_workgroups, const JobQueues& jobs, Counters* cnt,
                    const RasterTarget& rt, Stamp stamp);
 void launch_resolve(hipStream_t st, bool exact, const RasterTarget& rt, Counters* cnt, float* depth, const DevScene& s,
                     int32_t* ao_xs, int32_t* ao_cnt, const int4* tri_rec, Stamp stamp);

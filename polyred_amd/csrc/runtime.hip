@@ -1383,7 +1383,7 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
         launch_setup_shadow(ss, d, r->shc, r->tri_rec, r->ts, r->s_jobs, cs, r->smaps);
         RasterTarget rt{r->SW, r->SH, nullptr, nullptr, nullptr, r->smaps};
         wide_stage(6);
-        launch_raster(ss, 2, persistent, r->s_jobs, cs, rt, at(-1, ST_SHADOW_END));
+        launch_raster(ss, 2, r->tune.shadow_direct_max, persistent, r->s_jobs, cs, rt, at(-1, ST_SHADOW_END));
         if (split && !split_shade) (void)hipEventRecord(r->ev_join, ss);
     }
     wide_stage(7);
@@ -1394,12 +1394,12 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     wide_stage(8);
     // (a frame whose setup fits the chip at once waits for the setup's longest
     // wave: by default it hands the raster more triangles)
-    const int32_t draw_small = direct_centres(r->tune, d.n_tris, wide);
+    const int32_t draw_small = nan_mode ? 0 : direct_centres(r->tune, d.n_tris, wide);
     // (the exact-order pass keeps the frame's statistics: it draws nothing in
     // the setup, so its raster takes other primitives)
     launch_setup_main(st, d, r->vc, r->tv_scr, r->tv_nor, r->jobs, r->clips, r->tri_clip_slot, r->clip_list,
                       r->blk_prims, nan_mode ? nullptr : r->blk_pairs, cm, r->cap_main, (unsigned long long*)r->vis,
-                      nan_mode ? 0 : draw_small, r->tune.main_direct_max, r->tri_rec, at(-1, ST_SETUP_END));
+                      draw_small, r->tune.main_direct_max, r->tri_rec, at(-1, ST_SETUP_END));
     if (nan_mode) {
         launch_fill_u32(st, r->first_all, P, 0xffffffffu);
         launch_fill_u32(st, r->first_nan, P, 0xffffffffu);
@@ -1415,7 +1415,7 @@ int enqueue_frame(prh_renderer* r, bool nan_mode, hipStream_t st, bool timed, bo
     // (the pass ends with the resolve, else where k_shade_bg starts, else with
     // the raster: of its unequal workgroups a stamp sees a few)
     r->raster_end_last = resolve || bg_inline ? ST_RESOLVED : ST_BG, r->bg_last = !bg_inline;
-    launch_raster(st, nan_mode ? 1 : 0, persistent, r->jobs, cm, rt, at(-1, !resolve && bg_inline ? ST_RESOLVED : -1));
+    launch_raster(st, nan_mode ? 1 : 0, draw_small, persistent, r->jobs, cm, rt, at(-1, !resolve && bg_inline ? ST_RESOLVED : -1));
     wide_stage(12);
     if (resolve)
         launch_resolve(st, nan_mode, rt, cm, r->depth, d, r->sc->any_ao ? r->ao_xs : nullptr, r->ao_cnt, r->tri_rec,
