@@ -275,9 +275,13 @@ __device__ __forceinline__ DPix diff_pixel(Ops<SAFE>& op, const DTri& t, const i
 // copies (up to 18 materials) no two lanes of a half-wave share a bank or an
 // address, and the wave does no reduction at all (one reduction of 7 values
 // per distinct material, by shuffles, was a quarter of the adjoint).  More
-// materials take fewer copies; above DIFF_MAT_SLOTS / 7 of them the lanes go
-// to the global gradients.
-constexpr int DIFF_MAT_SLOTS = 4096;
+// materials take fewer copies; above DIFF_MAT_SLOTS / 7 of them the bins of the
+// materials the workgroup meets are found by open addressing (DIFF_MAT_KEYS of
+// them, their keys in the rest of the array), and only one that finds no bin in
+// DIFF_MAT_PROBES goes to memory.  (All lanes adding to memory took 6.5 ms a
+// step of 8 views with 700 materials; 0.09 now, 0.06 with 8.)
+constexpr int DIFF_MAT_SLOTS = 4096, DIFF_MAT_KEYS = 512, DIFF_MAT_PROBES = 8;
+static_assert(8 * DIFF_MAT_KEYS <= DIFF_MAT_SLOTS, "seven values and a key a bin");
 struct DiffAcc {
     float mat[DIFF_MAT_SLOTS];
     float light[4 * DIFF_MAX_LIGHTS];
@@ -289,8 +293,27 @@ __device__ __forceinline__ int mat_copies(int n_mats) {
     return c;
 }
 
+// The bin of material `mat` among the found ones (a bin's value j is at
+// mat[j * DIFF_MAT_KEYS + bin]), or -1.
+__device__ __forceinline__ int32_t* mat_keys(DiffAcc& a) {  // material + 1, 0: free
+    return reinterpret_cast<int32_t*>(a.mat + 7 * DIFF_MAT_KEYS);
+}
+__device__ __forceinline__ int mat_bin(DiffAcc& a, int mat) {
+    int32_t* keys = mat_keys(a);
+    int h = mat & (DIFF_MAT_KEYS - 1);
+    for (int probe = 0; probe < DIFF_MAT_PROBES; probe++, h = (h + 1) & (DIFF_MAT_KEYS - 1)) {
+        int32_t k = keys[h];
+        if (k == 0) {
+            k = atomicCAS(&keys[h], 0, mat + 1);
+            if (k == 0) k = mat + 1;
+        }
+        if (k == mat + 1) return h;
+    }
+    return -1;
+}
 __device__ __forceinline__ void acc_clear(DiffAcc& a, int n_mats, int copies) {
-    for (int i = threadIdx.x; i < 7 * n_mats * copies; i += blockDim.x) a.mat[i] = 0.0f;
+    const int used = copies > 0 ? 7 * n_mats * copies : 8 * DIFF_MAT_KEYS;
+    for (int i = threadIdx.x; i < used; i += blockDim.x) a.mat[i] = 0.0f;  // (a free key's bits too)
     if (threadIdx.x < 4 * DIFF_MAX_LIGHTS) a.light[threadIdx.x] = 0.0f;
     if (threadIdx.x == 0) a.loss = 0.0;
     __syncthreads();
@@ -311,12 +334,19 @@ __device__ __forceinline__ void acc_flush(const DevScene& s, const B& b, DiffAcc
         if (v != 0.0f && (want & (pos ? DIFF_LIGHT_POS : DIFF_LIGHT_INT)))
             atomicAdd((pos ? &b.g_lpos[3 * (i >> 2) + (i & 3)] : &b.g_lint[i >> 2]) + ro, v);
     }
+    auto material = [&](int m, int j, float v) {
+        if (v != 0.0f && (want & (j < 3 ? DIFF_KD : j < 6 ? DIFF_KS : DIFF_SHININESS)))
+            atomicAdd((j < 3 ? &b.g_kd[3 * (size_t)m + j] : (j < 6 ? &b.g_ks[3 * (size_t)m + j - 3] : &b.g_shin[m])) + ro, v);
+    };
     for (int i = threadIdx.x; copies > 0 && i < 7 * s.n_materials; i += blockDim.x) {
         float v = 0.0f;
         for (int k = 0; k < copies; k++) v += a.mat[i * copies + ((k + i) & (copies - 1))];  // (banks rotated)
-        const int m = i / 7, j = i - 7 * m;
-        if (v != 0.0f && (want & (j < 3 ? DIFF_KD : j < 6 ? DIFF_KS : DIFF_SHININESS)))
-            atomicAdd((j < 3 ? &b.g_kd[3 * m + j] : (j < 6 ? &b.g_ks[3 * m + j - 3] : &b.g_shin[m])) + ro, v);
+        const int m = i / 7;
+        material(m, i - 7 * m, v);
+    }
+    for (int i = threadIdx.x; copies == 0 && i < 7 * DIFF_MAT_KEYS; i += blockDim.x) {
+        const int k = mat_keys(a)[i & (DIFF_MAT_KEYS - 1)];
+        if (k != 0) material(k - 1, i / DIFF_MAT_KEYS, a.mat[i]);
     }
     if (threadIdx.x == 0 && a.loss != 0.0) atomicAdd(b.loss + rep, a.loss);
 }
@@ -548,9 +578,11 @@ __device__ __forceinline__ void diff_adjoint(const DFwd<NLMAX>& f, const DevScen
         const float d = div255(f.sLd);
         const float gm_[7] = {ga.x * d, ga.y * d, ga.z * d, gl.x * div255(f.sLs.x), gl.y * div255(f.sLs.y),
                               gl.z * div255(f.sLs.z), gshin};
-        if (copies > 0) {
-            float* bin = acc.mat + 7 * mat * copies + (threadIdx.x & (copies - 1));
-            for (int j = 0; j < 7; j++) atomicAdd(bin + j * copies, gm_[j]);
+        const int slot = copies > 0 ? 0 : mat_bin(acc, mat);
+        if (slot >= 0) {
+            float* bin = copies > 0 ? acc.mat + 7 * mat * copies + (threadIdx.x & (copies - 1)) : acc.mat + slot;
+            const int step = copies > 0 ? copies : DIFF_MAT_KEYS;
+            for (int j = 0; j < 7; j++) atomicAdd(bin + j * step, gm_[j]);
         } else {
             for (int j = 0; j < 3; j++) {
                 atomicAdd(&b.g_kd[3 * (size_t)mat + j], gm_[j]);
