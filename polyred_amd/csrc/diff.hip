@@ -278,7 +278,8 @@ __device__ __forceinline__ DPix diff_pixel(Ops<SAFE>& op, const DTri& t, const i
 // materials take fewer copies; above DIFF_MAT_SLOTS / 7 of them the bins of the
 // materials the workgroup meets are found by open addressing (DIFF_MAT_KEYS of
 // them, their keys in the rest of the array), and only one that finds no bin in
-// DIFF_MAT_PROBES goes to memory.  (All lanes adding to memory took 6.5 ms a
+// DIFF_MAT_PROBES goes to memory; kernels of their own (FOUND), as the search's
+// registers cost the others 1 to 4 %.  (All lanes adding to memory took 6.5 ms a
 // step of 8 views with 700 materials; 0.09 now, 0.06 with 8.)
 constexpr int DIFF_MAT_SLOTS = 4096, DIFF_MAT_KEYS = 512, DIFF_MAT_PROBES = 8;
 static_assert(8 * DIFF_MAT_KEYS <= DIFF_MAT_SLOTS, "seven values and a key a bin");
@@ -287,7 +288,7 @@ struct DiffAcc {
     float light[4 * DIFF_MAX_LIGHTS];
     double loss;
 };
-__device__ __forceinline__ int mat_copies(int n_mats) {
+__host__ __device__ __forceinline__ int mat_copies(int n_mats) {  // 0: found bins
     int c = 32;
     while (c > 0 && 7 * n_mats * c > DIFF_MAT_SLOTS) c >>= 1;
     return c;
@@ -311,8 +312,9 @@ __device__ __forceinline__ int mat_bin(DiffAcc& a, int mat) {
     }
     return -1;
 }
+template <bool FOUND>
 __device__ __forceinline__ void acc_clear(DiffAcc& a, int n_mats, int copies) {
-    const int used = copies > 0 ? 7 * n_mats * copies : 8 * DIFF_MAT_KEYS;
+    const int used = FOUND ? 8 * DIFF_MAT_KEYS : 7 * n_mats * copies;
     for (int i = threadIdx.x; i < used; i += blockDim.x) a.mat[i] = 0.0f;  // (a free key's bits too)
     if (threadIdx.x < 4 * DIFF_MAX_LIGHTS) a.light[threadIdx.x] = 0.0f;
     if (threadIdx.x == 0) a.loss = 0.0;
@@ -323,7 +325,7 @@ __device__ __forceinline__ void acc_clear(DiffAcc& a, int n_mats, int copies) {
 // Each workgroup adds to one of the DIFF_REPS replicas of these gradients and
 // of the loss (its XCD's, as the dispatcher deals them): 1024 workgroups adding
 // to the same five cache lines took 25 us of a launch, an eighth of them 4.
-template <class B>
+template <bool FOUND, class B>
 __device__ __forceinline__ void acc_flush(const DevScene& s, const B& b, DiffAcc& a, int copies) {
     __syncthreads();
     const size_t rep = b.reps > 1 ? blockIdx.x % DIFF_REPS : 0, ro = rep * b.rep_stride;
@@ -338,15 +340,18 @@ __device__ __forceinline__ void acc_flush(const DevScene& s, const B& b, DiffAcc
         if (v != 0.0f && (want & (j < 3 ? DIFF_KD : j < 6 ? DIFF_KS : DIFF_SHININESS)))
             atomicAdd((j < 3 ? &b.g_kd[3 * (size_t)m + j] : (j < 6 ? &b.g_ks[3 * (size_t)m + j - 3] : &b.g_shin[m])) + ro, v);
     };
-    for (int i = threadIdx.x; copies > 0 && i < 7 * s.n_materials; i += blockDim.x) {
-        float v = 0.0f;
-        for (int k = 0; k < copies; k++) v += a.mat[i * copies + ((k + i) & (copies - 1))];  // (banks rotated)
-        const int m = i / 7;
-        material(m, i - 7 * m, v);
-    }
-    for (int i = threadIdx.x; copies == 0 && i < 7 * DIFF_MAT_KEYS; i += blockDim.x) {
-        const int k = mat_keys(a)[i & (DIFF_MAT_KEYS - 1)];
-        if (k != 0) material(k - 1, i / DIFF_MAT_KEYS, a.mat[i]);
+    if constexpr (FOUND) {
+        for (int i = threadIdx.x; i < 7 * DIFF_MAT_KEYS; i += blockDim.x) {
+            const int k = mat_keys(a)[i & (DIFF_MAT_KEYS - 1)];
+            if (k != 0) material(k - 1, i / DIFF_MAT_KEYS, a.mat[i]);
+        }
+    } else {
+        for (int i = threadIdx.x; i < 7 * s.n_materials; i += blockDim.x) {
+            float v = 0.0f;
+            for (int k = 0; k < copies; k++) v += a.mat[i * copies + ((k + i) & (copies - 1))];  // (banks rotated)
+            const int m = i / 7;
+            material(m, i - 7 * m, v);
+        }
     }
     if (threadIdx.x == 0 && a.loss != 0.0) atomicAdd(b.loss + rep, a.loss);
 }
@@ -527,7 +532,7 @@ __device__ __forceinline__ DFwd<NLMAX> diff_forward(const DevScene& s, const V& 
 
 // Its adjoint, into the accumulators.  VTX: albedo or normal gradients are
 // wanted.
-template <int NLMAX, bool VTX, class B, class T>
+template <int NLMAX, bool VTX, bool FOUND, class B, class T>
 __device__ __forceinline__ void diff_adjoint(const DFwd<NLMAX>& f, const DevScene& s, const B& b,
                                              const LightC (&lc)[NLMAX], F3 tg, DiffAcc& acc, int copies,
                                              ThreadAcc<NLMAX>& mine, T& vtx) {
@@ -578,11 +583,11 @@ __device__ __forceinline__ void diff_adjoint(const DFwd<NLMAX>& f, const DevScen
         const float d = div255(f.sLd);
         const float gm_[7] = {ga.x * d, ga.y * d, ga.z * d, gl.x * div255(f.sLs.x), gl.y * div255(f.sLs.y),
                               gl.z * div255(f.sLs.z), gshin};
-        const int slot = copies > 0 ? 0 : mat_bin(acc, mat);
-        if (slot >= 0) {
-            float* bin = copies > 0 ? acc.mat + 7 * mat * copies + (threadIdx.x & (copies - 1)) : acc.mat + slot;
-            const int step = copies > 0 ? copies : DIFF_MAT_KEYS;
-            for (int j = 0; j < 7; j++) atomicAdd(bin + j * step, gm_[j]);
+        if constexpr (!FOUND) {
+            float* bin = acc.mat + 7 * mat * copies + (threadIdx.x & (copies - 1));
+            for (int j = 0; j < 7; j++) atomicAdd(bin + j * copies, gm_[j]);
+        } else if (const int bin = mat_bin(acc, mat); bin >= 0) {
+            for (int j = 0; j < 7; j++) atomicAdd(&acc.mat[j * DIFF_MAT_KEYS + bin], gm_[j]);
         } else {
             for (int j = 0; j < 3; j++) {
                 atomicAdd(&b.g_kd[3 * (size_t)mat + j], gm_[j]);
@@ -756,7 +761,7 @@ struct VtxOf<true> {
 // M shaded pixels): 1184 -> 369 us a step; 6 views of 200^2 to 500^2 from the
 // stored G-buffer 94 -> 37 us; one of 512^2 with the vertices' gradients 130 ->
 // 55 us, its list included.
-template <int NLMAX, bool VTX, class B, class F>
+template <int NLMAX, bool VTX, bool FOUND, class B, class F>
 __device__ __forceinline__ void adjoint_chunks(const DevScene& s, const B& b0, const uint2* __restrict__ chunks,
                                                int n_chunks, F&& view) {
     __shared__ DiffAcc acc;
@@ -769,7 +774,7 @@ __device__ __forceinline__ void adjoint_chunks(const DevScene& s, const B& b0, c
     const int copies = mat_copies(s.n_materials), lane = threadIdx.x & 63;
     ThreadAcc<NLMAX> mine;
     thread_acc_clear(mine);
-    acc_clear(acc, s.n_materials, copies);
+    acc_clear<FOUND>(acc, s.n_materials, copies);
     vtx_clear(vtx);
     LightC lc[NLMAX];
     load_lights(s, b0, lc);
@@ -810,27 +815,27 @@ __device__ __forceinline__ void adjoint_chunks(const DevScene& s, const B& b0, c
             const size_t o = at(px0, w.v.W);
             const F3 tg = ld3(w.b.target + 3 * o);
             const DFwd<NLMAX> f = diff_forward(s, w.v, w.b, lc, x, y, o, rec);
-            diff_adjoint<NLMAX, VTX>(f, s, w.b, lc, tg, acc, copies, mine, vtx);
+            diff_adjoint<NLMAX, VTX, FOUND>(f, s, w.b, lc, tg, acc, copies, mine, vtx);
         }
         rec1 = record(px1, v1, k1);
         if constexpr (VTX) vtx_flush(vtx, b0);
         px0 = px1, v0 = v1, px1 = px2, v1 = v2, rec = rec1;
     }
     thread_acc_reduce(mine, s.n_lights, acc);
-    acc_flush(s, b0, acc, copies);
+    acc_flush<FOUND>(s, b0, acc, copies);
 }
 
 // waves a SIMD holds: the registers bound them
 constexpr int adjoint_waves(int nlmax) { return nlmax > 4 ? 3 : 4; }
-template <int NLMAX, bool VTX>
+template <int NLMAX, bool VTX, bool FOUND>
 __global__ __launch_bounds__(256, adjoint_waves(NLMAX)) void k_adjoint(DevScene s, DiffView w,
                                                                     const uint2* __restrict__ chunks,
                                                                     const int32_t* __restrict__ count) {
-    adjoint_chunks<NLMAX, VTX>(s, w.b, chunks, *count, [&](int) -> const DiffView& { return w; });
+    adjoint_chunks<NLMAX, VTX, FOUND>(s, w.b, chunks, *count, [&](int) -> const DiffView& { return w; });
 }
 // Many views of one scene: their parameters, gradients and loss are the same.
 // `step` (may be null): a fit's step counter, advanced by one.
-template <int NLMAX, bool VTX>
+template <int NLMAX, bool VTX, bool FOUND>
 __global__ __launch_bounds__(256, adjoint_waves(NLMAX)) void k_adjoint_views(DevScene s,
                                                                           const DiffView* __restrict__ views,
                                                                           const uint2* __restrict__ chunks,
@@ -838,7 +843,7 @@ __global__ __launch_bounds__(256, adjoint_waves(NLMAX)) void k_adjoint_views(Dev
                                                                           int32_t* step) {
     if (step && blockIdx.x == 0 && threadIdx.x == 0) *step += 1;  // (k_adam reads it)
     Const<DiffView>* tab = konst(views);
-    adjoint_chunks<NLMAX, VTX>(s, tab[0].b, chunks, *count, [&](int i) -> Const<DiffView>& { return tab[i]; });
+    adjoint_chunks<NLMAX, VTX, FOUND>(s, tab[0].b, chunks, *count, [&](int i) -> Const<DiffView>& { return tab[i]; });
 }
 
 // Zeroes an adjoint's gradients, its loss and its count of chunks.
@@ -974,18 +979,30 @@ void launch_diff_list_views(hipStream_t st, const DiffView* views, int32_t n, in
 // keeps its sums over many chunks and the flushes, atomics to the same few
 // lines, stay few; of a small view one per four chunks it may have.
 static unsigned adjoint_grid(size_t max_chunks) { return (unsigned)std::min<size_t>((max_chunks + 31) / 32 * 8 + 8, 1024); }
+// The kernel for a scene's lights and materials: pick(NLMAX, VTX, FOUND).
+template <class F>
+static auto adjoint_variant(const DevScene& s, bool vtx, F&& pick) {
+    using std::integral_constant;
+    auto by_found = [&](auto nl, auto v) {
+        return mat_copies(s.n_materials) == 0 ? pick(nl, v, std::true_type{}) : pick(nl, v, std::false_type{});
+    };
+    auto by_vtx = [&](auto nl) { return vtx ? by_found(nl, std::true_type{}) : by_found(nl, std::false_type{}); };
+    return s.n_lights <= 4 ? by_vtx(integral_constant<int, 4>{}) : by_vtx(integral_constant<int, 8>{});
+}
 void launch_adjoint(hipStream_t st, const DevScene& s, const DiffView& w, const uint2* chunks, const int32_t* count) {
     const dim3 grid(adjoint_grid((size_t)w.v.W * w.v.H / 64 + n_strips(w.v)));
-    const bool vtx = (w.b.want & (DIFF_ALBEDO | DIFF_NORMAL)) != 0 && !w.b.gbuf, few = s.n_lights <= 4;
-    const auto k = vtx ? (few ? k_adjoint<4, true> : k_adjoint<8, true>) : (few ? k_adjoint<4, false> : k_adjoint<8, false>);
+    const bool vtx = (w.b.want & (DIFF_ALBEDO | DIFF_NORMAL)) != 0 && !w.b.gbuf;
+    const auto k = adjoint_variant(s, vtx, [](auto nl, auto v, auto found) {
+        return k_adjoint<decltype(nl)::value, decltype(v)::value, decltype(found)::value>;
+    });
     hipLaunchKernelGGL(k, grid, dim3(256), 0, st, s, w, chunks, count);
 }
 void launch_adjoint_views(hipStream_t st, const DevScene& s, const DiffView* views, size_t max_chunks,
                           const uint2* chunks, const int32_t* count, bool vertices, int32_t* step) {
     const dim3 grid(adjoint_grid(max_chunks));
-    const bool few = s.n_lights <= 4;
-    const auto k = vertices ? (few ? k_adjoint_views<4, true> : k_adjoint_views<8, true>)
-                            : (few ? k_adjoint_views<4, false> : k_adjoint_views<8, false>);
+    const auto k = adjoint_variant(s, vertices, [](auto nl, auto v, auto found) {
+        return k_adjoint_views<decltype(nl)::value, decltype(v)::value, decltype(found)::value>;
+    });
     hipLaunchKernelGGL(k, grid, dim3(256), 0, st, s, views, chunks, count, step);
 }
 
